@@ -8,32 +8,42 @@
 // rounds while the component count falls (mst_port.cpp:203-313) and prints
 // weight, components and edges.
 //
-// Here one persistent kernel runs every round.  Edges are totally ordered by
-// (weight, smaller endpoint, larger endpoint), so each component's choice is
-// unique and the chosen edges form a forest except for pairs of components
-// that chose the same edge; the smaller id of such a pair stays a root and
-// the edge is counted once.  Per round:
-//   A  reset the lightest-weight and best-key words of every root, parent = self
-//   B  every vertex: lightest cross edge -> atomicMin(minw[comp])
-//   C  every vertex: among its edges of that weight, the smallest key ->
-//      atomicMin(best[comp])
-//   D  every root with a choice points at the other side's component
-//   E  mutual pairs keep one root; the others add the edge's weight
-//   F  every vertex follows parents to its new root (path halving)
+// Here one persistent kernel runs every round.  A component's choice is the
+// smallest key (weight, id of the component on the other side) over its
+// cross edges, one 64-bit atomic min per vertex or wave.  With that order the
+// choices form no cycle but pairs: in a longer cycle all weights are equal
+// (each is at most the next), the component t that the cycle's smallest id s
+// chose has s among its own lightest targets, so t chose s, and the cycle is
+// the pair {s, t}.  The smaller id of a pair stays a root and the edge is
+// counted once.  Per round, three barriers:
+//   1  every vertex: smallest key of its cross edges -> best[comp]
+//   2  every root with a choice: adds the edge's weight and points at the
+//      other side; of a pair that chose each other the smaller id stays
+//   3  every vertex follows parents to its new root (path halving)
 // The weight of a minimum spanning forest is unique, so it and the
 // component and edge counts are compared exactly.
+//
+// What bounds it: gathers of the neighbours' components, one walk of the
+// edges per round.  Rows are walked kSlots edges per lane step, by their lane
+// up to kSerialLimit edges, by a wave up to kLongRow, and longer ones in
+// pieces of kLongRow edges spread over all waves (a skewed graph's longest row
+// has as many edges as a thousand others); a vertex or piece without a cross
+// edge never gets one again and is left out of later rounds.  R-MAT 18 (7.6 M
+// edges, longest row 25 k): 0.93 ms (one lane walking each row twice per
+// round, six barriers: 46.4 ms).  Walking the rows of a wave as one list, with
+// the minima in LDS, took 1.07 ms: the search for each edge's row costs more
+// than the steps it saves.
 #include "graph_common.hpp"
 #include "runtime.hpp"
 
 namespace {
 
-constexpr unsigned kNoW = 0xffffffffu;
-constexpr unsigned long long kNoKey = ~0ull;
-
-__device__ __forceinline__ unsigned long long edge_key(int a, int b) {
-  const unsigned lo = (unsigned)(a < b ? a : b), hi = (unsigned)(a < b ? b : a);
-  return ((unsigned long long)lo << 32) | hi;
-}
+typedef unsigned long long u64;
+constexpr u64 kNoKey = ~0ull;
+constexpr unsigned kNoW = 0xffffffffu;  // an edge of this weight is never chosen
+constexpr int kSerialLimit = 16;
+constexpr int kSlots = 4;
+constexpr int kLongRow = 1024;
 
 // Root of component c: follows parent pointers, halving the path (a pointer
 // is only ever replaced by one of its ancestors, so racing walkers agree).
@@ -48,93 +58,153 @@ __device__ __forceinline__ int find_root(int* parent, int c, int n) {
   return c;
 }
 
+// Lowers best[c] to key for every lane that holds one.  Lanes of the first
+// such lane's component (all of them, once one component spans most of the
+// graph) share one atomic; a key that is not below the current value sends
+// none.
+__device__ __forceinline__ void lower_best(u64* best, bool has, int c, u64 key) {
+  const u64 mask = __ballot(has);
+  if (!mask) return;
+  const int leader = __ffsll((long long)mask) - 1;
+  const bool same = has && c == gdb::bcast(c, leader);
+  u64 k = same ? key : kNoKey;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const u64 o = __shfl_xor(k, off, 64);
+    k = o < k ? o : k;
+  }
+  if (same) {
+    has = gdb::lane_id() == leader;
+    key = k;
+  }
+  if (has && key < __hip_atomic_load(&best[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    gdb::atomic_min_g(&best[c], key);
+}
+
 template <int WGS>
 __global__ __launch_bounds__(WGS) void k_mst(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                              const int* __restrict__ col, const unsigned* __restrict__ w,
-                                             int n, int* comp, int* parent, unsigned* minw,
-                                             unsigned long long* best, int* flags,
-                                             unsigned long long* total, int* out) {
+                                             int n, int* comp, int* parent, u64* best, unsigned char* dead,
+                                             int2* pieces, int piece_cap, int* npieces, int* flags, u64* total,
+                                             int* out) {
   DISCOVERY_PROTOCOL(ctx);
   const int tid = p_get_global_id(ctx, &local_ctx);
   const int stride = p_get_global_size(ctx, &local_ctx);
+  const int lane = gdb::lane_id();
+  const int wave = tid >> 6, nwaves = stride >> 6;
+  const int spare = (int)((unsigned)tid % (unsigned)n);
   int rounds = 0, nbar = 0;
-  unsigned long long wsum = 0;
+  u64 wsum = 0;
   int added = 0;
-  for (int v = tid; v < n; v += stride) comp[v] = v;
+  for (int v = tid; v < n; v += stride) {
+    comp[v] = v;
+    parent[v] = v;
+    best[v] = kNoKey;
+    dead[v] = 0;
+    const int b = row[v], e = row[v + 1];
+    if (e - b > kLongRow) {
+      const int k = (e - b + kLongRow - 1) / kLongRow;
+      const int at = gdb::fadd_rlx(npieces, k);
+      for (int j = 0; j < k && at + j < piece_cap; ++j) pieces[at + j] = make_int2(v, b + j * kLongRow);
+    }
+  }
+  if (!discovery_barrier(ctx, &local_ctx)) return;
+  ++nbar;
+  const int np = min(gdb::ld_rlx(npieces), piece_cap);
   for (;;) {
-    // A
-    for (int c = tid; c < n; c += stride) {
-      if (comp[c] == c) {
-        minw[c] = kNoW;
-        best[c] = kNoKey;
-        parent[c] = c;
-      }
-    }
     if (tid == 0) gdb::st_rlx(&flags[(rounds + 1) % 3], 0);
-    if (!discovery_barrier(ctx, &local_ctx)) return;
-    ++nbar;
-    // B
-    for (int v = tid; v < n; v += stride) {
-      const int cv = comp[v];
-      unsigned m = kNoW;
-      for (int k = row[v]; k < row[v + 1]; ++k) {
-        const int u = col[k];
-        if ((unsigned)u >= (unsigned)n) continue;
-        const unsigned wk = w[k];
-        if (wk < m && comp[u] != cv) m = wk;
+    const bool first = rounds == 0;  // every vertex is its own component
+    auto step = [&](const bool (&ok)[kSlots], const int (&kk)[kSlots], int cv) -> u64 {
+      if (!gdb::any_slot(ok)) return kNoKey;  // no slot: no loads
+      int u[kSlots], cu[kSlots];
+      unsigned wk[kSlots];
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        const int k = ok[j] ? kk[j] : 0;  // edge 0 exists here
+        u[j] = gdb::ldg(col + k);
+        wk[j] = gdb::ldg(w + k);
       }
-      if (m != kNoW && (unsigned)cv < (unsigned)n) atomicMin(&minw[cv], m);
-    }
-    if (!discovery_barrier(ctx, &local_ctx)) return;
-    ++nbar;
-    // C
-    for (int v = tid; v < n; v += stride) {
-      const int cv = comp[v];
-      if ((unsigned)cv >= (unsigned)n) continue;
-      const unsigned m = minw[cv];
-      if (m == kNoW) continue;
-      unsigned long long key = kNoKey;
-      for (int k = row[v]; k < row[v + 1]; ++k) {
-        const int u = col[k];
-        if ((unsigned)u >= (unsigned)n || w[k] != m || comp[u] == cv) continue;
-        const unsigned long long kk = edge_key(v, u);
-        if (kk < key) key = kk;
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        const bool in = ok[j] && (unsigned)u[j] < (unsigned)n;
+        if (!in) wk[j] = kNoW;
+        cu[j] = first ? u[j] : gdb::ldg(comp + (in ? u[j] : spare));
       }
-      if (key != kNoKey) atomicMin(&best[cv], key);
+      u64 key = kNoKey;
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        const u64 k = ((u64)wk[j] << 32) | (unsigned)cu[j];
+        if (wk[j] != kNoW && cu[j] != cv && k < key) key = k;
+      }
+      return key;
+    };
+    auto least = [](u64 a, u64 c) { return a < c ? a : c; };
+    // 1: rows of up to kLongRow edges, then the pieces of the longer ones.
+    GDB_FOR_UNIFORM(v, valid, tid, stride, n) {
+      int b = 0, e = 0, cv = 0;
+      if (valid && !dead[v]) {
+        cv = comp[v];
+        b = row[v];
+        e = row[v + 1];
+        if (e - b > kLongRow) b = e;
+      }
+      const u64 key = gdb::wave_walk_np<kSlots>(e > b, b, e, cv, kNoKey, step, least, kSerialLimit);
+      const bool has = key != kNoKey && (unsigned)cv < (unsigned)n;
+      if (e > b && !has) dead[v] = 1;
+      if (first) {
+        if (has) best[v] = key;  // v's own word
+      } else {
+        lower_best(best, has, cv, key);
+      }
+    }
+    for (int i = wave; i < np; i += nwaves) {
+      const int2 pc = pieces[i];
+      if (pc.x < 0) continue;  // no cross edge left
+      const int e = min(row[pc.x + 1], pc.y + kLongRow), cv = comp[pc.x];
+      u64 key = kNoKey;
+      for (int base = pc.y; base < e; base += 64 * kSlots) {
+        bool ok[kSlots];
+        int kk[kSlots];
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) {
+          kk[j] = base + lane + 64 * j;
+          ok[j] = kk[j] < e;
+        }
+        key = least(key, step(ok, kk, cv));
+      }
+      if (__ballot(key != kNoKey) == 0) {
+        if (lane == 0) pieces[i].x = -1;
+      } else if ((unsigned)cv < (unsigned)n) {
+        lower_best(best, key != kNoKey, cv, key);
+      }
     }
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
-    // D
-    for (int c = tid; c < n; c += stride) {
-      if (comp[c] != c || best[c] == kNoKey) continue;
-      const int a = (int)(best[c] >> 32), b = (int)(best[c] & 0xffffffffu);
-      if ((unsigned)a >= (unsigned)n || (unsigned)b >= (unsigned)n) continue;
-      const int ca = comp[a], cb = comp[b];
-      parent[c] = ca == c ? cb : ca;
-    }
-    if (!discovery_barrier(ctx, &local_ctx)) return;
-    ++nbar;
-    // E
+    // 2
     bool progress = false;
     for (int c = tid; c < n; c += stride) {
       if (comp[c] != c) continue;
-      const int p = parent[c];
-      if (p == c || (unsigned)p >= (unsigned)n) continue;
-      if (parent[p] == c && c < p) {
-        parent[c] = c;  // the pair's smaller id stays the root; p counts the edge
-      } else {
-        wsum += minw[c];
-        ++added;
-        progress = true;
-      }
+      const u64 k = best[c];
+      if (k == kNoKey) continue;
+      const int p = (int)(unsigned)k;
+      if ((unsigned)p >= (unsigned)n) continue;
+      if (best[p] != kNoKey && (int)(unsigned)best[p] == c && c < p) continue;  // the pair's root; p counts the edge
+      parent[c] = p;
+      wsum += k >> 32;
+      ++added;
+      progress = true;
     }
-    if (gdb::wave_any(progress) && gdb::lane_id() == 0) gdb::st_rlx(&flags[rounds % 3], 1);
+    if (gdb::wave_any(progress) && lane == 0) gdb::st_rlx(&flags[rounds % 3], 1);
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
-    // F
+    // 3
     for (int v = tid; v < n; v += stride) {
       const int c = comp[v];
-      if ((unsigned)c < (unsigned)n) comp[v] = find_root(parent, c, n);
+      if (best[v] != kNoKey) best[v] = kNoKey;
+      if ((unsigned)c < (unsigned)n) {
+        const int r = find_root(parent, c, n);
+        if (r != c) comp[v] = r;
+      }
     }
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
@@ -146,7 +216,7 @@ __global__ __launch_bounds__(WGS) void k_mst(gdb_kernel_ctx_t* ctx, const int* _
     }
   }
   // Totals: one atomic per wave.
-  unsigned long long ws = wsum;
+  u64 ws = wsum;
   int ad = added, roots = 0;
   for (int v = tid; v < n; v += stride) roots += comp[v] == v;
   for (int off = 32; off > 0; off >>= 1) {
@@ -154,7 +224,7 @@ __global__ __launch_bounds__(WGS) void k_mst(gdb_kernel_ctx_t* ctx, const int* _
     ad += __shfl_xor(ad, off, 64);
     roots += __shfl_xor(roots, off, 64);
   }
-  if (gdb::lane_id() == 0) {
+  if (lane == 0) {
     if (ws) atomicAdd(total, ws);
     if (ad) atomicAdd(&out[2], ad);
     if (roots) atomicAdd(&out[3], roots);
@@ -185,22 +255,25 @@ extern "C" int gdb_mst(gdb_ctx* ctx, int n, int m, const int* row, const int* co
     if (stats) *stats = st;
     return GDB_SUCCESS;
   }
-  const size_t bytes = carve_bytes<int>(n) * 2 + carve_bytes<unsigned>(n) +
-                       carve_bytes<unsigned long long>(n) + carve_bytes<int>(32) +
-                       carve_bytes<unsigned long long>(1);
+  // Each row longer than kLongRow has at most 2 * edges / kLongRow pieces.
+  const int piece_cap = 2 * (m / kLongRow) + 1;
+  const size_t bytes = carve_bytes<int>(n) * 2 + carve_bytes<u64>(n) + carve_bytes<unsigned char>(n) +
+                       carve_bytes<int2>(piece_cap) + carve_bytes<int>(32) + carve_bytes<u64>(1);
   int rc = ensure_workspace(ctx, bytes);
   if (rc) return rc;
   Carve cv(ctx->ws);
   int* comp = cv.take<int>(n);
   int* parent = cv.take<int>(n);
-  unsigned* minw = cv.take<unsigned>(n);
-  unsigned long long* best = cv.take<unsigned long long>(n);
+  u64* best = cv.take<u64>(n);
+  unsigned char* dead = cv.take<unsigned char>(n);
+  int2* pieces = cv.take<int2>(piece_cap);
   int* flags = cv.take<int>(32);
-  unsigned long long* total = cv.take<unsigned long long>(1);
+  u64* total = cv.take<u64>(1);
   rc = fill_i32(ctx, flags, 0, 32);
   if (!rc) rc = fill_i32(ctx, (int*)total, 0, 2);
   if (rc) return rc;
   int* out = flags + 8;
+  int* npieces = flags + 16;
   rc = prepare_launch(ctx);
   if (rc) return rc;
   rc = gdb_dispatch_wgs(wgs, [&](auto W) -> int {
@@ -211,7 +284,7 @@ extern "C" int gdb_mst(gdb_ctx* ctx, int n, int m, const int* row, const int* co
     r2 = timer_start(ctx);
     if (r2) return r2;
     hipLaunchKernelGGL(k_mst<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col, w, n, comp, parent,
-                       minw, best, flags, total, out);
+                       best, dead, pieces, piece_cap, npieces, flags, total, out);
     GDB_HIP(hipGetLastError());
     return timer_stop(ctx, &st.kernel_ms);
   });

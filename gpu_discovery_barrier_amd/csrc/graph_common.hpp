@@ -21,6 +21,9 @@ __device__ __forceinline__ int shfl_xor(int x, int o) { return __shfl_xor(x, o, 
 __device__ __forceinline__ unsigned shfl_xor(unsigned x, int o) {
   return (unsigned)__shfl_xor((int)x, o, 64);
 }
+__device__ __forceinline__ unsigned long long shfl_xor(unsigned long long x, int o) {
+  return __shfl_xor(x, o, 64);
+}
 
 // Global-address-space accessors.  Graph arrays reach the kernels through
 // structs, so the compiler sees generic pointers and emits flat instructions,

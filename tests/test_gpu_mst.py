@@ -51,3 +51,17 @@ def test_mst_small_fixtures(ctx):
         g = gdb.CSR(n, row, col, w if len(w) else np.zeros(0, np.int32))
         wt, ed, cp, _ = gdb.mst(ctx, gdb.DeviceCSR(g))
         assert (wt, ed, cp) == want, (n, edges)
+
+
+@pytest.mark.parametrize("wgs,groups", [(0, 0), (64, 3), (512, 256)])
+@pytest.mark.parametrize("leaves", [15, 16, 17, 1023, 1024, 1025, 2047, 2049, 5000])
+def test_mst_row_lengths(ctx, wgs, groups, leaves):
+    # Two hubs that share `leaves` neighbours, with ties: rows at the edges of
+    # the per-lane, per-wave and per-piece walks.
+    rng = np.random.default_rng(leaves)
+    n = leaves + 2
+    edges = [(h, 2 + i) for h in range(2) for i in range(leaves)] + [(0, 1)]
+    row, col, w = csr_from_edges(n, edges, rng.integers(1, 9, len(edges)).tolist())
+    want = oracle.mst_kruskal(row, col, w)
+    wt, ed, cp, _ = gdb.mst(ctx, gdb.DeviceCSR(gdb.CSR(n, row, col, w)), gdb.Opts.make(wgs=wgs, groups=groups))
+    assert (wt, ed, cp) == want
