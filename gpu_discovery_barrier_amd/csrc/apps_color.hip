@@ -11,7 +11,10 @@
 // Schedules:
 //   plain persistent  - the mega_kernel structure (lines 159-252): two phases
 //                       and two barriers per round, thread per vertex.
-//   tuned persistent  - one barrier per round: phase r also applies round
+//   tuned persistent  - where every blocking edge fits a register of the
+//                       launch: no rounds at all (k_color_flow,
+//                       k_color_flow1 below).  Otherwise one barrier per
+//                       round (k_color_tuned): phase r also applies round
 //                       r-1's colouring (v coloured in r-1 iff uncoloured and
 //                       node_value[v] > max_d_{r-1}[v]), so a neighbour's state
 //                       is read as "uncoloured after r-1" from color[] and the
@@ -23,6 +26,7 @@
 //   relaunch          - color / color2 kernels per round with a host loop
 //                       (color.cpp:294-334).
 #include <algorithm>
+#include <climits>
 
 #include "graph_common.hpp"
 #include "runtime.hpp"
@@ -173,6 +177,8 @@ __device__ __forceinline__ int fkey(float f) {
   return b < 0 ? b ^ 0x7fffffff : b;
 }
 
+constexpr int kFlowWgs = 1024;   // group size of k_color_flow when the caller left it open (512: 0.71
+                                 // against 0.57 ms on R-MAT 15, 1.24 against 0.95 on the 400^2 grid)
 constexpr int kHeavyDeg = 16;    // rows longer than this are split into chunks
 constexpr int kChunkEdges = 64;  // edges of a heavy row per chunk (one per lane)
 constexpr int kSlots = 8;        // edges a lane gathers per step on light rows
@@ -364,6 +370,327 @@ __global__ __launch_bounds__(WGS) void k_color_tuned(gdb_kernel_ctx_t* ctx, cons
   }
 }
 
+// ---- the max rule without rounds ---------------------------------------------
+// v takes its colour in the first round in which every neighbour u with
+// nv[u] >= nv[v] (a blocker) is coloured, so colour(v) = 1 + the largest
+// colour of its blockers (1 without one; blockers are ignored when deg(v) ==
+// 1; a v with nv[v] <= -1 or NaN is never coloured).  The rule's rounds are a
+// dataflow over the blocking edges, and the number of rounds is 1 + the largest
+// min(colour(v), colour(u)) over the edges (v, u) with deg(v) != 1: a round
+// continues the loop iff such an edge had both ends uncoloured at its start.
+//
+// k_color_flow gives each lane kFlowK edges, held in registers (window w of the
+// edge array, WGS * kFlowK edges, belongs to participating group w).  Each lane
+// polls the colours of its blockers, counts its rows' remaining blockers down
+// in LDS and stores the colour of a row that has none left.  A colour thus
+// travels along an edge in one store and one poll (a cross-XCD hand-off,
+// about 0.6 us), where a round of k_color_tuned costs a barrier and three
+// dependent gathers.  A row that spans windows meets in two device words
+// (gmx, gcnt).  Every window needs its group resident: fewer participants
+// than windows, or no progress for `limit` ticks (ties, which never resolve),
+// raise a flag and the host runs k_color_tuned instead.
+// R-MAT 14 (213 k blocking edges, 294 rounds): 0.52 ms against 6.5 with rounds;
+// the 400^2 grid with index-ordered values (799 rounds): 0.95 against 17.
+constexpr int kFlowK = 4;
+enum FlowWord { FW_ROUNDS = 0, FW_GAVE_UP, FW_INVALID, FW_WORDS };
+
+__device__ __forceinline__ bool colourable(float x) { return x > -1.f; }
+
+// poll[v]: 0 uncoloured, else the colour; poll[n] stays 0.  Rows outside the
+// edge arrays raise FW_INVALID.
+__global__ void k_flow_init(const int* __restrict__ row, const float* __restrict__ nv, int n, int m, int window,
+                            int* poll, int* gmx, int* gcnt, int* fw) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v > n) return;
+  if (v == n) {
+    poll[n] = 0;
+    return;
+  }
+  const int b = row[v], e = row[v + 1];
+  if (b < 0 || e < b || e > m) fw[FW_INVALID] = 1;
+  poll[v] = b == e && colourable(nv[v]) ? 1 : 0;
+  gmx[v] = 0;
+  gcnt[v] = e > b ? (e - 1) / window - b / window + 1 : 0;
+}
+
+// Whether a wave that made no progress since t_last should stop.
+__device__ __forceinline__ bool flow_stuck(int* fw, unsigned it, unsigned long long t_last, unsigned long long limit) {
+  if ((it & 63u) != 63u) return false;
+  if (gdb::ld_rlx(&fw[FW_GAVE_UP])) return true;
+  if (gdb::now() - t_last <= limit) return false;
+  gdb::st_rlx(&fw[FW_GAVE_UP], 1);
+  return true;
+}
+
+template <int WGS>
+__global__ __launch_bounds__(WGS) void k_color_flow(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
+                                                    const int* __restrict__ col, const float* __restrict__ nv,
+                                                    int n, int m, int* poll, int* gmx, int* gcnt, int* fw,
+                                                    unsigned long long limit) {
+  DISCOVERY_PROTOCOL(ctx);
+  extern __shared__ int flow_lds[];
+  constexpr int K = kFlowK, C = WGS * K;
+  int* const cnt = flow_lds;    // blockers left of the row whose first edge in this window is edge ws + i
+  int* const mx = flow_lds + C; // largest colour of its blockers so far
+  const int nwin = m > 0 ? (m - 1) / C + 1 : 1;
+  if (p_get_num_groups(ctx, &local_ctx) < nwin) {
+    if (threadIdx.x == 0) gdb::st_rlx(&fw[FW_GAVE_UP], 1);
+    return;
+  }
+  if (gdb::ld_rlx(&fw[FW_INVALID])) return;
+  const int w = p_get_group_id(ctx, &local_ctx);
+  if (w >= nwin) return;
+  const int ws = w * C;
+  for (int i = threadIdx.x; i < C; i += WGS) {
+    cnt[i] = 0;
+    mx[i] = 0;
+  }
+  __syncthreads();
+  // This lane's edges ws + j * WGS + thread: row (binary search), blocker
+  // or not, and the row's slot.  u == n marks an entry with nothing to wait for.
+  constexpr int kSpans = 1 << 30;  // in slot: the row goes beyond this window
+  int u[K], v[K], slot[K];
+  unsigned first = 0;  // bit j: the row's first edge in this window
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const int e = ws + j * WGS + (int)threadIdx.x;
+    int lo = 0, hi = n;  // first vertex whose row ends beyond e
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (row[mid + 1] > e) hi = mid; else lo = mid + 1;
+    }
+    v[j] = lo < n ? lo : 0;
+    u[j] = n;
+    slot[j] = 0;
+    if (e < m && lo < n && row[lo] <= e) {
+      const int b = row[lo], end = row[lo + 1], x = col[e];
+      const float xv = nv[lo];
+      const int at = (b > ws ? b : ws) - ws;
+      slot[j] = at | ((b < ws || end > ws + C) ? kSpans : 0);
+      if (colourable(xv)) {
+        if (e == ws + at) first |= 1u << j;
+        if (end - b != 1 && (unsigned)x < (unsigned)n && nv[x] >= xv) {
+          u[j] = x;
+          atomicAdd(&cnt[at], 1);
+        }
+      }
+    }
+  }
+  // Called by the lane that found row v's last blocker of this window coloured.
+  auto complete = [&](int vv, int sl) {
+    const int at = sl & (kSpans - 1);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);  // the maximum is read after the count (LDS operations are in order)
+    int c = mx[at];
+    if (sl & kSpans) {
+      // The maximum is in place (a returned atomic) before the piece is
+      // counted off; the last piece reads them all.
+      const int old = gdb::atomic_max_g(&gmx[vv], c);
+      asm volatile("" ::"v"(old) : "memory");
+      if (gdb::fadd(&gcnt[vv], -1) != 1) return;
+      c = gdb::ld_rlx(&gmx[vv]);
+    }
+    gdb::st_rlx(&poll[vv], c + 1);
+  };
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < K; ++j)
+    if (cnt[slot[j] & (kSpans - 1)] != 0) first &= ~(1u << j);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < K; ++j)
+    if ((first >> j) & 1u) complete(v[j], slot[j]);
+  unsigned long long t_last = gdb::now();
+  for (unsigned it = 0;; ++it) {
+    bool pending = false;
+#pragma unroll
+    for (int j = 0; j < K; ++j) pending |= u[j] != n;
+    if (!gdb::wave_any(pending)) break;
+    int c[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) asm volatile("" : "+v"(v[j]), "+v"(slot[j]));  // no addresses kept beside the entries
+#pragma unroll
+    for (int j = 0; j < K; ++j) c[j] = gdb::ld_rlx_g(poll + u[j]);  // finished entries read poll[n], 0
+    bool moved = false;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      if (c[j] != 0) {
+        const int at = slot[j] & (kSpans - 1);
+        atomicMax(&mx[at], c[j]);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        u[j] = n;
+        moved = true;
+        if (atomicSub(&cnt[at], 1) == 1) complete(v[j], slot[j]);
+      }
+    }
+    if (gdb::wave_any(moved)) t_last = gdb::now();
+    else if (flow_stuck(fw, it, t_last, limit)) break;
+  }
+}
+
+// Colours and round count of a finished k_color_flow.
+__global__ __launch_bounds__(256) void k_flow_out(const int* __restrict__ row, const int* __restrict__ col, int n,
+                                                  const int* __restrict__ poll, int* color, int* fw) {
+  if (fw[FW_GAVE_UP] || fw[FW_INVALID]) return;
+  const int v = blockIdx.x * 256 + threadIdx.x;
+  const bool valid = v < n;
+  int b = 0, e = 0, cv = 0;
+  if (valid) {
+    b = row[v];
+    e = row[v + 1];
+    cv = poll[v];
+    color[v] = cv ? cv : -1;
+    if (!cv) cv = INT_MAX;
+    if (e - b == 1) e = b;
+  }
+  const int spare = valid ? v : 0;
+  const int r = gdb::wave_walk_np<4>(
+      valid, b, e, cv, 0,
+      [&](const bool (&ok)[4], const int (&kk)[4], int own) -> int {
+        if (!gdb::any_slot(ok)) return 0;
+        int u[4], c[4], best = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) u[j] = gdb::ldg(col + (ok[j] ? kk[j] : 0));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bool in = ok[j] && (unsigned)u[j] < (unsigned)n;
+          c[j] = gdb::ldg(poll + (in ? u[j] : spare));
+          if (!c[j]) c[j] = INT_MAX;
+          if (in) best = max(best, min(own, c[j]));
+        }
+        return best;
+      },
+      [](int a, int c) { return max(a, c); }, kSerialLimit);
+  const int rm = gdb::wave_max(r);
+  if (gdb::lane_id() == 0 && rm > 0) atomicMax(&fw[FW_ROUNDS], rm);
+}
+
+// The same in one group, for a graph of at most kFlow1N vertices and 1024 *
+// kFlow1K edges: colours, counts and row offsets sit in LDS and a poll is an LDS
+// read (about 0.1 us with 32 edges per lane, against 0.7 us for a device
+// word).  R-MAT 10 (10.6 k blocking edges, 77 rounds): 0.115 ms against
+// 0.94 with rounds, and 0.137 with k_color_flow on 21 groups.
+constexpr int kFlow1N = 8192, kFlow1K = 32;
+inline size_t flow1_lds(int n) { return sizeof(int) * (4 * (size_t)n + 2); }
+
+__global__ __launch_bounds__(1024) void k_color_flow1(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
+                                                      const int* __restrict__ col, const float* __restrict__ nv,
+                                                      int n, int m, int* color, int* fw, unsigned long long limit) {
+  DISCOVERY_PROTOCOL(ctx);
+  extern __shared__ int flow_lds[];
+  __shared__ int s_rounds, s_bad;
+  constexpr int K = kFlow1K;
+  int* const c = flow_lds;       // colours, c[n] = 0
+  int* const cnt = c + n + 1;    // blockers left
+  int* const mx = cnt + n;       // largest colour of the blockers so far
+  int* const off = mx + n;       // row offsets
+  if (threadIdx.x == 0) s_rounds = s_bad = 0;
+  __syncthreads();
+  bool bad = false;
+  for (int i = threadIdx.x; i <= n; i += 1024) {
+    const int o = row[i];
+    off[i] = o;
+    c[i] = 0;
+    if (i < n) {
+      cnt[i] = mx[i] = 0;
+      bad |= o < 0 || row[i + 1] < o || row[i + 1] > m;
+    }
+  }
+  if (bad) s_bad = 1;
+  __syncthreads();
+  if (s_bad) {
+    if (threadIdx.x == 0) fw[FW_INVALID] = 1;
+    return;
+  }
+  // Edge j * 1024 + thread as u << 16 | v (both below 2^16), pending bit j.
+  unsigned ent[K], pend = 0;
+  constexpr unsigned kNoEdge = ~0u;  // none, or the edge of a row of one edge
+#pragma unroll
+  for (int j0 = 0; j0 < K; j0 += 8) {
+    int lo[8], x[8];
+    float xv[8], xu[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int e = (j0 + j) * 1024 + (int)threadIdx.x;
+      x[j] = e < m ? col[e] : -1;
+      lo[j] = 0;
+    }
+    if (j0 * 1024 < m)
+#pragma nounroll
+      for (int step = kFlow1N; step > 0; step >>= 1)  // number of rows that end at or before e
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int mid = lo[j] + step;
+          if (mid <= n && off[mid] <= (j0 + j) * 1024 + (int)threadIdx.x) lo[j] = mid;
+        }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int e = (j0 + j) * 1024 + (int)threadIdx.x;
+      const bool in = (unsigned)x[j] < (unsigned)n && lo[j] < n && off[lo[j]] <= e && off[lo[j] + 1] - off[lo[j]] != 1;
+      if (!in) x[j] = -1;
+      xv[j] = nv[in ? lo[j] : 0];
+      xu[j] = nv[in ? x[j] : 0];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      ent[j0 + j] = x[j] >= 0 ? ((unsigned)x[j] << 16) | (unsigned)lo[j] : kNoEdge;
+      if (x[j] >= 0 && colourable(xv[j]) && xu[j] >= xv[j]) {
+        pend |= 1u << (j0 + j);
+        atomicAdd(&cnt[lo[j]], 1);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one group of eight at a time: registers
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += 1024)  // rows without a blocker
+    if (cnt[i] == 0 && colourable(nv[i])) c[i] = 1;
+  __syncthreads();
+  unsigned long long t_last = gdb::now();
+  for (unsigned it = 0; gdb::wave_any(pend != 0); ++it) {
+    bool moved = false;
+#pragma unroll
+    for (int j0 = 0; j0 < K; j0 += 8) {  // eight reads in flight; groups of eight without a pending edge are skipped
+      if (!gdb::wave_any(((pend >> j0) & 0xffu) != 0)) continue;
+      int x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(ent[j0 + j]));  // no addresses kept beside the entries
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        x[j] = __hip_atomic_load(&c[(pend >> (j0 + j)) & 1u ? (int)(ent[j0 + j] >> 16) : n], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (x[j] != 0) {
+          const int vv = (int)(ent[j0 + j] & 0xffffu);
+          atomicMax(&mx[vv], x[j]);
+          __atomic_signal_fence(__ATOMIC_SEQ_CST);  // maximum, count, then the maximum's value: in this order
+          pend &= ~(1u << (j0 + j));
+          moved = true;
+          if (atomicSub(&cnt[vv], 1) == 1) {
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __hip_atomic_store(&c[vv], mx[vv] + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+        }
+    }
+    if (gdb::wave_any(moved)) t_last = gdb::now();
+    else if (flow_stuck(fw, it, t_last, limit)) break;
+  }
+  __syncthreads();
+  if (gdb::ld_rlx(&fw[FW_GAVE_UP])) return;
+  int r = 0;
+#pragma unroll
+  for (int j = 0; j < K; ++j)
+    if (ent[j] != kNoEdge) {
+      const int a = c[ent[j] >> 16], b = c[ent[j] & 0xffffu];
+      r = max(r, min(a ? a : INT_MAX, b ? b : INT_MAX));
+    }
+  r = gdb::wave_max(r);
+  if (gdb::lane_id() == 0 && r > 0) atomicMax(&s_rounds, r);
+  for (int i = threadIdx.x; i < n; i += 1024) color[i] = c[i] ? c[i] : -1;
+  __syncthreads();
+  if (threadIdx.x == 0) fw[FW_ROUNDS] = s_rounds;
+}
+
 // ---- relaunch schedule: color (color_kernel.cl:80-123) and color2 (134-154)
 // `flags` = {stop[0..2], done, last}.  Round r writes stop[r % 3]; a kernel of
 // round r is a no-op once round r-1 ended with stop 0 (done is sticky).
@@ -424,6 +751,98 @@ __global__ void k_color_init(int* color, float* max_d, int* mdk, int* flags, int
 
 using namespace gdbrt;
 
+namespace {
+
+// Launches the round-free kernels.  *done: the colouring is finished and s
+// filled in; otherwise (a shape that cannot hold the edges, too few
+// participants, ties) the caller runs the round-based kernel.
+//
+// The rule: one group when the graph fits its LDS and the caller left the
+// shape open; else as many groups as cover the edges, if the caller's launch
+// or, with the shape open, one 1024-thread group per CU does (1 M edges).
+// Beyond that the polls bound it: every pending edge reads a device word again
+// and again, and those of a skewed graph's hubs meet in a few L2 lines.  R-MAT
+// 15 (0.88 M edges) 0.57 ms against 8.5 with rounds; R-MAT 17 at 16 edges a
+// lane 94 ms against 45.
+int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const float* nv, int* color,
+               const gdb_opts& asked, gdb_stats* s, bool* done) {
+  *done = false;
+  const bool open = asked.wgs == 0;
+  gdb_opts o = asked;
+  if (open) o.wgs = kFlowWgs;
+  const bool one = open && asked.groups == 0 && n <= kFlow1N && m <= 1024 * kFlow1K;
+  // A wave that sees no progress for this long gives up: ties, or a chain of
+  // more hops than there are vertices.  2 us a vertex, well over a hop.
+  const unsigned long long limit =
+      std::min<unsigned long long>(ctx->timeout_ticks, 200000ull + 200ull * (unsigned long long)n);
+  const size_t bytes = carve_bytes<int>((size_t)n + 1) + 2 * carve_bytes<int>(n) + carve_bytes<int>(FW_WORDS);
+  int rc = ensure_workspace(ctx, bytes);
+  if (rc) return rc;
+  Carve cv(ctx->ws);
+  int* fw = cv.take<int>(FW_WORDS);
+  int* poll = cv.take<int>((size_t)n + 1);
+  int* gmx = cv.take<int>(n);
+  int* gcnt = cv.take<int>(n);
+  auto begin = [&]() -> int {
+    int r = fill_i32(ctx, fw, 0, FW_WORDS);
+    if (!r) r = prepare_launch(ctx);
+    return r;
+  };
+  if (one) {
+    const size_t lds = flow1_lds(n);
+    if (lds > 49152)
+      GDB_HIP(hipFuncSetAttribute((const void*)k_color_flow1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    rc = begin();
+    if (!rc) rc = timer_start(ctx);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_color_flow1, dim3(1), dim3(1024), lds, ctx->stream, ctx->d, row, col, nv, n, m, color, fw,
+                       limit);
+    GDB_HIP(hipGetLastError());
+    rc = timer_stop(ctx, &s->kernel_ms);
+    if (rc) return rc;
+    s->launches = 1;
+  } else {
+    bool ran = false;
+    rc = gdb_dispatch_wgs(o.wgs, [&](auto W) -> int {
+      constexpr int WG = decltype(W)::value;
+      constexpr int C = WG * kFlowK;
+      const void* kern = (const void*)k_color_flow<WG>;
+      const size_t lds = 2 * sizeof(int) * C;
+      const int nwin = m > 0 ? (m - 1) / C + 1 : 1;
+      int groups = 0;
+      int r = launch_groups(ctx, kern, &o, (long long)GDB_MAX_GROUPS * WG, &groups, lds);
+      if (r) return r;
+      if (nwin > (open ? std::min(groups, ctx->num_cus) : groups)) return GDB_SUCCESS;
+      r = begin();
+      if (!r) r = timer_start(ctx);
+      if (r) return r;
+      hipLaunchKernelGGL(k_flow_init, dim3(n / 256 + 1), dim3(256), 0, ctx->stream, row, nv, n, m, C, poll, gmx, gcnt,
+                         fw);
+      hipLaunchKernelGGL(k_color_flow<WG>, dim3(nwin), dim3(WG), lds, ctx->stream, ctx->d, row, col, nv, n, m, poll,
+                         gmx, gcnt, fw, limit);
+      hipLaunchKernelGGL(k_flow_out, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, row, col, n, poll, color, fw);
+      GDB_HIP(hipGetLastError());
+      ran = true;
+      s->launches = 3;
+      return timer_stop(ctx, &s->kernel_ms);
+    });
+    if (rc || !ran) return rc;
+  }
+  int h[FW_WORDS] = {};
+  GDB_HIP(hipMemcpy(h, fw, sizeof(h), hipMemcpyDeviceToHost));
+  rc = check_device_error(ctx);
+  if (rc) return rc;
+  if (h[FW_INVALID]) return GDB_E_INVALID;
+  if (h[FW_GAVE_UP] || h[FW_ROUNDS] == INT_MAX) return GDB_SUCCESS;  // INT_MAX: neighbours that are never coloured
+  rc = read_participating(ctx, &s->participating);
+  if (rc) return rc;
+  s->rounds = h[FW_ROUNDS] + 1;
+  *done = true;
+  return GDB_SUCCESS;
+}
+
+}  // namespace
+
 extern "C" int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* col,
                          const float* node_value, int* color, const gdb_opts* opts,
                          gdb_stats* stats) {
@@ -431,6 +850,7 @@ extern "C" int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* 
     return GDB_E_INVALID;
   gdb_opts o{};
   if (opts) o = *opts;
+  const gdb_opts asked = o;
   if (o.variant == GDB_VARIANT_TUNED && o.schedule == GDB_SCHED_PERSISTENT) gdbrt::apply_tuning("color", n, &o);
   const int wgs = default_wgs(&o);
   gdb_stats s{};
@@ -439,6 +859,18 @@ extern "C" int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* 
     return GDB_SUCCESS;
   }
   const bool tuned_persistent = o.variant == GDB_VARIANT_TUNED && o.schedule != GDB_SCHED_RELAUNCH;
+  if (tuned_persistent) {
+    bool done = false;
+    const int frc = color_flow(ctx, n, m, row, col, node_value, color, asked, &s, &done);
+    if (frc) return frc;
+    if (done) {
+      s.work_edges = m;
+      s.work_items = n;
+      if (stats) *stats = s;
+      return GDB_SUCCESS;
+    }
+    s = gdb_stats{};
+  }
   // Tuned schedule: rows longer than kHeavyDeg are split into chunks of
   // kChunkEdges edges; the rows and the (row, first edge) of every chunk
   // are listed here from the row offsets.

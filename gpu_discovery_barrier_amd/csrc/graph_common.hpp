@@ -32,6 +32,10 @@ template <typename T>
 __device__ __forceinline__ T ldg(const T* p) {
   return *(const __attribute__((address_space(1))) T*)p;
 }
+__device__ __forceinline__ int ld_rlx_g(const int* p) {  // agent scope, relaxed
+  return __hip_atomic_load((const __attribute__((address_space(1))) int*)p, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ unsigned atomic_min_g(unsigned* p, unsigned v) {
   return __hip_atomic_fetch_min((__attribute__((address_space(1))) unsigned*)p, v, __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_AGENT);

@@ -112,6 +112,57 @@ def test_color_tuned_blockers(ctx, shape, order):
     assert st.rounds == rr
 
 
+def directed(n, m, seed, hub=0):
+    """A random directed CSR (no symmetry, parallel edges kept), with one row
+    of `hub` edges."""
+    rng = np.random.default_rng(seed)
+    src = np.concatenate([rng.integers(0, n, m - hub), np.full(hub, n // 3)])
+    dst = rng.integers(0, n, m)
+    dst = np.where(dst == src, (dst + 1) % n, dst)
+    order = np.lexsort((dst, src))
+    row = np.zeros(n + 1, np.int32)
+    np.add.at(row, src + 1, 1)
+    return np.cumsum(row).astype(np.int32), dst[order].astype(np.int32)
+
+
+# Launch shapes of the round-free kernels: left open (one group with LDS
+# colours up to 8192 vertices and 32768 edges, else 1024-thread groups), and
+# fixed ones whose windows of four edges a lane cut rows (the last one covers
+# too few edges for most of the graphs, which take the kernel with rounds).
+@pytest.mark.parametrize("wgs,groups", [(0, 0), (64, 0), (64, 64), (256, 8)])
+@pytest.mark.parametrize("n,m,hub", [(1, 0, 0), (2, 2, 0), (1000, 255, 0), (1000, 256, 0), (3000, 257, 200),
+                                     (8192, 32768, 3000), (8193, 32768, 0), (8192, 32769, 5000), (700, 4097, 2500),
+                                     (20000, 60000, 700)])
+def test_color_flow_edges(ctx, n, m, hub, wgs, groups):
+    row, col = directed(n, m, n + m, hub) if n > 1 else (np.zeros(2, np.int32), np.zeros(0, np.int32))
+    nv = np.random.default_rng(m).permutation(n).astype(np.float32) / np.float32(n + 1)
+    nv[np.argsort(nv)[-3:]] = -2.0  # never coloured (not above -1), and blocking nobody
+    want, rr = oracle.color_ref(row, col, nv)
+    kw = dict(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED)
+    if rr < 0:  # neighbours that are never coloured: the loop cannot end
+        with pytest.raises(gdb.GdbError) as e:
+            run(ctx, row, col, nv, **kw)
+        assert e.value.code == gdb.GDB_E_TIMEOUT
+        return
+    got, st = run(ctx, row, col, nv, **kw)
+    assert (got == want).all() and st.rounds == rr
+
+
+@pytest.mark.parametrize("n", [3, 9000])
+def test_color_flow_ties_then_clean(ctx, n):
+    # A cycle of equal priorities never resolves; the next solve on the same
+    # context is unaffected.
+    edges = [(i, (i + 1) % n) for i in range(n)]
+    row, col, _ = csr_from_edges(n, edges)
+    with pytest.raises(gdb.GdbError) as e:
+        run(ctx, row, col, np.full(n, 0.5, np.float32), wgs=0, variant=gdb.VARIANT_TUNED)
+    assert e.value.code == gdb.GDB_E_TIMEOUT
+    nv = gdb.pannotia_values(n)
+    want, rr = oracle.color_ref(row, col, nv)
+    got, st = run(ctx, row, col, nv, wgs=0, variant=gdb.VARIANT_TUNED)
+    assert (got == want).all() and st.rounds == rr
+
+
 # ---------------------------------------------------------------- max-min colouring
 @pytest.mark.parametrize("wgs,groups", [(64, 3), (256, 0), (1024, 16)])
 @pytest.mark.parametrize("graph", ["rmat14", "grid", "gnp", "hubs"])
