@@ -7,6 +7,7 @@ import pytest
 
 import gpu_discovery_barrier_amd as gdb
 import oracle
+from conftest import csr_from_edges
 
 pytestmark = pytest.mark.gpu
 
@@ -257,3 +258,45 @@ def test_batch_rejects_lds_queue_outside_range(ctx, qcap):
         gdb.batch_solve(ctx, [gdb.make_task(gdb.TASK_BFS, dg, out, 0)], 1, gdb.Opts.make(wgs=128, groups=2,
                                                                                       lds_queue=qcap))
     assert e.value.code == gdb.GDB_E_INVALID
+
+
+def colour_graphs():
+    rng = np.random.default_rng(11)
+    perm = lambda n: (rng.permutation(n) / (n + 1)).astype(np.float32)
+    gs = [("grid256", gdb.gen_grid(256, 256, 0.0, seed=1), gdb.pannotia_values(65536)),
+          ("grid_perm", gdb.gen_grid(61, 90, 0.1, seed=2), perm(61 * 90)),
+          ("gnp40000", gdb.gen_gnp(40000, 8.0, seed=3), perm(40000)),  # first queues longer than the LDS list
+          ("gnp70000", gdb.gen_gnp(70000, 6.0, seed=4), perm(70000)),
+          ("rmat12", gdb.gen_rmat(12, 16, seed=5), perm(4096)),
+          ("star", star(5000), gdb.pannotia_values(5001)),
+          ("star_low_hub", star(5000), gdb.pannotia_values(5001)[::-1].copy())]
+    # Directed: a vertex's awaited neighbour may not list it.
+    src, dst = rng.integers(0, 3000, 9000), rng.integers(0, 3000, 9000)
+    src, dst = src[src != dst], dst[src != dst]
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=3000))]).astype(np.int32)
+    col = dst[order].astype(np.int32)
+    gs.append(("directed", gdb.CSR(3000, row, col, np.ones_like(col)), perm(3000)))
+    nv = perm(61 * 90)
+    nv[np.argsort(nv)[-2:]] = -2.0  # never coloured, and blocking nobody
+    gs.append(("uncolourable", gdb.gen_grid(61, 90, 0.1, seed=2), nv))
+    return gs
+
+
+def star(leaves):
+    edges = [(0, i) for i in range(1, leaves + 1)]
+    row, col, w = csr_from_edges(leaves + 1, edges)
+    return gdb.CSR(leaves + 1, row, col, w)
+
+
+@pytest.mark.parametrize("wgs,groups,team", [(64, 4, 1), (256, 0, 1), (512, 3, 1), (1024, 0, 1), (256, 8, 2)])
+def test_batch_colour_queue(ctx, wgs, groups, team):
+    tasks, outs = [], []
+    for name, g, nv in colour_graphs():
+        dg, out = gdb.DeviceCSR(g), gdb.DeviceBuffer.empty(g.n, np.int32)
+        tasks.append(gdb.make_task(gdb.TASK_COLOR, dg, out, node_value=gdb.DeviceBuffer.from_numpy(nv)))
+        outs.append((name, g, nv, out))
+    rounds, _ = gdb.batch_solve(ctx, tasks, team, gdb.Opts.make(wgs=wgs, groups=groups))
+    for (name, g, nv, out), r in zip(outs, rounds):
+        want, rr = oracle.color_ref(g.row, g.col, nv)
+        assert (out.to_numpy() == want).all() and r == rr, (name, r, rr)
