@@ -594,11 +594,23 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
           cls[j] = 0;
         }
         if constexpr (!WEIGHTED) {
-          // An unused slot compares against all ones, which no distance is.
+          // Most targets are reached already: a load first, and claims only from
+          // lanes that saw an unreached one (a stale load can only let a
+          // needless claim through).  A slot without one compares against
+          // all ones, which no distance is.
           unsigned old[kChunk];
+          bool any_need = false;
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j) old[j] = gdb::ldg(&dist[at[j]]);
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j) {
+            act[j] = act[j] && old[j] == kInf;
+            any_need |= act[j];
+          }
+          if (!any_need) return;
 #pragma unroll
           for (int j = 0; j < kChunk; ++j)
-            old[j] = gdb::atomic_cas_g(&dist[at[j]], act[j] ? kInf : ~0u, act[j] ? src_d : ~0u);
+            old[j] = gdb::atomic_cas_g(&dist[act[j] ? dst[j] : spare], act[j] ? kInf : ~0u, act[j] ? src_d : ~0u);
 #pragma unroll
           for (int j = 0; j < kChunk; ++j) cls[j] = (act[j] && old[j] == kInf) ? 1 : 0;
         } else {
@@ -618,13 +630,25 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
               if (imp[j] && nearp[j]) cls[j] = 3;
             }
           } else {
+            // As in the BFS: the distance word first, then the 64-bit minima
+            // from lanes with a candidate below it.
+            unsigned cur[kChunk];
+            bool any_need = false;
+#pragma unroll
+            for (int j = 0; j < kChunk; ++j) cur[j] = gdb::ldg(reinterpret_cast<unsigned*>(&d64[at[j]]) + 1);
+#pragma unroll
+            for (int j = 0; j < kChunk; ++j) {
+              act[j] = act[j] && cand[j] < cur[j];
+              any_need |= act[j];
+            }
+            if (!any_need) return;
             unsigned long long old[kChunk];
 #pragma unroll
             for (int j = 0; j < kChunk; ++j) {
               nearp[j] = cand[j] < thresh;
               const unsigned long long nw =
                   ((unsigned long long)cand[j] << 32) | (nearp[j] ? near_mark : far_mark);
-              old[j] = gdb::atomic_min_g(&d64[at[j]], act[j] ? nw : ~0ull);
+              old[j] = gdb::atomic_min_g(&d64[act[j] ? dst[j] : spare], act[j] ? nw : ~0ull);
             }
 #pragma unroll
             for (int j = 0; j < kChunk; ++j) {
@@ -1946,6 +1970,7 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
   if (!ctx || ntasks <= 0 || !tasks || team_groups < 0) return GDB_E_INVALID;
   gdb_opts o{};
   if (opts) o = *opts;
+  bool open_shape = false;  // the launch shape is the table's "batch" row
   {
     // A batch with an owner-partitioned task takes the "batch_owned" row
     // when the table has one (one group per CU), else the "batch" row.
@@ -1956,7 +1981,7 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
       any_owned |= tasks[t].owned != 0;
     }
     if (!any_owned || !apply_tuning("batch_owned", nmax, &o, &team_groups))
-      apply_tuning("batch", nmax, &o, &team_groups);
+      open_shape = apply_tuning("batch", nmax, &o, &team_groups) && !any_owned;
   }
   P->ctx = ctx;
   P->ntasks = ntasks;
@@ -1984,6 +2009,17 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
     return ((long long)a.n + a.m) * f;
   };
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost(x) > cost(y); });
+  // The table's shape is tuned for thousands of graphs.  Where the longest
+  // task takes a quarter or more of one CU's share of the work, its own time
+  // decides and one group per CU is faster (512 threads, one group per CU
+  // against two: 100 graphs 4.9 against 6.0 ms, 1024 graphs 15.0 against 16.8,
+  // 4096 graphs 62 against 53).
+  if (open_shape && P->G == 1) {
+    long long total = 0;
+    for (int t = 0; t < ntasks; ++t) total += cost(t);
+    if (4 * cost(order[0]) >= total / ctx->num_cus && (o.groups == 0 || o.groups > ctx->num_cus))
+      o.groups = ctx->num_cus;
+  }
   // Per-task scratch sizes (ints) and the device task table.
   std::vector<DevTask> dt((size_t)ntasks);
   std::vector<size_t> sints((size_t)ntasks);
