@@ -21,11 +21,11 @@
 //                      a thread walks its item's edges.
 //   tuned persistent - one barrier per iteration (queue tails rotate over
 //                      three slots so the reset of the next-next tail needs
-//                      no barrier); edges of long rows are walked by a whole
-//                      wave; pushes are compacted with ballot + one atomic per
-//                      wave.
+//                      no barrier); rows are walked by lanes, waves or in
+//                      pieces; pushes are staged in LDS.
 //   relaunch         - one launch per iteration with a host loop reading the
 //                      output size (the non-persistent schedule).
+#include <algorithm>
 #include <mutex>
 #include "graph_common.hpp"
 #include "runtime.hpp"
@@ -152,19 +152,37 @@ __global__ __launch_bounds__(WGS) void k_wl_plain(gdb_kernel_ctx_t* ctx, const i
   }
 }
 
+// Tuned persistent schedule.  What bounded it on skewed graphs was not the
+// edges but two serial points: one returning atomic on the queue's size per
+// wave step (about 8 ns each on one word, 0.5 M of them on R-MAT 20), and the
+// longest row, walked by one wave.  Pushes therefore collect in LDS and a group
+// reserves queue space for a batch of them at once; a row longer than kLongRow
+// is cut into pieces that all waves share in a second phase of the iteration
+// (one more barrier, only in iterations with such a row).  R-MAT 20 BFS: 4.3
+// ms -> 0.88 with 256 groups of 256 (2.0 with 64); R-MAT 18 SSSP: 4.0 -> 1.43
+// (1.76 with 128).
+constexpr int kLongRow = 1024;
+
 template <int WGS, bool WEIGHTED>
 __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                                   const int* __restrict__ col,
                                                   const int* __restrict__ w, unsigned* dist,
                                                   int* stamp, int* q0, int* q1, int* tails, int n,
-                                                  long long* work, int* out) {
+                                                  int4* pieces, int piece_cap, long long* work, int* out) {
   DISCOVERY_PROTOCOL(ctx);
+  constexpr int kStage = 8 * WGS;  // pushes of this group awaiting queue space
+  __shared__ int s_q[kStage];
+  __shared__ int s_n, s_base;
   const int tid = p_get_global_id(ctx, &local_ctx);
   const int threads = p_get_global_size(ctx, &local_ctx);
+  const int lane = gdb::lane_id(), wave = tid >> 6, nwaves = threads >> 6;
   const int spare = n > 0 ? (int)((unsigned)tid % (unsigned)n) : 0;
+  int* const piece_counts = tails + 3;  // rotating, like the tails
   int iteration = 1, nbar = 0;
   long long items = 0, edges = 0;
   int nin = gdb::ld_rlx(&tails[1]);
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
   while (nin > 0) {
     if (nin > n) {
       gdb::set_error(ctx, GDB_ERR_QUEUE_OVERFLOW);
@@ -173,8 +191,121 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
     const int* in = (iteration & 1) ? q0 : q1;
     int* outq = (iteration & 1) ? q1 : q0;
     int* out_tail = &tails[(iteration + 1) % 3];
-    if (tid == 0) gdb::st_rlx(&tails[(iteration + 2) % 3], 0);
+    int* npieces = &piece_counts[iteration % 3];
+    if (tid == 0) {
+      gdb::st_rlx(&tails[(iteration + 2) % 3], 0);
+      gdb::st_rlx(&piece_counts[(iteration + 1) % 3], 0);
+    }
     items += nin;
+    // Moves the staged pushes to the queue when more than `above` wait.  All
+    // threads of the group call it.
+    auto flush = [&](int above) {
+      __syncthreads();
+      const int c = min(s_n, kStage);
+      __syncthreads();
+      if (c <= above) return;
+      if (threadIdx.x == 0) {
+        s_base = gdb::fadd_rlx(out_tail, c);
+        s_n = 0;
+      }
+      __syncthreads();
+      for (int i = threadIdx.x; i < c; i += WGS) outq[s_base + i] = s_q[i];
+      __syncthreads();
+    };
+    // kChunk edges per lane step (long rows: the whole wave, carrying the
+    // row owner's distance): the column and weight loads, then the
+    // targets' distances, then atomics only where a candidate improves
+    // (lanes with none send no atomic), then the once-per-iteration stamps
+    // of the improved targets, then the pushes.  Unused slots read edge
+    // 0 and this thread's spare vertex, so that the slots stay branch-free.
+    auto step = [&](const bool (&ok)[kChunk], const int (&kk)[kChunk], int pd) -> int {
+      const unsigned src = (unsigned)pd;
+      int dst[kChunk];
+      bool push[kChunk];
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j) {
+        dst[j] = -1;
+        push[j] = false;
+      }
+      if (gdb::any_slot(ok)) {
+        unsigned wt[kChunk], cur[kChunk];
+        bool act[kChunk], need[kChunk];
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+          const int e0 = ok[j] ? kk[j] : 0;  // edge 0 exists here
+          dst[j] = gdb::ldg(col + e0);
+          wt[j] = WEIGHTED ? (unsigned)gdb::ldg(w + e0) : 1u;
+        }
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+          act[j] = ok[j] && (unsigned)dst[j] < (unsigned)n && wt[j] < kInf;
+          if (!ok[j]) dst[j] = -1;
+          cur[j] = gdb::ldg(dist + (act[j] ? dst[j] : spare));
+        }
+        // A stale distance is never below the current one, so it can
+        // only let a needless atomic through.
+        bool any_need = false;
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+          need[j] = act[j] && (WEIGHTED ? src + wt[j] < cur[j] : cur[j] == kInf);
+          any_need |= need[j];
+        }
+        if (any_need) {
+          unsigned old[kChunk];
+          bool imp[kChunk], any_imp = false;
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j) {
+            unsigned* dp = &dist[need[j] ? dst[j] : spare];
+            old[j] = WEIGHTED ? gdb::atomic_min_g(dp, need[j] ? src + wt[j] : ~0u)
+                              : gdb::atomic_cas_g(dp, need[j] ? kInf : ~0u, need[j] ? (unsigned)iteration : ~0u);
+          }
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j) {
+            imp[j] = need[j] && (WEIGHTED ? src + wt[j] < old[j] : old[j] == kInf);
+            any_imp |= imp[j];
+          }
+          if (!WEIGHTED) {
+#pragma unroll
+            for (int j = 0; j < kChunk; ++j) push[j] = imp[j];
+          } else if (any_imp) {
+            // Stamps only grow (iteration numbers): the first to raise
+            // one to this iteration queues the target.
+            int sp[kChunk];
+#pragma unroll
+            for (int j = 0; j < kChunk; ++j)
+              sp[j] = gdb::atomic_max_g(&stamp[imp[j] ? dst[j] : spare], imp[j] ? iteration : INT_MIN);
+#pragma unroll
+            for (int j = 0; j < kChunk; ++j) push[j] = imp[j] && sp[j] < iteration;
+          }
+        }
+      }
+      // Pushes, staged in LDS.
+      unsigned long long m[kChunk];
+      int cnt = 0;
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j) {
+        m[j] = __ballot(push[j]);
+        cnt += __popcll(m[j]);
+      }
+      if (cnt == 0) return 0;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&s_n, cnt);
+      base = gdb::bcast(base, 0);
+      const bool full = base + cnt > kStage;  // what does not fit goes straight to the queue
+      const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j) {
+        const int pos = base + __popcll(m[j] & lt);
+        if (push[j] && pos < kStage) {
+          s_q[pos] = dst[j];
+          push[j] = false;
+        }
+        base += __popcll(m[j]);
+      }
+      if (full) gdb::wave_push_n<kChunk>(push, dst, outq, out_tail);
+      return 0;
+    };
+    auto any = [](int a, int c) { return a | c; };
     GDB_FOR_UNIFORM(i, valid, tid, threads, nin) {
       int v = -1, b = 0, e = 0;
       unsigned dv = 0;
@@ -187,89 +318,47 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
         e = row[v + 1];
         if (WEIGHTED) dv = dist[v];
         edges += e - b;
+        if (e - b > kLongRow) {
+          const int k = (e - b + kLongRow - 1) / kLongRow;
+          const int at = gdb::fadd_rlx(npieces, k);
+          for (int j = 0; j < k && at + j < piece_cap; ++j, b += kLongRow)
+            pieces[at + j] = make_int4(b, min(e, b + kLongRow), (int)dv, 0);
+          valid = b < e;  // the part the list has no room for is walked here
+        }
       }
-      // kChunk edges per lane step (long rows: the whole wave, carrying the
-      // row owner's distance): the column and weight loads, then the
-      // targets' distances, then atomics only where a candidate improves
-      // (lanes with none send no atomic), then the once-per-iteration stamps
-      // of the improved targets, then one wave push.  Unused slots read edge
-      // 0 and this thread's spare vertex, so that the slots stay branch-free.
-      gdb::wave_walk_np<kChunk>(
-          valid != 0, b, e, (int)dv, 0,
-          [&](const bool (&ok)[kChunk], const int (&kk)[kChunk], int pd) -> int {
-            const unsigned src = (unsigned)pd;
-            int dst[kChunk];
-            bool push[kChunk];
-#pragma unroll
-            for (int j = 0; j < kChunk; ++j) {
-              dst[j] = -1;
-              push[j] = false;
-            }
-            if (gdb::any_slot(ok)) {
-              unsigned wt[kChunk], cur[kChunk];
-              bool act[kChunk], need[kChunk];
-#pragma unroll
-              for (int j = 0; j < kChunk; ++j) {
-                const int e0 = ok[j] ? kk[j] : 0;  // edge 0 exists here
-                dst[j] = gdb::ldg(col + e0);
-                wt[j] = WEIGHTED ? (unsigned)gdb::ldg(w + e0) : 1u;
-              }
-#pragma unroll
-              for (int j = 0; j < kChunk; ++j) {
-                act[j] = ok[j] && (unsigned)dst[j] < (unsigned)n && wt[j] < kInf;
-                if (!ok[j]) dst[j] = -1;
-                cur[j] = gdb::ldg(dist + (act[j] ? dst[j] : spare));
-              }
-              // A stale distance is never below the current one, so it can
-              // only let a needless atomic through.
-              bool any_need = false;
-#pragma unroll
-              for (int j = 0; j < kChunk; ++j) {
-                need[j] = act[j] && (WEIGHTED ? src + wt[j] < cur[j] : cur[j] == kInf);
-                any_need |= need[j];
-              }
-              if (any_need) {
-                unsigned old[kChunk];
-                bool imp[kChunk], any_imp = false;
-#pragma unroll
-                for (int j = 0; j < kChunk; ++j) {
-                  unsigned* dp = &dist[need[j] ? dst[j] : spare];
-                  old[j] = WEIGHTED ? gdb::atomic_min_g(dp, need[j] ? src + wt[j] : ~0u)
-                                    : gdb::atomic_cas_g(dp, need[j] ? kInf : ~0u, need[j] ? (unsigned)iteration : ~0u);
-                }
-#pragma unroll
-                for (int j = 0; j < kChunk; ++j) {
-                  imp[j] = need[j] && (WEIGHTED ? src + wt[j] < old[j] : old[j] == kInf);
-                  any_imp |= imp[j];
-                }
-                if (!WEIGHTED) {
-#pragma unroll
-                  for (int j = 0; j < kChunk; ++j) push[j] = imp[j];
-                } else if (any_imp) {
-                  // Stamps only grow (iteration numbers): the first to raise
-                  // one to this iteration queues the target.
-                  int sp[kChunk];
-#pragma unroll
-                  for (int j = 0; j < kChunk; ++j)
-                    sp[j] = gdb::atomic_max_g(&stamp[imp[j] ? dst[j] : spare], imp[j] ? iteration : INT_MIN);
-#pragma unroll
-                  for (int j = 0; j < kChunk; ++j) push[j] = imp[j] && sp[j] < iteration;
-                }
-              }
-            }
-            gdb::wave_push_n<kChunk>(push, dst, outq, out_tail);
-            return 0;
-          },
-          [](int a, int c) { return a | c; }, kSerialLimit);
+      gdb::wave_walk_np<kChunk>(valid != 0, b, e, (int)dv, 0, step, any, kSerialLimit);
+      flush(kStage / 2);
     }
+    flush(0);
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
+    const int np = min(gdb::ld_rlx(npieces), piece_cap);
+    if (np > 0) {
+      for (int p0 = 0; p0 < np; p0 += nwaves) {  // the same trips in every wave
+        const int p = p0 + wave;
+        const int4 pc = p < np ? pieces[p] : make_int4(0, 0, 0, 0);
+        for (int base = pc.x; base < pc.y; base += 64 * kChunk) {
+          bool ok[kChunk];
+          int kk[kChunk];
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j) {
+            kk[j] = base + lane + 64 * j;
+            ok[j] = kk[j] < pc.y;
+          }
+          step(ok, kk, pc.z);
+        }
+        flush(kStage / 2);
+      }
+      flush(0);
+      if (!discovery_barrier(ctx, &local_ctx)) return;
+      ++nbar;
+    }
     nin = gdb::ld_rlx(out_tail);
     ++iteration;
   }
   // Edges examined, summed over threads (one atomic per wave).
   for (int off = 32; off > 0; off >>= 1) edges += __shfl_xor(edges, off, 64);
-  if (gdb::lane_id() == 0 && edges) atomicAdd((unsigned long long*)&work[1], (unsigned long long)edges);
+  if (lane == 0 && edges) atomicAdd((unsigned long long*)&work[1], (unsigned long long)edges);
   if (tid == 0) {
     out[0] = iteration - 1;
     out[1] = nbar;
@@ -373,7 +462,15 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
     if (stats) *stats = st;
     return GDB_SUCCESS;
   }
-  const size_t bytes = carve_bytes<int>(n) * 3 + carve_bytes<int>(32) + carve_bytes<long long>(2);
+  const bool tuned_wl = o.variant == GDB_VARIANT_TUNED && o.schedule != GDB_SCHED_RELAUNCH;
+  // A row longer than kLongRow has at most 2 * edges / kLongRow pieces.
+  int piece_cap = tuned_wl ? (int)(2LL * m / kLongRow) + 1 : 0;
+  size_t bytes = carve_bytes<int>(n) * 3 + carve_bytes<int>(32) + carve_bytes<long long>(2);
+  if (fixed_ws) {  // the list takes what the caller's buffer has left
+    if (bytes > fixed_bytes) return GDB_E_SCRATCH;
+    piece_cap = (int)std::min<size_t>(piece_cap, (fixed_bytes - bytes) / sizeof(int4) & ~(size_t)15);
+  }
+  bytes += carve_bytes<int4>(piece_cap);
   void* base = fixed_ws;
   int rc = GDB_SUCCESS;
   if (base) {
@@ -389,8 +486,9 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   int* q1 = cv.take<int>(n);
   int* flags = cv.take<int>(32);
   long long* work = cv.take<long long>(2);
+  int4* pieces = cv.take<int4>(piece_cap);
   int* tails = flags + 4;
-  int* out = flags + 8;
+  int* out = flags + 12;
   rc = fill_i32(ctx, (int*)work, 0, 4);
   if (rc) return rc;
   hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, dist, stamp, q0, q1,
@@ -403,7 +501,7 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
     const int check = o.relaunch_check > 1 ? o.relaunch_check : 1;
     int grid = (n + wgs - 1) / wgs;
     if (grid > 4096) grid = 4096;
-    int* active = flags + 12;
+    int* active = flags + 14;
     rc = timer_start(ctx);
     if (rc) return rc;
     int it = 0;
@@ -438,7 +536,8 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
       if (r2) return r2;
       if (tuned)
         hipLaunchKernelGGL((k_wl_tuned<WG, WEIGHTED>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
-                           row, col, w, dist, stamp, q0, q1, tails, n, work, out);
+                           row, col, w, dist, stamp, q0, q1, tails, n, pieces, piece_cap,
+                           work, out);
       else
         hipLaunchKernelGGL((k_wl_plain<WG, WEIGHTED>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
                            row, col, w, dist, stamp, q0, q1, flags, n, out);

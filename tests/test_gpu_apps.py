@@ -326,3 +326,29 @@ def test_batch_multigraph_parallel_edges_with_different_weights(ctx, hops):
     gdb.batch_solve(ctx, tasks, 2, gdb.Opts.make(wgs=128, groups=4))
     assert (ob.to_numpy() == oracle.bfs_tb(row, col, 3)).all()
     assert (os_.to_numpy().astype(np.int64) == oracle.dijkstra_tb(row, col, w, 3)).all()
+
+
+@pytest.mark.parametrize("wgs,groups", [(64, 1), (64, 9), (256, 64), (1024, 4)])
+@pytest.mark.parametrize("leaves", [1023, 1024, 1025, 2049, 40000])
+def test_worklist_long_rows_and_stages(ctx, wgs, groups, leaves):
+    # Two hubs of `leaves` edges one level apart (rows at the edges of the
+    # per-wave and per-piece walks), whose leaves overflow a small group's
+    # push stage, then a second ring of vertices behind the leaves.
+    n = 2 + 2 * leaves
+    edges = [(0, 1)] + [(h, 2 + i) for h in range(2) for i in range(leaves)]
+    edges += [(2 + i, 2 + leaves + i) for i in range(leaves)]
+    src = np.array([a for a, _ in edges] + [b for _, b in edges], np.int64)
+    dst = np.array([b for _, b in edges] + [a for a, _ in edges], np.int64)
+    wt = np.random.default_rng(leaves).integers(1, 50, len(edges))
+    wt = np.concatenate([wt, wt])
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int32)
+    d = dev(row, dst[order].astype(np.int32), wt[order].astype(np.int32))
+    o = gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED)
+    source = n - 1
+    got_b, st = gdb.bfs_worklist(ctx, d, source, o)
+    want_b, iters = oracle.bfs_worklist_ref(row, dst[order].astype(np.int32), source)
+    assert (got_b == want_b).all() and st.rounds == iters
+    got_s, _ = gdb.sssp_worklist(ctx, d, source, o)
+    assert (got_s.astype(np.int64) == oracle.dijkstra_tb(row, dst[order].astype(np.int32),
+                                                          wt[order].astype(np.int32), source)).all()

@@ -57,3 +57,23 @@ def test_noalloc_refuses_inputs_above_the_limit():
         # The context is still usable afterwards.
         got, _ = solve(gdb.lib().gdb_sssp_worklist_noalloc, ctx, dg, out, SCHEDS[0])
         assert (got.astype(np.int64) == oracle.dijkstra_tb(g.row, g.col, g.w, 0)).all()
+
+
+def test_noalloc_rows_longer_than_its_piece_list():
+    # At the size limit the static array has room for the pieces of rows of
+    # about 230,000 edges: a longer row's rest is walked by its wave.
+    n, leaves = 1 << 22, 300000
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = leaves
+    row[2:] += 1  # vertex 1 continues to vertex n - 1
+    col = np.concatenate([np.arange(1, leaves + 1), [n - 1]]).astype(np.int32)
+    w = (1 + np.arange(leaves + 1) % 97).astype(np.int32)
+    with gdb.Context() as ctx:
+        dg = gdb.DeviceCSR(gdb.CSR(n, row, col, w))
+        out = gdb.DeviceBuffer.empty(n, np.uint32)
+        got, _ = solve(gdb.lib().gdb_sssp_worklist_noalloc, ctx, dg, out, SCHEDS[0])
+    want = np.full(n, gdb.LONESTAR_INF, np.uint32)
+    want[0] = 0
+    want[1:leaves + 1] = w[:leaves]
+    want[n - 1] = w[0] + w[leaves]
+    assert (got == want).all()
