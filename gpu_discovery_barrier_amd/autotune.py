@@ -127,15 +127,16 @@ def tune_mis_bc(ctx, quick=False):
 
 
 def tune_worklist(ctx, quick=False):
-    side = 1024 if quick else 2048
-    g = api.gen_grid(side, side, 0.05, seed=2, wlo=1, whi=255)
+    # A skewed graph: local ones (grids) take the owner-partitioned solve when
+    # the shape is left open, so the rows serve the others.
+    g = api.gen_rmat(16 if quick else 18, 16, seed=2, wlo=1, whi=100)
     dg = api.DeviceCSR(g)
     out = api.DeviceBuffer.empty(g.n, np.uint32)
     rows, trials = [], []
     for name, fn in (("bfs_wl", api.bfs_worklist), ("sssp_wl", api.sssp_worklist)):
         run = lambda w, gr: fn(ctx, dg, 0, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
                                out=out)[1].kernel_ms
-        r, t = tune_solver(ctx, name, 1 << 30, run, (256, 512), (64, 128, 256), repeats=1)
+        r, t = tune_solver(ctx, name, 1 << 30, run, (256, 512), (64, 128, 256, 512), repeats=3)
         rows.append(r)
         trials += t
     return rows, trials

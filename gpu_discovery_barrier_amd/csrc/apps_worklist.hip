@@ -23,6 +23,9 @@
 //                      three slots so the reset of the next-next tail needs
 //                      no barrier); rows are walked by lanes, waves or in
 //                      pieces; pushes are staged in LDS.
+//                      With the launch shape left open, a sparse graph whose
+//                      vertex ids follow locality takes the batched engine's
+//                      owner-partitioned ranges instead (solve_if_local).
 //   relaunch         - one launch per iteration with a host loop reading the
 //                      output size (the non-persistent schedule).
 #include <algorithm>
@@ -443,6 +446,126 @@ __global__ void k_verify(const int* __restrict__ row, const int* __restrict__ co
   if (bad) atomicAdd(nerr, bad);
 }
 
+// ---- local graphs: the owner-partitioned solve --------------------------------
+// A sample of the graph's edges: how many, how far apart their ends are (hist[b]:
+// |u - v| < 2^b and not less than 2^(b-1)), and the sum of their weights.
+struct Locality {
+  int hist[32];
+  int edges;
+  int pad;
+  unsigned long long wsum;
+};
+constexpr int kSampleVertices = 8192, kSampleEdges = 4;  // evenly spaced vertices, edges of each
+
+__global__ __launch_bounds__(256) void k_locality(const int* __restrict__ row, const int* __restrict__ col,
+                                                  const int* __restrict__ w, int n, Locality* out) {
+  __shared__ int s_hist[32];
+  if (threadIdx.x < 32) s_hist[threadIdx.x] = 0;
+  __syncthreads();
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int count = n < kSampleVertices ? n : kSampleVertices;
+  int edges = 0;
+  unsigned long long ws = 0;
+  if (i < count) {
+    const int v = (int)((long long)i * n / count);
+    const int b = row[v], e = min(row[v + 1], b + kSampleEdges);
+    for (int k = b; k < e; ++k) {
+      const int d = abs(col[k] - v);
+      atomicAdd(&s_hist[d == 0 ? 0 : 32 - __clz(d)], 1);
+      ++edges;
+      if (w) ws += min((unsigned)w[k], kInf);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    edges += __shfl_xor(edges, off, 64);
+    ws += __shfl_xor(ws, off, 64);
+  }
+  if (gdb::lane_id() == 0 && edges) {
+    atomicAdd(&out->edges, edges);
+    if (w) atomicAdd(&out->wsum, ws);
+  }
+  __syncthreads();
+  if (threadIdx.x < 32 && s_hist[threadIdx.x]) atomicAdd(&out->hist[threadIdx.x], s_hist[threadIdx.x]);
+}
+
+// Largest finite distance plus one: the iterations of a BFS worklist.
+__global__ void k_levels(const unsigned* __restrict__ dist, int n, int* out) {
+  int m = 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    if (dist[i] < kInf) m = max(m, (int)dist[i] + 1);
+  m = gdb::wave_max(m);
+  if (gdb::lane_id() == 0 && m > 0) atomicMax(out, m);
+}
+
+// Solves a sparse local graph (grids, meshes, road networks) by the batched
+// engine's owner-partitioned ranges: such a graph has thousands of short
+// iterations, and there a hop inside a range costs an LDS round instead of
+// an inter-group barrier.  *done is false when the graph is none.
+//
+// The rule: at most kLocalDegree edges per vertex (denser graphs, the sample's
+// cost not spent on them, are skewed or random in use, and a slot record holds
+// four edges), and 98% of the sampled edges shorter than half a range.  Ranges
+// of kLocalRange vertices, one group each (1024^2 grid: 64 ranges 4.63 ms,
+// 128 4.92, 256 6.0; 128^2: 1 to 8 within 10%), at most one per CU.  SSSP
+// bands of 96 mean weights (24 to 200 measured, within 15%).  1024^2 grid:
+// SSSP 33.4 ms with iteration queues, 4.7 here; BFS 13.7 and 2.7; a 64^2 grid
+// 0.57 and 0.20, 0.46 and 0.15.
+constexpr int kLocalDegree = 6, kLocalRange = 12288, kLocalBand = 96;
+constexpr int kLocalRangeMax = 30000;  // distances, marks, queues and boundary list of a range fit a CU's LDS
+
+template <bool WEIGHTED>
+int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const int* w, int source,
+                   unsigned* dist, gdb_stats* st, bool* done) {
+  using namespace gdbrt;
+  *done = false;
+  if (ctx->xcd_only >= 0 || (long long)m > (long long)kLocalDegree * n || m < n / 2) return GDB_SUCCESS;
+  int rc = ensure_workspace(ctx, sizeof(Locality));
+  if (rc) return rc;
+  Locality* d = (Locality*)ctx->ws;
+  rc = fill_i32(ctx, (int*)d, 0, sizeof(Locality) / sizeof(int));
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_locality, dim3(kSampleVertices / 256), dim3(256), 0, ctx->stream, row, col,
+                     WEIGHTED ? w : nullptr, n, d);
+  GDB_HIP(hipGetLastError());
+  Locality h;
+  GDB_HIP(hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+  GDB_HIP(hipStreamSynchronize(ctx->stream));
+  if (h.edges == 0) return GDB_SUCCESS;
+  const int G = std::max(1, std::min(ctx->num_cus, (n + kLocalRange - 1) / kLocalRange));
+  const int range = (n + G - 1) / G;
+  long long near = 0;
+  for (int b = 0; b < 31 && (1LL << b) <= range / 2; ++b) near += h.hist[b];
+  if (near * 100 < 98LL * h.edges || range > kLocalRangeMax) return GDB_SUCCESS;
+  gdb_task t{};
+  t.algo = WEIGHTED ? GDB_TASK_SSSP : GDB_TASK_BFS;
+  t.n = n;
+  t.m = m;
+  t.row = row;
+  t.col = col;
+  t.w = w;
+  t.source = source;
+  t.out = dist;
+  t.delta = WEIGHTED ? (int)std::min<unsigned long long>(kInf, 1 + kLocalBand * h.wsum / (unsigned)h.edges) : 0;
+  t.owned = 1;
+  gdb_opts o{};
+  o.wgs = 1024;
+  o.groups = G;
+  o.barrier = -1;
+  rc = gdb_batch_solve(ctx, &t, 1, G, &o, st);
+  if (rc) return rc;
+  if (!WEIGHTED) {
+    int* levels = (int*)ctx->ws;
+    rc = fill_i32(ctx, levels, 0, 1);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_levels, dim3(std::min(256, (n + 255) / 256)), dim3(256), 0, ctx->stream, dist, n, levels);
+    GDB_HIP(hipGetLastError());
+    GDB_HIP(hipMemcpyAsync(&st->rounds, levels, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    GDB_HIP(hipStreamSynchronize(ctx->stream));
+  }
+  *done = true;
+  return GDB_SUCCESS;
+}
+
 // `fixed_ws`: a caller-provided device buffer of `fixed_bytes` bytes that
 // replaces the context's grow-only workspace (no allocation), or nullptr.
 template <bool WEIGHTED>
@@ -461,6 +584,16 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   if (n == 0) {
     if (stats) *stats = st;
     return GDB_SUCCESS;
+  }
+  if (opts && opts->wgs == 0 && opts->groups == 0 && o.variant == GDB_VARIANT_TUNED &&
+      o.schedule == GDB_SCHED_PERSISTENT && !fixed_ws) {
+    bool done = false;
+    const int lrc = solve_if_local<WEIGHTED>(ctx, n, m, row, col, w, source, dist, &st, &done);
+    if (lrc || done) {
+      if (stats) *stats = st;
+      return lrc;
+    }
+    st = gdb_stats{};
   }
   const bool tuned_wl = o.variant == GDB_VARIANT_TUNED && o.schedule != GDB_SCHED_RELAUNCH;
   // A row longer than kLongRow has at most 2 * edges / kLongRow pieces.

@@ -352,3 +352,53 @@ def test_worklist_long_rows_and_stages(ctx, wgs, groups, leaves):
     got_s, _ = gdb.sssp_worklist(ctx, d, source, o)
     assert (got_s.astype(np.int64) == oracle.dijkstra_tb(row, dst[order].astype(np.int32),
                                                           wt[order].astype(np.int32), source)).all()
+
+
+def local_graph(name):
+    rng = np.random.default_rng(7)
+    if name == "path":
+        n = 5000
+        src = np.arange(n - 1)
+        return csr_directed(n, np.concatenate([src, src + 1]), np.concatenate([src + 1, src]), rng, 100)
+    if name == "chain_one_way":  # reached from the low end only
+        return csr_directed(3000, np.arange(2999), np.arange(1, 3000), rng, 9)
+    if name == "band6":  # six edges a vertex, up to 40 apart, parallel edges and self-loops kept
+        src = np.repeat(np.arange(20000), 6)
+        return csr_directed(20000, src, np.clip(src + rng.integers(-40, 41, src.size), 0, 19999), rng, 50)
+    if name == "grid_shuffled":  # the same grid without locality: iteration queues
+        g = gdb.gen_grid(150, 150, 0.05, seed=3, wlo=1, whi=255)
+        g = g.relabel(gdb.permutation(g.n, 5))
+        return g.row, g.col, g.w
+    rows, cols, hole, whi = {"grid": (160, 97, 0.05, 255), "holes": (120, 130, 0.35, 10), "tall": (2000, 7, 0.0, 3),
+                             "wide": (3, 9001, 0.0, 255), "two_ranges": (128, 110, 0.0, 100),
+                             "tiny": (2, 3, 0.0, 5)}[name]
+    g = gdb.gen_grid(rows, cols, hole, seed=4, wlo=1, whi=whi)
+    return g.row, g.col, g.w
+
+
+def csr_directed(n, src, dst, rng, whi):
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int32)
+    return row, dst[order].astype(np.int32), rng.integers(0, whi, src.size).astype(np.int32)
+
+
+@pytest.mark.parametrize("name", ["path", "chain_one_way", "band6", "grid_shuffled", "grid", "holes", "tall", "wide",
+                                  "two_ranges", "tiny"])
+def test_worklist_open_shape_on_local_graphs(ctx, name):
+    # The shape left open takes the owner-partitioned solve on local graphs:
+    # equal to the iteration queues (a given shape) and to the oracle, for the
+    # first, a middle and the last vertex as the source.
+    row, col, w = local_graph(name)
+    n = row.size - 1
+    if name == "band6":
+        w[::1000] = 2000000000  # at or above the unreachable distance: never relaxed
+    d = dev(row, col, w)
+    for source in (0, n // 2, n - 1):
+        want_b, iters = oracle.bfs_worklist_ref(row, col, source)
+        want_s, _ = oracle.sssp_worklist_ref(row, col, w, source)
+        for wgs, groups in ((0, 0), (256, 64)):
+            o = gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED)
+            got_b, st = gdb.bfs_worklist(ctx, d, source, o)
+            assert (got_b == want_b).all() and st.rounds == iters, (name, source, wgs)
+            got_s, _ = gdb.sssp_worklist(ctx, d, source, o)
+            assert (got_s == want_s).all(), (name, source, wgs)
