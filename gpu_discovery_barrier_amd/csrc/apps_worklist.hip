@@ -162,8 +162,8 @@ __global__ __launch_bounds__(WGS) void k_wl_plain(gdb_kernel_ctx_t* ctx, const i
 // reserves queue space for a batch of them at once; a row longer than kLongRow
 // is cut into pieces that all waves share in a second phase of the iteration
 // (one more barrier, only in iterations with such a row).  R-MAT 20 BFS: 4.3
-// ms -> 0.88 with 256 groups of 256 (2.0 with 64); R-MAT 18 SSSP: 4.0 -> 1.43
-// (1.76 with 128).
+// ms -> 0.88 with 256 groups of 256 (2.0 with 64), 0.64 with 512-thread groups and
+// the queue's items dealt to the waves; R-MAT 18 SSSP: 4.0 -> 1.43 -> 0.86.
 constexpr int kLongRow = 1024;
 
 template <int WGS, bool WEIGHTED>
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
       return 0;
     };
     auto any = [](int a, int c) { return a | c; };
-    GDB_FOR_UNIFORM(i, valid, tid, threads, nin) {
+    GDB_FOR_SPREAD(i, valid, tid, threads, nin) {
       int v = -1, b = 0, e = 0;
       unsigned dv = 0;
       if (valid) {
