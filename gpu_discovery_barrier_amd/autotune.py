@@ -122,7 +122,7 @@ def tune_mis_bc(ctx, quick=False):
     bout = api.DeviceBuffer.empty(g.n, np.float32)
     bc = lambda w, gr: api.bc(ctx, dg, dg, src, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
                               out=bout)[1].kernel_ms
-    r2, t2 = tune_solver(ctx, "bc", 1 << 30, bc, (256, 512), (1024, 2048), repeats=1)
+    r2, t2 = tune_solver(ctx, "bc", 1 << 30, bc, (256, 512), (256, 512, 1024), repeats=1)
     return [r1, r2], t1 + t2
 
 

@@ -824,7 +824,7 @@ extern "C" int gdb_bc(gdb_ctx* ctx, int n, int m, const int* row, const int* col
                          : tuned ? (const void*)k_bc_tuned<WG>
                                  : (const void*)k_bc_plain<WG>;
       int groups = 0;
-      int r2 = launch_groups(ctx, kern, &o, n, &groups);
+      int r2 = launch_groups(ctx, kern, &o, tuned ? row_walk_items(n, m, wgs) : n, &groups);
       if (r2) return r2;
       r2 = timer_start(ctx);
       if (r2) return r2;

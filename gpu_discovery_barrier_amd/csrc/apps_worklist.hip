@@ -663,7 +663,7 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
       constexpr int WG = decltype(W)::value;
       const void* kern = tuned ? (const void*)k_wl_tuned<WG, WEIGHTED> : (const void*)k_wl_plain<WG, WEIGHTED>;
       int groups = 0;
-      int r2 = launch_groups(ctx, kern, &o, n, &groups);
+      int r2 = launch_groups(ctx, kern, &o, tuned ? row_walk_items(n, m, wgs) : n, &groups);
       if (r2) return r2;
       r2 = timer_start(ctx);
       if (r2) return r2;

@@ -402,3 +402,24 @@ def test_worklist_open_shape_on_local_graphs(ctx, name):
             assert (got_b == want_b).all() and st.rounds == iters, (name, source, wgs)
             got_s, _ = gdb.sssp_worklist(ctx, d, source, o)
             assert (got_s == want_s).all(), (name, source, wgs)
+
+
+@pytest.mark.parametrize("wgs,groups", [(0, 0), (64, 2), (256, 64)])
+@pytest.mark.parametrize("leaves", [16, 17, 1024, 1025, 2500])
+def test_sssp_pull_row_lengths(ctx, wgs, groups, leaves):
+    # A hub that gathers from `leaves` vertices, which it reaches through a
+    # second hub: in-edge rows at the edges of the per-lane, per-wave and
+    # per-piece walks, with the change in the last edge of the long row.
+    n = leaves + 3
+    rng = np.random.default_rng(leaves)
+    src = np.concatenate([np.arange(1, leaves + 1), np.zeros(leaves, np.int64), [leaves + 1, 0]])
+    dst = np.concatenate([np.full(leaves, leaves + 1), np.arange(1, leaves + 1), [leaves + 2, leaves + 2]])
+    wt = np.concatenate([rng.integers(5, 90, leaves), rng.integers(5, 90, leaves), [1, 500]])
+    wt[leaves - 1] = wt[2 * leaves - 1] = 1  # the shortest way runs over the last leaf
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int32)
+    gt = gdb.CSR(n, row, dst[order].astype(np.int32), wt[order].astype(np.int32)).transpose()
+    want, rounds = oracle.sssp_pull_ref(gt.row, gt.col, gt.w, 0)
+    got, st = gdb.sssp_pull(ctx, dev(gt.row, gt.col, gt.w), 0, gdb.Opts.make(wgs=wgs, groups=groups,
+                                                                            variant=gdb.VARIANT_TUNED))
+    assert (got == want).all() and st.rounds == rounds
