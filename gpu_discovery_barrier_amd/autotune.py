@@ -116,7 +116,7 @@ def tune_mis_bc(ctx, quick=False):
     out = api.DeviceBuffer.empty(g.n, np.int32)
     mis = lambda w, gr: api.mis(ctx, dg, nv, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
                                 out=out)[1].kernel_ms
-    r1, t1 = tune_solver(ctx, "mis", 1 << 30, mis, (256, 512, 1024), (512, 1024, 2048, 4096))
+    r1, t1 = tune_solver(ctx, "mis", 1 << 30, mis, (256, 512, 1024), (256, 512, 1024, 2048))
     deg = np.diff(g.row)
     src = np.sort(np.random.default_rng(3).choice(np.flatnonzero(deg > 0), 16, replace=False)).astype(np.int32)
     bout = api.DeviceBuffer.empty(g.n, np.float32)

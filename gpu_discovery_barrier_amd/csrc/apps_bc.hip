@@ -173,7 +173,7 @@ __global__ __launch_bounds__(WGS) void k_bc_tuned(gdb_kernel_ctx_t* ctx, const i
     // same tail after each barrier.
     int lb = 0, le = 1, l = 0;
     for (;;) {
-      GDB_FOR_SPREAD(i, valid, tid, stride, le - lb) {
+      GDB_FOR_SPREAD(i, valid, tid, stride, le - lb, 0) {
         int v = -1, b = 0, e = 0;
         if (valid) {
           v = q[lb + i];
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(WGS) void k_bc_tuned(gdb_kernel_ctx_t* ctx, const i
         if (((unsigned)v < (unsigned)n ? ds[v].x : -1) < ll + 1) lo = mid + 1; else hi = mid;
       }
       const int qe = lo;
-      GDB_FOR_SPREAD(i, valid, tid, stride, qe - qb) {
+      GDB_FOR_SPREAD(i, valid, tid, stride, qe - qb, 0) {
         int w = -1, b = 0, e = 0;
         if (valid) {
           w = q[qb + i];
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     for (;;) {
       const unsigned par = (unsigned)(t - 1) & 3u;                    // parents' level mod 4
       const unsigned nxt_nib = 8u | ((unsigned)(t + 1) & 3u);         // a claimed nibble
-      GDB_FOR_SPREAD(i, valid, tid, stride, le - lb) {
+      GDB_FOR_SPREAD(i, valid, tid, stride, le - lb, 0) {
         int v = -1, b = 0, e = 0;
         unsigned mask = 0;
         if (valid) {
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     for (int tt = t; tt >= 0; --tt) {
       const int qb = tt == t ? lb : loff[tt];
       const int qe = tt == t ? le : loff[tt + 1];
-      GDB_FOR_SPREAD(i, valid, tid, stride, qe - qb) {
+      GDB_FOR_SPREAD(i, valid, tid, stride, qe - qb, 0) {
         int v = -1, b = 0, e = 0;
         unsigned mask = 0;
         Half sv;

@@ -85,6 +85,9 @@ __global__ __launch_bounds__(WGS) void k_mis_plain(gdb_kernel_ctx_t* ctx, const 
 
 constexpr int kSlots = 4;  // edges a lane gathers per step in the tuned walks
 
+// What bounds it: random gathers, three dependent ones per walk step, and the
+// waves with the most long rows.  R-MAT 22: 3.1 ms with the vertices dealt to the
+// waves one by one (4.3 with 64 neighbours each).
 // Packed per-vertex state for one 8-byte gather per edge: x = status
 // (-1 undecided, -2 decided), y = node_value bits.
 template <int WGS>
@@ -99,6 +102,7 @@ __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const 
   // Unused edge slots gather this thread's spare vertex, so that a step's
   // loads are issued branch-free, before any of them is used.
   const int spare = n > 0 ? (int)((unsigned)tid % (unsigned)n) : 0;
+  const int sh = gdb::spread_rows(n, row[n]);
   int* qin = q0;
   int* qout = q1;
   int rounds = 0, nbar = 0;
@@ -115,7 +119,7 @@ __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const 
       break;
     }
     // Phase A: minimum over undecided neighbours, join decision.
-    GDB_FOR_UNIFORM(i, valid, tid, stride, qn) {
+    GDB_FOR_SPREAD(i, valid, tid, stride, qn, rounds == 1 ? sh : 0) {
       int v = -1, b = 0, e = 0;
       if (valid) {
         v = rounds == 1 ? i : qin[i];
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const 
     ++nbar;
     // Phase B: retire joiners and their neighbours, compact survivors.
     int* tail = &tails[rounds % 3];
-    GDB_FOR_UNIFORM(i, valid, tid, stride, qn) {
+    GDB_FOR_SPREAD(i, valid, tid, stride, qn, rounds == 1 ? sh : 0) {
       int v = -1, b = 0, e = 0;
       bool joined = false;
       if (valid) {
@@ -329,7 +333,7 @@ extern "C" int gdb_mis(gdb_ctx* ctx, int n, int m, const int* row, const int* co
       constexpr int WG = decltype(W)::value;
       const void* kern = tuned ? (const void*)k_mis_tuned<WG> : (const void*)k_mis_plain<WG>;
       int groups = 0;
-      int r2 = launch_groups(ctx, kern, &o, n, &groups);
+      int r2 = launch_groups(ctx, kern, &o, tuned ? row_walk_items(n, m, wgs) : n, &groups);
       if (r2) return r2;
       r2 = timer_start(ctx);
       if (r2) return r2;

@@ -29,8 +29,8 @@
 // pieces of kLongRow edges spread over all waves (a skewed graph's longest row
 // has as many edges as a thousand others); a vertex or piece without a cross
 // edge never gets one again and is left out of later rounds.  R-MAT 18 (7.6 M
-// edges, longest row 25 k): 0.93 ms (one lane walking each row twice per
-// round, six barriers: 46.4 ms).  Walking the rows of a wave as one list, with
+// edges, longest row 25 k): 0.60 ms (one lane walking each row twice per
+// round, six barriers: 46.4 ms; vertices 64 at a time: 0.93).  Walking the rows of a wave as one list, with
 // the minima in LDS, took 1.07 ms: the search for each edge's row costs more
 // than the steps it saves.
 #include "graph_common.hpp"
@@ -93,6 +93,7 @@ __global__ __launch_bounds__(WGS) void k_mst(gdb_kernel_ctx_t* ctx, const int* _
   const int lane = gdb::lane_id();
   const int wave = tid >> 6, nwaves = stride >> 6;
   const int spare = (int)((unsigned)tid % (unsigned)n);
+  const int sh = gdb::spread_rows(n, row[n]);
   int rounds = 0, nbar = 0;
   u64 wsum = 0;
   int added = 0;
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(WGS) void k_mst(gdb_kernel_ctx_t* ctx, const int* _
     };
     auto least = [](u64 a, u64 c) { return a < c ? a : c; };
     // 1: rows of up to kLongRow edges, then the pieces of the longer ones.
-    GDB_FOR_UNIFORM(v, valid, tid, stride, n) {
+    GDB_FOR_SPREAD(v, valid, tid, stride, n, sh) {
       int b = 0, e = 0, cv = 0;
       if (valid && !dead[v]) {
         cv = comp[v];
@@ -279,7 +280,7 @@ extern "C" int gdb_mst(gdb_ctx* ctx, int n, int m, const int* row, const int* co
   rc = gdb_dispatch_wgs(wgs, [&](auto W) -> int {
     constexpr int WG = decltype(W)::value;
     int groups = 0;
-    int r2 = launch_groups(ctx, (const void*)k_mst<WG>, &o, n, &groups);
+    int r2 = launch_groups(ctx, (const void*)k_mst<WG>, &o, row_walk_items(n, m, wgs), &groups);
     if (r2) return r2;
     r2 = timer_start(ctx);
     if (r2) return r2;

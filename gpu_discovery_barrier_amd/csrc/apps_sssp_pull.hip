@@ -73,7 +73,7 @@ __global__ __launch_bounds__(WGS) void k_sssp_pull_plain(gdb_kernel_ctx_t* ctx, 
 // waves, which meet in cur[v] by atomic minima: cur holds b_{k-2}, never below
 // b_{k-1}, so it needs no reset, and the minimum of the pieces and b_{k-1} is
 // b_k.  What bounds a round is the wave with the most long rows.  R-MAT 16 (longest
-// row 7 k, ten rounds): 0.70 ms against 1.15 with each row on one wave, one edge
+// row 7 k, ten rounds): 0.43 ms against 1.15 with each row on one wave, one edge
 // per lane and step.
 constexpr int kSlots = 4;
 constexpr int kLongRow = 1024;
@@ -89,6 +89,7 @@ __global__ __launch_bounds__(WGS) void k_sssp_pull_tuned(gdb_kernel_ctx_t* ctx, 
   const int tid = p_get_global_id(ctx, &local_ctx);
   const int stride = p_get_global_size(ctx, &local_ctx);
   const int lane = gdb::lane_id(), wave = tid >> 6, nwaves = stride >> 6;
+  const int sh = gdb::spread_rows(n, row_t[n]);
   int K = 0, nbar = 0, np = 0;
   for (int k = 1; k < n; ++k) {
     K = k;
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(WGS) void k_sssp_pull_tuned(gdb_kernel_ctx_t* ctx, 
       return mn;
     };
     auto least = [](int a, int c) { return a < c ? a : c; };
-    GDB_FOR_SPREAD(v, valid, tid, stride, n) {
+    GDB_FOR_SPREAD(v, valid, tid, stride, n, sh) {
       int b = 0, e = 0;
       bool mine = valid != 0;
       if (valid) {

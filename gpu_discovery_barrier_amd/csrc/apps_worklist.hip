@@ -309,7 +309,7 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
       return 0;
     };
     auto any = [](int a, int c) { return a | c; };
-    GDB_FOR_SPREAD(i, valid, tid, threads, nin) {
+    GDB_FOR_SPREAD(i, valid, tid, threads, nin, 0) {
       int v = -1, b = 0, e = 0;
       unsigned dv = 0;
       if (valid) {

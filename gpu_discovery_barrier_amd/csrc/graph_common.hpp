@@ -345,18 +345,30 @@ __device__ __forceinline__ T wave_walk_n(bool active, int b, int e, T identity, 
              valid = (_base + (long long)threadIdx.x) < (long long)(n);          \
          _once; _once = 0)
 
-// The same trips over the items [0, n) of a queue, dealt to the waves one by
-// one (lane l of wave w takes item w + l * waves) instead of 64 at a time.  A
-// wave walks its long rows one after the other, so in a queue shorter than the
-// grid some waves would walk 64 rows and the others none.  R-MAT 22 BC of 16
-// sources: 86 -> 33 ms, R-MAT 18 SSSP 1.4 -> 0.97.  (For loops over all
-// vertices it gains nothing and their words are no longer read 64 at a time.)
-__device__ __forceinline__ long long spread_item(int start, int stride) {
-  return (long long)lane_id() * (stride >> 6) + (start >> 6);
+// The same trips over the items [0, n), dealt to the waves 2^SH at a time
+// (SH 0 to 6) instead of 64 at a time, in another order for each of a wave's
+// shares.  A wave walks its long rows one after the other, so neighbouring
+// items are better spread: in a queue shorter than the grid some waves would
+// walk 64 rows and the others none, and in a skewed graph long rows are
+// neighbours, or, as in an R-MAT graph, share low bits of their ids (dealt in
+// a fixed order, a wave would get all of one residue).  Measured: R-MAT 22 BC
+// of 16 sources 86 -> 33 ms, R-MAT 18 SSSP 1.4 -> 0.97 (queues); R-MAT 18 MST
+// 0.93 -> 0.63, R-MAT 16 pull SSSP 0.69 -> 0.43 (all vertices, where a fixed
+// order gained nothing).  SH = 6 keeps a wave's 64 items together: short rows,
+// whose words it then reads in one line.
+__device__ __forceinline__ long long spread_item(int start, int stride, int sh) {
+  const unsigned waves = (unsigned)stride >> 6, l = (unsigned)lane_id(), share = l >> sh;
+  const unsigned turn = (waves * 5u / 8u) | 1u;
+  return (((long long)share * waves + ((unsigned)start / 64u + share * turn) % waves) << sh) + (l & ((1u << sh) - 1u));
 }
-#define GDB_FOR_SPREAD(i, valid, start, stride, n)                              \
-  for (long long _base = 0, _at = gdb::spread_item((start), (stride)); _base < (long long)(n); \
+#define GDB_FOR_SPREAD(i, valid, start, stride, n, SH)                          \
+  for (long long _base = 0, _at = gdb::spread_item((start), (stride), (SH)); _base < (long long)(n); \
        _base += (long long)(stride))                                            \
     for (int _once = 1, i = (int)(_base + _at), valid = _base + _at < (long long)(n); _once; _once = 0)
+// SH of a loop over all vertices of a graph of n vertices and m edges: one by
+// one where rows are long enough to be walked by waves (four or eight at a time
+// measured 2 to 25% slower on R-MAT graphs), 64 together where they are short
+// (2^20-vertex grid MST 1.16 ms against 1.44).
+__device__ __forceinline__ int spread_rows(int n, long long m) { return m >= 8LL * n ? 0 : 6; }
 
 }  // namespace gdb
