@@ -24,6 +24,7 @@
 // (selector.hpp) and publishes it with the release.  All arms reach the same
 // fixpoint, so outputs do not depend on the choices.
 #include <algorithm>
+#include <cstring>
 
 #include "graph_common.hpp"
 #include "runtime.hpp"
@@ -2021,7 +2022,9 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
       o.groups = ctx->num_cus;
   }
   // Per-task scratch sizes (ints) and the device task table.
-  std::vector<DevTask> dt((size_t)ntasks);
+  int rc = ensure_stage(ctx, sizeof(DevTask) * (size_t)ntasks);
+  if (rc) return rc;
+  DevTask* const dt = (DevTask*)ctx->h_stage;
   std::vector<size_t> sints((size_t)ntasks);
   size_t scratch_total = 0;
   for (int t = 0; t < ntasks; ++t) {
@@ -2056,7 +2059,7 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
   const size_t sel_bytes = (cfg.mode == GDB_SEL_MLP && cfg.w) ? sizeof(unsigned short) * gdbsel::kParams : 0;
   P->region = (int)(sizeof(int) * 2 * (size_t)P->qcap);
   if (P->owned_kernel) P->region = std::max<int>(P->region, (int)kOwnedLdsTotal);
-  int rc = gdb_dispatch_wgs(P->wgs, [&](auto W) -> int {
+  rc = gdb_dispatch_wgs(P->wgs, [&](auto W) -> int {
     constexpr int WG = decltype(W)::value;
     const void* kern = cfg.mode != GDB_SEL_NONE ? (const void*)k_batch<WG, true>
                        : P->owned_kernel        ? (const void*)k_batch<WG, false, true>
@@ -2106,17 +2109,16 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
     dt[t].scratch = scratch + off;
     off += sints[t];
   }
-  GDB_HIP(hipMemcpyAsync(P->d_tasks, dt.data(), sizeof(DevTask) * ntasks, hipMemcpyHostToDevice, ctx->stream));
-  GDB_HIP(hipStreamSynchronize(ctx->stream));  // dt is a local copy
+  GDB_HIP(hipMemcpyAsync(P->d_tasks, dt, sizeof(DevTask) * ntasks, hipMemcpyHostToDevice, ctx->stream));
+  // A graph is planned without being launched: its upload ends here.
+  if (own_memory) GDB_HIP(hipStreamSynchronize(ctx->stream));
   return GDB_SUCCESS;
 }
 
-// Clears the team state, counters and work words, and the context's error
-// word (kernels only, so that the sequence can be captured in a graph).
+// Clears the team state, counters and work words (one array), and the context's
+// error word (kernels only, so that the sequence can be captured in a graph).
 int enqueue_prep(const BatchPlan& P) {
-  int rc = fill_i32(P.ctx, P.team_state, 0, (long long)P.team_ints);
-  if (!rc) rc = fill_i32(P.ctx, P.misc, 0, P.ntasks + 64);
-  if (!rc) rc = fill_i32(P.ctx, (int*)P.work, 0, 16 * (long long)P.ntasks);
+  int rc = fill_i32(P.ctx, P.team_state, 0, (int*)(P.work + 8 * (size_t)P.ntasks) - P.team_state);
   if (!rc) rc = prepare_launch(P.ctx);
   return rc;
 }
@@ -2145,19 +2147,27 @@ int enqueue_kernel(const BatchPlan& P) {
   });
 }
 
-// Copies rounds, work and per-task times back into the caller's tasks.
+// Stops the timer, waits, and copies rounds, work and per-task times back into the
+// caller's tasks.
 int collect_batch(const BatchPlan& P, gdb_task* tasks, gdb_stats* st) {
   gdb_ctx* ctx = P.ctx;
   const int ntasks = P.ntasks;
-  std::vector<int> hres((size_t)ntasks);
-  std::vector<unsigned long long> hwork((size_t)8 * ntasks);
-  GDB_HIP(hipMemcpy(hres.data(), P.misc + 64, sizeof(int) * ntasks, hipMemcpyDeviceToHost));
-  GDB_HIP(hipMemcpy(hwork.data(), P.work, sizeof(unsigned long long) * 8 * ntasks, hipMemcpyDeviceToHost));
+  // Results and work words lie side by side: few of them come with the words
+  // that finish_launch collects, more in one copy.
+  const int* const first = P.misc + 64;
+  const size_t nwords = (int*)(P.work + 8 * (size_t)ntasks) - first, work_at = (int*)P.work - first;
+  const bool few = nwords <= (size_t)kCollectMax;
+  int rc = finish_launch(ctx, &st->kernel_ms, first, few ? (int)nwords : 0);
+  if (rc) return rc;
+  std::vector<int> copy(few ? 0 : nwords);
+  if (!few) GDB_HIP(hipMemcpy(copy.data(), first, sizeof(int) * nwords, hipMemcpyDeviceToHost));
+  const int* const h = few ? collected_words(ctx) : copy.data();
   for (int i = 0; i < ntasks; ++i) {
-    const unsigned long long* wk = &hwork[(size_t)8 * i];
+    unsigned long long wk[8];
+    memcpy(wk, h + work_at + 16 * (size_t)i, sizeof(wk));
     gdb_task& tk = tasks[P.order[i]];
-    tk.rounds = hres[i];
-    st->rounds += hres[i];
+    tk.rounds = h[i];
+    st->rounds += h[i];
     // Worklist tasks report items / edges processed; colour tasks count the
     // graph once.
     const bool wl = tk.algo != GDB_TASK_COLOR;
@@ -2170,9 +2180,8 @@ int collect_batch(const BatchPlan& P, gdb_task* tasks, gdb_stats* st) {
     for (int a = 0; a < 4; ++a) tk.arm_iters[a] = (int)wk[4 + a];
   }
   st->launches = 1;
-  int rc = read_participating(ctx, &st->participating);
-  if (rc) return rc;
-  return check_device_error(ctx);
+  st->participating = collected_participating(ctx);
+  return collected_error(ctx);
 }
 
 }  // namespace
@@ -2190,7 +2199,6 @@ extern "C" int gdb_batch_solve_sel(gdb_ctx* ctx, gdb_task* tasks, int ntasks, in
   if (!rc) rc = enqueue_prep(P);
   if (!rc) rc = timer_start(ctx);
   if (!rc) rc = enqueue_kernel(P);
-  if (!rc) rc = timer_stop(ctx, &st.kernel_ms);
   if (rc) return rc;
   rc = collect_batch(P, tasks, &st);
   if (stats) *stats = st;
@@ -2244,8 +2252,6 @@ extern "C" int gdb_batch_graph_launch(gdb_batch_graph* g, gdb_stats* stats) {
   int rc = timer_start(ctx);
   if (rc) return rc;
   GDB_HIP(hipGraphLaunch(g->exec, ctx->stream));
-  rc = timer_stop(ctx, &st.kernel_ms);
-  if (rc) return rc;
   rc = collect_batch(g->plan, g->tasks, &st);
   if (stats) *stats = st;
   return rc;

@@ -778,9 +778,7 @@ extern "C" int gdb_bc(gdb_ctx* ctx, int n, int m, const int* row, const int* col
   int4* mst = multi ? cv.take<int4>((size_t)2 * kNR * n) : nullptr;
   int* mq = multi ? cv.take<int>(qcap) : nullptr;
   int* mloff = multi ? cv.take<int>(qcap + 2) : nullptr;
-  rc = fill_i32(ctx, flags, 0, 32);
-  if (rc) return rc;
-  rc = prepare_launch(ctx);
+  rc = prepare_launch(ctx, flags, 32);
   if (rc) return rc;
   const int grid = (n + wgs - 1) / wgs;
 
@@ -839,18 +837,15 @@ extern "C" int gdb_bc(gdb_ctx* ctx, int n, int m, const int* row, const int* col
         hipLaunchKernelGGL(k_bc_plain<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col,
                            row_t, col_t, d, rho, delta, bc, sources, nsrc, flags, n, out);
       GDB_HIP(hipGetLastError());
-      return timer_stop(ctx, &st.kernel_ms);
+      return finish_launch(ctx, &st.kernel_ms, out, 2);
     });
     if (rc) return rc;
     st.launches = 1;
-    int hout[2] = {0, 0};
-    GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-    st.rounds = hout[0];
-    st.barriers = hout[1];
-    rc = read_participating(ctx, &st.participating);
-    if (rc) return rc;
+    st.rounds = collected_words(ctx)[0];
+    st.barriers = collected_words(ctx)[1];
+    st.participating = collected_participating(ctx);
   }
-  rc = check_device_error(ctx);
+  rc = o.schedule == GDB_SCHED_RELAUNCH ? check_device_error(ctx) : collected_error(ctx);
   st.work_edges = (long long)m * nsrc;
   st.work_items = (long long)n * nsrc;
   if (stats) *stats = st;

@@ -783,22 +783,17 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
   int* poll = cv.take<int>((size_t)n + 1);
   int* gmx = cv.take<int>(n);
   int* gcnt = cv.take<int>(n);
-  auto begin = [&]() -> int {
-    int r = fill_i32(ctx, fw, 0, FW_WORDS);
-    if (!r) r = prepare_launch(ctx);
-    return r;
-  };
   if (one) {
     const size_t lds = flow1_lds(n);
     if (lds > 49152)
       GDB_HIP(hipFuncSetAttribute((const void*)k_color_flow1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    rc = begin();
+    rc = prepare_launch(ctx, fw, FW_WORDS);
     if (!rc) rc = timer_start(ctx);
     if (rc) return rc;
     hipLaunchKernelGGL(k_color_flow1, dim3(1), dim3(1024), lds, ctx->stream, ctx->d, row, col, nv, n, m, color, fw,
                        limit);
     GDB_HIP(hipGetLastError());
-    rc = timer_stop(ctx, &s->kernel_ms);
+    rc = finish_launch(ctx, &s->kernel_ms, fw, FW_WORDS);
     if (rc) return rc;
     s->launches = 1;
   } else {
@@ -813,7 +808,7 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
       int r = launch_groups(ctx, kern, &o, (long long)GDB_MAX_GROUPS * WG, &groups, lds);
       if (r) return r;
       if (nwin > (open ? std::min(groups, ctx->num_cus) : groups)) return GDB_SUCCESS;
-      r = begin();
+      r = prepare_launch(ctx, fw, FW_WORDS);
       if (!r) r = timer_start(ctx);
       if (r) return r;
       hipLaunchKernelGGL(k_flow_init, dim3(n / 256 + 1), dim3(256), 0, ctx->stream, row, nv, n, m, C, poll, gmx, gcnt,
@@ -824,18 +819,16 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
       GDB_HIP(hipGetLastError());
       ran = true;
       s->launches = 3;
-      return timer_stop(ctx, &s->kernel_ms);
+      return finish_launch(ctx, &s->kernel_ms, fw, FW_WORDS);
     });
     if (rc || !ran) return rc;
   }
-  int h[FW_WORDS] = {};
-  GDB_HIP(hipMemcpy(h, fw, sizeof(h), hipMemcpyDeviceToHost));
-  rc = check_device_error(ctx);
+  const int* h = collected_words(ctx);
+  rc = collected_error(ctx);
   if (rc) return rc;
   if (h[FW_INVALID]) return GDB_E_INVALID;
   if (h[FW_GAVE_UP] || h[FW_ROUNDS] == INT_MAX) return GDB_SUCCESS;  // INT_MAX: neighbours that are never coloured
-  rc = read_participating(ctx, &s->participating);
-  if (rc) return rc;
+  s->participating = collected_participating(ctx);
   s->rounds = h[FW_ROUNDS] + 1;
   *done = true;
   return GDB_SUCCESS;
@@ -969,18 +962,15 @@ extern "C" int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* 
         hipLaunchKernelGGL(k_color_plain<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row,
                            col, node_value, color, flags, flags + 4, maxd, n, max_rounds, out);
       GDB_HIP(hipGetLastError());
-      return timer_stop(ctx, &s.kernel_ms);
+      return finish_launch(ctx, &s.kernel_ms, out, 2);
     });
     if (rc) return rc;
     s.launches = 1;
-    int hout[2] = {0, 0};
-    GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-    s.rounds = hout[0];
-    s.barriers = hout[1];
-    rc = read_participating(ctx, &s.participating);
-    if (rc) return rc;
+    s.rounds = collected_words(ctx)[0];
+    s.barriers = collected_words(ctx)[1];
+    s.participating = collected_participating(ctx);
   }
-  rc = check_device_error(ctx);
+  rc = o.schedule == GDB_SCHED_RELAUNCH ? check_device_error(ctx) : collected_error(ctx);
   if (rc == GDB_E_OVERFLOW) rc = GDB_E_TIMEOUT;  // round cap hit: equal priorities never resolve
   s.work_edges = m;
   s.work_items = n;
@@ -1007,8 +997,7 @@ extern "C" int gdb_color_maxmin(gdb_ctx* ctx, int n, int m, const int* row, cons
   int* code = cv.take<int>(n);
   int* flags = cv.take<int>(16);
   rc = fill_i32(ctx, color, -1, n);
-  if (!rc) rc = fill_i32(ctx, flags, 0, 16);
-  if (!rc) rc = prepare_launch(ctx);
+  if (!rc) rc = prepare_launch(ctx, flags, 16);
   if (rc) return rc;
   int* out = flags + 8;
   rc = gdb_dispatch_wgs(wgs, [&](auto W) -> int {
@@ -1021,17 +1010,14 @@ extern "C" int gdb_color_maxmin(gdb_ctx* ctx, int n, int m, const int* row, cons
     hipLaunchKernelGGL(k_color_maxmin<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col, node_value,
                        color, code, flags, n, n + 1, out);
     GDB_HIP(hipGetLastError());
-    return timer_stop(ctx, &s.kernel_ms);
+    return finish_launch(ctx, &s.kernel_ms, out, 2);
   });
   if (rc) return rc;
   s.launches = 1;
-  int hout[2] = {0, 0};
-  GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-  s.rounds = hout[0];
-  s.barriers = hout[1];
-  rc = read_participating(ctx, &s.participating);
-  if (rc) return rc;
-  rc = check_device_error(ctx);
+  s.rounds = collected_words(ctx)[0];
+  s.barriers = collected_words(ctx)[1];
+  s.participating = collected_participating(ctx);
+  rc = collected_error(ctx);
   if (rc == GDB_E_OVERFLOW) rc = GDB_E_TIMEOUT;  // round cap hit: adjacent equal values never resolve
   s.work_edges = m;
   s.work_items = n;

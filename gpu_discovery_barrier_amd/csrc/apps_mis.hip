@@ -344,18 +344,15 @@ extern "C" int gdb_mis(gdb_ctx* ctx, int n, int m, const int* row, const int* co
         hipLaunchKernelGGL(k_mis_plain<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col,
                            node_value, s, c, cu, min_array, flags, n, max_rounds, out);
       GDB_HIP(hipGetLastError());
-      return timer_stop(ctx, &st.kernel_ms);
+      return finish_launch(ctx, &st.kernel_ms, out, 2);
     });
     if (rc) return rc;
     st.launches = 1;
-    int hout[2] = {0, 0};
-    GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-    st.rounds = hout[0];
-    st.barriers = hout[1];
-    rc = read_participating(ctx, &st.participating);
-    if (rc) return rc;
+    st.rounds = collected_words(ctx)[0];
+    st.barriers = collected_words(ctx)[1];
+    st.participating = collected_participating(ctx);
   }
-  rc = check_device_error(ctx);
+  rc = o.schedule == GDB_SCHED_RELAUNCH ? check_device_error(ctx) : collected_error(ctx);
   if (rc == GDB_E_OVERFLOW) rc = GDB_E_TIMEOUT;  // round cap: equal priorities never resolve
   st.work_edges = m;
   st.work_items = n;

@@ -33,6 +33,7 @@
 // round, six barriers: 46.4 ms; vertices 64 at a time: 0.93).  Walking the rows of a wave as one list, with
 // the minima in LDS, took 1.07 ms: the search for each edge's row costs more
 // than the steps it saves.
+#include <cstring>
 #include "graph_common.hpp"
 #include "runtime.hpp"
 
@@ -270,12 +271,10 @@ extern "C" int gdb_mst(gdb_ctx* ctx, int n, int m, const int* row, const int* co
   int2* pieces = cv.take<int2>(piece_cap);
   int* flags = cv.take<int>(32);
   u64* total = cv.take<u64>(1);
-  rc = fill_i32(ctx, flags, 0, 32);
-  if (!rc) rc = fill_i32(ctx, (int*)total, 0, 2);
-  if (rc) return rc;
   int* out = flags + 8;
   int* npieces = flags + 16;
-  rc = prepare_launch(ctx);
+  const int nwords = (int)((int*)(total + 1) - flags);  // flags and total are neighbours in the workspace
+  rc = prepare_launch(ctx, flags, nwords);
   if (rc) return rc;
   rc = gdb_dispatch_wgs(wgs, [&](auto W) -> int {
     constexpr int WG = decltype(W)::value;
@@ -287,21 +286,19 @@ extern "C" int gdb_mst(gdb_ctx* ctx, int n, int m, const int* row, const int* co
     hipLaunchKernelGGL(k_mst<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col, w, n, comp, parent,
                        best, dead, pieces, piece_cap, npieces, flags, total, out);
     GDB_HIP(hipGetLastError());
-    return timer_stop(ctx, &st.kernel_ms);
+    return finish_launch(ctx, &st.kernel_ms, flags, nwords);
   });
   if (rc) return rc;
-  int hout[4] = {0, 0, 0, 0};
+  const int* hout = collected_words(ctx) + 8;
   unsigned long long hw = 0;
-  GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-  GDB_HIP(hipMemcpy(&hw, total, sizeof(hw), hipMemcpyDeviceToHost));
+  memcpy(&hw, collected_words(ctx) + nwords - 2, sizeof(hw));
   st.rounds = hout[0];
   st.barriers = hout[1];
   st.launches = 1;
   st.work_edges = (long long)m * hout[0];
   st.work_items = (long long)n * hout[0];
-  rc = read_participating(ctx, &st.participating);
-  if (rc) return rc;
-  rc = check_device_error(ctx);
+  st.participating = collected_participating(ctx);
+  rc = collected_error(ctx);
   if (weight) *weight = hw;
   if (edges) *edges = hout[2];
   if (components) *components = hout[3];

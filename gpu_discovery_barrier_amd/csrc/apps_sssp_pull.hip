@@ -290,18 +290,15 @@ extern "C" int gdb_sssp_pull(gdb_ctx* ctx, int n, int m, const int* row_t, const
         hipLaunchKernelGGL(k_sssp_pull_plain<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, n,
                            row_t, col_t, w_t, x, y, flags, out);
       GDB_HIP(hipGetLastError());
-      return timer_stop(ctx, &st.kernel_ms);
+      return finish_launch(ctx, &st.kernel_ms, out, 2);
     });
     if (rc) return rc;
     st.launches = 1;
-    int hout[2] = {0, 0};
-    GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-    st.rounds = hout[0];
-    st.barriers = hout[1];
-    rc = read_participating(ctx, &st.participating);
-    if (rc) return rc;
+    st.rounds = collected_words(ctx)[0];
+    st.barriers = collected_words(ctx)[1];
+    st.participating = collected_participating(ctx);
   }
-  rc = check_device_error(ctx);
+  rc = o.schedule == GDB_SCHED_RELAUNCH ? check_device_error(ctx) : collected_error(ctx);
   st.work_edges = (long long)m * (st.rounds > 0 ? st.rounds : 1);
   st.work_items = (long long)n * (st.rounds > 0 ? st.rounds : 1);
   if (stats) *stats = st;

@@ -29,6 +29,7 @@
 //   relaunch         - one launch per iteration with a host loop reading the
 //                      output size (the non-persistent schedule).
 #include <algorithm>
+#include <cstring>
 #include <mutex>
 #include "graph_common.hpp"
 #include "runtime.hpp"
@@ -522,14 +523,17 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
   int rc = ensure_workspace(ctx, sizeof(Locality));
   if (rc) return rc;
   Locality* d = (Locality*)ctx->ws;
-  rc = fill_i32(ctx, (int*)d, 0, sizeof(Locality) / sizeof(int));
+  constexpr int kWords = sizeof(Locality) / sizeof(int);
+  rc = prepare_launch(ctx, (int*)d, kWords);
+  if (!rc) rc = timer_start(ctx);
   if (rc) return rc;
   hipLaunchKernelGGL(k_locality, dim3(kSampleVertices / 256), dim3(256), 0, ctx->stream, row, col,
                      WEIGHTED ? w : nullptr, n, d);
   GDB_HIP(hipGetLastError());
   Locality h;
-  GDB_HIP(hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-  GDB_HIP(hipStreamSynchronize(ctx->stream));
+  rc = finish_launch(ctx, nullptr, d, kWords);
+  if (rc) return rc;
+  memcpy(&h, collected_words(ctx), sizeof(h));
   if (h.edges == 0) return GDB_SUCCESS;
   const int G = std::max(1, std::min(ctx->num_cus, (n + kLocalRange - 1) / kLocalRange));
   const int range = (n + G - 1) / G;
@@ -555,12 +559,14 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
   if (rc) return rc;
   if (!WEIGHTED) {
     int* levels = (int*)ctx->ws;
-    rc = fill_i32(ctx, levels, 0, 1);
+    rc = prepare_launch(ctx, levels, 1);
+    if (!rc) rc = timer_start(ctx);
     if (rc) return rc;
     hipLaunchKernelGGL(k_levels, dim3(std::min(256, (n + 255) / 256)), dim3(256), 0, ctx->stream, dist, n, levels);
     GDB_HIP(hipGetLastError());
-    GDB_HIP(hipMemcpyAsync(&st->rounds, levels, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    GDB_HIP(hipStreamSynchronize(ctx->stream));
+    rc = finish_launch(ctx, nullptr, levels, 1);
+    if (rc) return rc;
+    st->rounds = collected_words(ctx)[0];
   }
   *done = true;
   return GDB_SUCCESS;
@@ -622,13 +628,11 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   int4* pieces = cv.take<int4>(piece_cap);
   int* tails = flags + 4;
   int* out = flags + 12;
-  rc = fill_i32(ctx, (int*)work, 0, 4);
+  rc = prepare_launch(ctx, (int*)work, 4);
   if (rc) return rc;
   hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, dist, stamp, q0, q1,
                      flags, n, source);
   GDB_HIP(hipGetLastError());
-  rc = prepare_launch(ctx);
-  if (rc) return rc;
 
   if (o.schedule == GDB_SCHED_RELAUNCH) {
     const int check = o.relaunch_check > 1 ? o.relaunch_check : 1;
@@ -659,6 +663,7 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
     st.participating = grid;
   } else {
     const bool tuned = o.variant == GDB_VARIANT_TUNED;
+    const int nwords = (int)((int*)(work + 2) - flags);  // flags and work are neighbours in the workspace
     rc = gdb_dispatch_wgs(wgs, [&](auto W) -> int {
       constexpr int WG = decltype(W)::value;
       const void* kern = tuned ? (const void*)k_wl_tuned<WG, WEIGHTED> : (const void*)k_wl_plain<WG, WEIGHTED>;
@@ -675,24 +680,22 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
         hipLaunchKernelGGL((k_wl_plain<WG, WEIGHTED>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
                            row, col, w, dist, stamp, q0, q1, flags, n, out);
       GDB_HIP(hipGetLastError());
-      return timer_stop(ctx, &st.kernel_ms);
+      return finish_launch(ctx, &st.kernel_ms, flags, nwords);
     });
     if (rc) return rc;
     st.launches = 1;
-    int hout[2] = {0, 0};
-    GDB_HIP(hipMemcpy(hout, out, sizeof(hout), hipMemcpyDeviceToHost));
-    st.rounds = hout[0];
-    st.barriers = hout[1];
+    const int* h = collected_words(ctx);
+    st.rounds = h[out - flags];
+    st.barriers = h[out + 1 - flags];
     if (tuned) {
-      long long hw[2] = {0, 0};
-      GDB_HIP(hipMemcpy(hw, work, sizeof(hw), hipMemcpyDeviceToHost));
+      long long hw[2];
+      memcpy(hw, h + nwords - 4, sizeof(hw));
       st.work_items = hw[0];
       st.work_edges = hw[1];
     }
-    rc = read_participating(ctx, &st.participating);
-    if (rc) return rc;
+    st.participating = collected_participating(ctx);
   }
-  rc = check_device_error(ctx);
+  rc = o.schedule == GDB_SCHED_RELAUNCH ? check_device_error(ctx) : collected_error(ctx);
   if (stats) *stats = st;
   return rc;
 }

@@ -45,8 +45,19 @@ __global__ void gdb_k_fill_i32(int* p, int value, long long count) {
   if (i < count) p[i] = value;
 }
 
-// Clears the sticky error word before a solve.
-__global__ void gdb_k_clear_error(gdb_kernel_ctx_t* ctx) { gdb::st_rlx(&ctx->error.v, GDB_OK); }
+// Before a solve: clears the sticky error word and `count` ints.
+__global__ void gdb_k_begin(gdb_kernel_ctx_t* ctx, int* words, int count) {
+  if (threadIdx.x == 0) gdb::st_rlx(&ctx->error.v, GDB_OK);
+  if ((int)threadIdx.x < count) words[threadIdx.x] = 0;
+}
+
+// After a solve: the words the host reads, into pinned host memory.
+__global__ void gdb_k_collect(gdb_kernel_ctx_t* ctx, const int* words, int count, int* host) {
+  const int i = (int)threadIdx.x;
+  if (i == 0) host[0] = gdb::ld_rlx(&ctx->error.v);
+  if (i == 1) host[1] = gdb::ld_rlx(&ctx->num_participating.v);
+  if (i < count) host[2 + i] = words[i];
+}
 
 // Rewrites the wait bounds of a context without resetting its other words.
 __global__ void gdb_k_set_timeouts(gdb_kernel_ctx_t* ctx, int quiet_ticks, int timeout_ticks) {
@@ -124,8 +135,20 @@ int ensure_workspace(gdb_ctx* ctx, size_t bytes) {
   return GDB_SUCCESS;
 }
 
-int prepare_launch(gdb_ctx* ctx) {
-  hipLaunchKernelGGL(gdb_k_clear_error, dim3(1), dim3(1), 0, ctx->stream, ctx->d);
+int ensure_stage(gdb_ctx* ctx, size_t bytes) {
+  if (bytes <= ctx->stage_bytes) return GDB_SUCCESS;
+  if (ctx->h_stage) GDB_HIP(hipHostFree(ctx->h_stage));
+  ctx->h_stage = nullptr;
+  ctx->stage_bytes = 0;
+  const size_t want = bytes + bytes / 4 + 4096;
+  GDB_HIP(hipHostMalloc(&ctx->h_stage, want, hipHostMallocDefault));
+  ctx->stage_bytes = want;
+  return GDB_SUCCESS;
+}
+
+int prepare_launch(gdb_ctx* ctx, int* words, int count) {
+  if (count > 256) return GDB_E_INVALID;
+  hipLaunchKernelGGL(gdb_k_begin, dim3(1), dim3(256), 0, ctx->stream, ctx->d, words, count);
   GDB_HIP(hipGetLastError());
   return GDB_SUCCESS;
 }
@@ -140,10 +163,7 @@ int fill_i32(gdb_ctx* ctx, int* p, int value, long long count) {
 
 static int init_ctx(gdb_ctx* ctx, int skip);
 
-int check_device_error(gdb_ctx* ctx) {
-  int err = 0;
-  GDB_HIP(hipMemcpyAsync(&err, &ctx->d->error.v, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  GDB_HIP(hipStreamSynchronize(ctx->stream));
+static int report_error(gdb_ctx* ctx, int err) {
   if (err == GDB_ERR_BARRIER_TIMEOUT || err == GDB_ERR_DISCOVERY_TIMEOUT) {
     // A wait that gave up leaves arrival counters, XF flags or protocol
     // words part-way through an episode; the next launch would start from
@@ -152,6 +172,28 @@ int check_device_error(gdb_ctx* ctx) {
     return rc ? rc : GDB_E_TIMEOUT;
   }
   if (err == GDB_ERR_QUEUE_OVERFLOW) return GDB_E_OVERFLOW;
+  return GDB_SUCCESS;
+}
+
+int check_device_error(gdb_ctx* ctx) {
+  int err = 0;
+  GDB_HIP(hipMemcpyAsync(&err, &ctx->d->error.v, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  GDB_HIP(hipStreamSynchronize(ctx->stream));
+  return report_error(ctx, err);
+}
+
+int collected_error(gdb_ctx* ctx) { return report_error(ctx, ctx->h_flag[kCollectBase]); }
+
+int finish_launch(gdb_ctx* ctx, double* ms, const void* words, int count) {
+  if (count < 0 || count > kCollectMax) return GDB_E_INVALID;
+  GDB_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+  hipLaunchKernelGGL(gdb_k_collect, dim3(1), dim3(256), 0, ctx->stream, ctx->d, (const int*)words, count,
+                     ctx->h_flag + kCollectBase);
+  GDB_HIP(hipGetLastError());
+  GDB_HIP(hipStreamSynchronize(ctx->stream));
+  float f = 0.f;
+  GDB_HIP(hipEventElapsedTime(&f, ctx->ev0, ctx->ev1));
+  if (ms) *ms = f;
   return GDB_SUCCESS;
 }
 
@@ -382,7 +424,7 @@ int gdb_ctx_create(gdb_ctx** out) {
     GDB_HIP(hipMalloc(&p, sizeof(gdb_kernel_ctx_t)));
   }
   ctx->d = (gdb_kernel_ctx_t*)p;
-  GDB_HIP(hipHostMalloc((void**)&ctx->h_flag, sizeof(int) * 4, hipHostMallocDefault));
+  GDB_HIP(hipHostMalloc((void**)&ctx->h_flag, sizeof(int) * (kCollectBase + 2 + kCollectMax), hipHostMallocDefault));
   GDB_HIP(hipEventCreate(&ctx->ev0));
   GDB_HIP(hipEventCreate(&ctx->ev1));
   int rc = resolve_noalloc_scratch(ctx);
@@ -399,6 +441,7 @@ int gdb_ctx_destroy(gdb_ctx* ctx) {
   if (ctx->ws) GDB_HIP(hipFree(ctx->ws));
   if (ctx->d) GDB_HIP(hipFree(ctx->d));
   if (ctx->h_flag) GDB_HIP(hipHostFree(ctx->h_flag));
+  if (ctx->h_stage) GDB_HIP(hipHostFree(ctx->h_stage));
   if (ctx->ev0) GDB_HIP(hipEventDestroy(ctx->ev0));
   if (ctx->ev1) GDB_HIP(hipEventDestroy(ctx->ev1));
   if (ctx->stream) GDB_HIP(hipStreamDestroy(ctx->stream));

@@ -27,8 +27,12 @@ struct gdb_ctx {
   // Device address, on this context's device, of the library's static
   // scratch array (gdb_sssp_worklist_noalloc); resolved at context creation.
   void* noalloc_scratch = nullptr;
-  // Pinned host word for stop-flag readbacks of the relaunch schedule.
+  // Pinned host words: [0, 8) stop-flag readbacks of the relaunch schedule, then
+  // what finish_launch collects (GDB_COLLECT_WORDS).
   int* h_flag = nullptr;
+  // Grow-only pinned host buffer that uploads go through (a batch's task table).
+  void* h_stage = nullptr;
+  size_t stage_bytes = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
@@ -45,6 +49,10 @@ int hip_fail(hipError_t e, const char* what, const char* file, int line);
 
 // Ensures ctx->ws holds at least `bytes`; returns GDB_SUCCESS or an error.
 int ensure_workspace(gdb_ctx* ctx, size_t bytes);
+
+// Ensures ctx->h_stage holds at least `bytes`.  Free for reuse whenever no call on
+// the context is running: every call waits for its work.
+int ensure_stage(gdb_ctx* ctx, size_t bytes);
 
 // Bump allocator over the workspace: 256-byte aligned slices.
 struct Carve {
@@ -64,8 +72,20 @@ inline size_t carve_bytes(size_t count) { return (count * sizeof(T) + 255) & ~(s
 // Fills count ints with value on the context stream (a kernel, not a memset).
 int fill_i32(gdb_ctx* ctx, int* p, int value, long long count);
 
-// Writes the per-launch protocol configuration and clears the sticky error.
-int prepare_launch(gdb_ctx* ctx);
+// Clears the sticky error and sets `count` (at most 256) ints at `words` to 0.
+int prepare_launch(gdb_ctx* ctx, int* words = nullptr, int count = 0);
+
+// Ends a solve: stops the timer and waits, after one small kernel has written the
+// context's error and participating words and `count` ints from `words` into
+// pinned host memory.  A blocking copy costs about 15 us of host and device
+// time each; a solve used to make four of them.
+constexpr int kCollectBase = 8, kCollectMax = 246;
+int finish_launch(gdb_ctx* ctx, double* ms, const void* words, int count);
+// What the last finish_launch collected: its ints, the participating count,
+// and the sticky error as check_device_error reports it.
+inline const int* collected_words(gdb_ctx* ctx) { return ctx->h_flag + kCollectBase + 2; }
+inline int collected_participating(gdb_ctx* ctx) { return ctx->h_flag[kCollectBase + 1]; }
+int collected_error(gdb_ctx* ctx);
 
 // Reads the device sticky error after a launch (blocking).  Returns
 // GDB_SUCCESS, GDB_E_TIMEOUT or GDB_E_OVERFLOW.
