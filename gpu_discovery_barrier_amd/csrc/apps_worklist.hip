@@ -175,8 +175,8 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
                                                   int4* pieces, int piece_cap, long long* work, int* out) {
   DISCOVERY_PROTOCOL(ctx);
   constexpr int kStage = 8 * WGS;  // pushes of this group awaiting queue space
-  __shared__ int s_q[kStage];
-  __shared__ int s_n, s_base;
+  __shared__ int s_q[kStage], s_n, s_base;
+  const gdb::PushStage stage{s_q, &s_n, &s_base, kStage};
   const int tid = p_get_global_id(ctx, &local_ctx);
   const int threads = p_get_global_size(ctx, &local_ctx);
   const int lane = gdb::lane_id(), wave = tid >> 6, nwaves = threads >> 6;
@@ -201,21 +201,6 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
       gdb::st_rlx(&piece_counts[(iteration + 1) % 3], 0);
     }
     items += nin;
-    // Moves the staged pushes to the queue when more than `above` wait.  All
-    // threads of the group call it.
-    auto flush = [&](int above) {
-      __syncthreads();
-      const int c = min(s_n, kStage);
-      __syncthreads();
-      if (c <= above) return;
-      if (threadIdx.x == 0) {
-        s_base = gdb::fadd_rlx(out_tail, c);
-        s_n = 0;
-      }
-      __syncthreads();
-      for (int i = threadIdx.x; i < c; i += WGS) outq[s_base + i] = s_q[i];
-      __syncthreads();
-    };
     // kChunk edges per lane step (long rows: the whole wave, carrying the
     // row owner's distance): the column and weight loads, then the
     // targets' distances, then atomics only where a candidate improves
@@ -283,30 +268,7 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
         }
       }
-      // Pushes, staged in LDS.
-      unsigned long long m[kChunk];
-      int cnt = 0;
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) {
-        m[j] = __ballot(push[j]);
-        cnt += __popcll(m[j]);
-      }
-      if (cnt == 0) return 0;
-      int base = 0;
-      if (lane == 0) base = atomicAdd(&s_n, cnt);
-      base = gdb::bcast(base, 0);
-      const bool full = base + cnt > kStage;  // what does not fit goes straight to the queue
-      const unsigned long long lt = (1ull << lane) - 1ull;
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) {
-        const int pos = base + __popcll(m[j] & lt);
-        if (push[j] && pos < kStage) {
-          s_q[pos] = dst[j];
-          push[j] = false;
-        }
-        base += __popcll(m[j]);
-      }
-      if (full) gdb::wave_push_n<kChunk>(push, dst, outq, out_tail);
+      gdb::wave_stage_n<kChunk>(stage, push, dst, outq, out_tail);
       return 0;
     };
     auto any = [](int a, int c) { return a | c; };
@@ -331,9 +293,9 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
         }
       }
       gdb::wave_walk_np<kChunk>(valid != 0, b, e, (int)dv, 0, step, any, kSerialLimit);
-      flush(kStage / 2);
+      gdb::group_flush(stage, kStage / 2, outq, out_tail);
     }
-    flush(0);
+    gdb::group_flush(stage, 0, outq, out_tail);
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
     const int np = min(gdb::ld_rlx(npieces), piece_cap);
@@ -351,9 +313,9 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
           step(ok, kk, pc.z);
         }
-        flush(kStage / 2);
+        gdb::group_flush(stage, kStage / 2, outq, out_tail);
       }
-      flush(0);
+      gdb::group_flush(stage, 0, outq, out_tail);
       if (!discovery_barrier(ctx, &local_ctx)) return;
       ++nbar;
     }

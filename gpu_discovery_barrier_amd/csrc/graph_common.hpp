@@ -208,6 +208,59 @@ __device__ __forceinline__ void wave_push_n(const bool (&push)[N], const int (&i
   }
 }
 
+// Queue pushes staged in LDS.  One returning atomic on a queue's size per wave
+// step serialises at about 8 ns each; a group that stages its pushes reserves
+// space for a batch of them at once.  wave_stage_n appends the items of N push
+// slots of every lane to the stage (what does not fit goes straight to the
+// queue); group_flush, called by all threads of the group, moves the staged items
+// to the queue when more than `above` wait.
+struct PushStage {
+  int* items;  // LDS, `cap` entries
+  int* count;  // LDS, zeroed before the first use
+  int* base;   // LDS
+  int cap;
+};
+template <int N>
+__device__ __forceinline__ void wave_stage_n(const PushStage& st, bool (&push)[N], const int (&item)[N], int* queue,
+                                             int* tail) {
+  unsigned long long m[N];
+  int cnt = 0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    m[j] = __ballot(push[j]);
+    cnt += __popcll(m[j]);
+  }
+  if (cnt == 0) return;
+  const int lane = lane_id();
+  int base = 0;
+  if (lane == 0) base = atomicAdd(st.count, cnt);
+  base = bcast(base, 0);
+  const bool full = base + cnt > st.cap;
+  const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int pos = base + __popcll(m[j] & lt);
+    if (push[j] && pos < st.cap) {
+      st.items[pos] = item[j];
+      push[j] = false;
+    }
+    base += __popcll(m[j]);
+  }
+  if (full) wave_push_n<N>(push, item, queue, tail);
+}
+__device__ __forceinline__ void group_flush(const PushStage& st, int above, int* queue, int* tail) {
+  __syncthreads();
+  const int c = *st.count < st.cap ? *st.count : st.cap;
+  __syncthreads();
+  if (c <= above) return;
+  if (threadIdx.x == 0) {
+    *st.base = fadd_rlx(tail, c);
+    *st.count = 0;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < c; i += blockDim.x) queue[*st.base + i] = st.items[i];
+  __syncthreads();
+}
 
 // Wave-wide OR of a predicate.
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0ull; }

@@ -423,3 +423,27 @@ def test_sssp_pull_row_lengths(ctx, wgs, groups, leaves):
     got, st = gdb.sssp_pull(ctx, dev(gt.row, gt.col, gt.w), 0, gdb.Opts.make(wgs=wgs, groups=groups,
                                                                             variant=gdb.VARIANT_TUNED))
     assert (got == want).all() and st.rounds == rounds
+
+
+@pytest.mark.parametrize("leaves", [4095, 4096, 4097, 6145, 30000])
+def test_bc_rows_walked_by_a_group(ctx, leaves):
+    # Two hubs sharing `leaves` neighbours, with a second ring behind them:
+    # rows at the edges of the per-wave and per-group walks; the sums do not
+    # depend on the launch shape.
+    n = 2 + leaves + leaves // 3
+    edges = [(h, 2 + i) for h in range(2) for i in range(leaves)]
+    edges += [(2 + 3 * i, 2 + leaves + i) for i in range(leaves // 3)]
+    a = np.array(edges, np.int64)
+    src, dst = np.concatenate([a[:, 0], a[:, 1]]), np.concatenate([a[:, 1], a[:, 0]])
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int32)
+    col = dst[order].astype(np.int32)
+    d = dev(row, col)
+    sources = np.array([0, 2, n - 1, 1, 5, 7, 11, 2 + leaves, 3, n // 2], np.int32)
+    want = oracle.bc_brandes_mt(row, col, sources)
+    first = None
+    for wgs, groups in ((512, 0), (64, 5), (256, 16), (0, 0)):
+        got, _ = gdb.bc(ctx, d, d, sources, gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED))
+        bc_close(got, want)
+        first = got if first is None else first
+        assert (got == first).all(), (wgs, groups)
