@@ -447,3 +447,42 @@ def test_bc_rows_walked_by_a_group(ctx, leaves):
         bc_close(got, want)
         first = got if first is None else first
         assert (got == first).all(), (wgs, groups)
+
+
+@pytest.mark.parametrize("wgs,groups", [(0, 0), (64, 3), (512, 16)])
+@pytest.mark.parametrize("nsrc", [1, 2, 8, 11])
+@pytest.mark.parametrize("shape", ["random", "layers", "levels253", "levels256", "hub"])
+def test_bc_directed_sweeps(ctx, shape, nsrc, wgs, groups):
+    # Sources of a directed graph share sweeps with a byte of level each:
+    # skipping levels, back edges, the deepest search a byte holds and one
+    # beyond it (solved source by source), and a row walked by waves.
+    rng = np.random.default_rng(nsrc)
+    if shape == "random":
+        n = 3000
+        src, dst = rng.integers(0, n, 15000), rng.integers(0, n, 15000)
+    elif shape == "layers":  # forward edges of any length, a few back
+        n = 900
+        src = rng.integers(0, n, 4000)
+        dst = np.minimum(n - 1, src + rng.integers(1, 60, 4000))
+        dst[::50] = rng.integers(0, n, dst[::50].size)
+    elif shape == "hub":
+        n = 5000
+        src = np.concatenate([np.arange(1, 2500), np.zeros(2500, np.int64), rng.integers(0, n, 4000)])
+        dst = np.concatenate([np.zeros(2499, np.int64), np.arange(2500, 5000), rng.integers(0, n, 4000)])
+    else:  # two parallel chains of so many levels
+        k = int(shape[6:])
+        n = 2 * k + 1
+        a = np.arange(k)
+        src = np.concatenate([a, [0], k + a[1:]])
+        dst = np.concatenate([a + 1, [k + 1], k + a[1:] + 1])
+    keep = src != dst
+    src, dst = src[keep], dst[keep]
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int32)
+    col = dst[order].astype(np.int32)
+    g = gdb.CSR(n, row, col, np.ones_like(col))
+    gt = g.transpose()
+    sources = np.concatenate([[0], rng.integers(0, n, nsrc - 1)]).astype(np.int32)
+    got, _ = gdb.bc(ctx, gdb.DeviceCSR(g), gdb.DeviceCSR(gt), sources,
+                    gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED))
+    bc_close(got, np.asarray(oracle.bc_brandes_tb(row, col, sources), np.float64))
