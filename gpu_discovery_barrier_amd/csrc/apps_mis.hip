@@ -14,7 +14,7 @@
 //   tuned persistent - two barriers per round over a queue of the undecided
 //                      vertices: phase A computes the minimum over neighbours
 //                      from a packed (status, value) gather and decides joins
-//                      (s = 2); phase B retires joiners and vertices with a
+//                      (s = 2 and a bit in a bitmap); phase B retires joiners and vertices with a
 //                      joining neighbour (c = -2) and compacts the survivors
 //                      into the next queue.  Same joins as the reference: a
 //                      join only reads statuses fixed in the previous round.
@@ -26,6 +26,9 @@
 namespace {
 
 constexpr float kBigNum = 99999999.0f;  // mis_kernel.cl:68
+// Edges of a row that its own lane walks before the whole wave takes over.  R-MAT
+// 22 / R-MAT 17 / G(300k) in ms: 8: 2.40 / .226 / .266, 16: 2.28 / .221 / .236, 32:
+// 2.29 / .237 / .235.
 constexpr int kSerialLimit = 16;
 
 template <int WGS>
@@ -85,15 +88,18 @@ __global__ __launch_bounds__(WGS) void k_mis_plain(gdb_kernel_ctx_t* ctx, const 
 
 constexpr int kSlots = 4;  // edges a lane gathers per step in the tuned walks
 
-// What bounds it: random gathers, three dependent ones per walk step, and the
-// waves with the most long rows.  R-MAT 22: 3.1 ms with the vertices dealt to the
-// waves one by one (4.3 with 64 neighbours each).
+// What bounds it: random gathers, two dependent ones per walk step, and the
+// waves with the most long rows.  R-MAT 22 (4.2M vertices, 67M edges): 4.3 ms with
+// 64 neighbours per wave, 3.1 with the vertices dealt to the waves one by one, 2.28
+// with the first kSerialLimit edges of a long row walked by its own lane, where
+// most walks end, and 2.13 with the joiners read from a bitmap (0.5 MB: it stays in
+// every L2) instead of s.
 // Packed per-vertex state for one 8-byte gather per edge: x = status
 // (-1 undecided, -2 decided), y = node_value bits.
 template <int WGS>
 __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                                    const int* __restrict__ col, int2* cv, int* s,
-                                                   int* q0, int* q1, int* tails, int n,
+                                                   int* joined_bits, int* q0, int* q1, int* tails, int n,
                                                    int max_rounds, int* out) {
   DISCOVERY_PROTOCOL(ctx);
   const int tid = p_get_global_id(ctx, &local_ctx);
@@ -156,7 +162,10 @@ __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const 
       };
       const bool blocked =
           gdb::wave_walk_any<kSlots>(valid != 0, b, e, __float_as_int(vv), step, kSerialLimit);
-      if (valid && vv < kBigNum && !blocked) s[v] = 2;
+      if (valid && vv < kBigNum && !blocked) {
+        s[v] = 2;
+        gdb::atomic_or_g(&joined_bits[v >> 5], (int)(1u << (v & 31)));
+      }
     }
     if (tid == 0) gdb::st_rlx(&tails[(rounds + 1) % 3], 0);
     if (!discovery_barrier(ctx, &local_ctx)) return;
@@ -186,12 +195,13 @@ __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const 
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) {
           const bool in = ok[j] && (unsigned)u[j] < (unsigned)n;
-          sj[j] = gdb::ldg(s + (in ? u[j] : spare));
+          if (!in) u[j] = spare;
+          sj[j] = gdb::ldg(joined_bits + (u[j] >> 5));
           if (!in) sj[j] = 0;
         }
         bool h = false;
 #pragma unroll
-        for (int j = 0; j < kSlots; ++j) h |= sj[j] == 2;
+        for (int j = 0; j < kSlots; ++j) h |= ((sj[j] >> (u[j] & 31)) & 1) != 0;
         return h;
       };
       const bool hit = gdb::wave_walk_any<kSlots>(valid && !joined, b, e, 0, step, kSerialLimit);
@@ -218,14 +228,15 @@ __global__ __launch_bounds__(WGS) void k_mis_tuned(gdb_kernel_ctx_t* ctx, const 
   }
 }
 
-__global__ void k_mis_init(const float* __restrict__ nv, int* s, int* c, int* cu, int2* cv, int* flags,
-                           int n) {
+__global__ void k_mis_init(const float* __restrict__ nv, int* s, int* c, int* cu, int2* cv,
+                           int* joined_bits, int* flags, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {  // init kernel, mis_kernel.cl:78-93
     c[i] = -1;
     cu[i] = -1;
     s[i] = 0;
     cv[i] = make_int2(-1, __float_as_int(nv[i]));
+    if ((i & 31) == 0) joined_bits[i >> 5] = 0;
   }
   if (i < 16) flags[i] = 0;
 }
@@ -293,9 +304,12 @@ extern "C" int gdb_mis(gdb_ctx* ctx, int n, int m, const int* row, const int* co
   int2* cv = cvw.take<int2>(n);
   float* min_array = cvw.take<float>(n);
   int* flags = cvw.take<int>(32);
+  // Only the mega and relaunch kernels keep minima, only the tuned one a bitmap:
+  // its n / 32 + 1 words lie in the same n words.
+  int* joined_bits = (int*)min_array;
   const int max_rounds = n + 1;
   hipLaunchKernelGGL(k_mis_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, node_value, s, c,
-                     cu, cv, flags, n);
+                     cu, cv, joined_bits, flags, n);
   GDB_HIP(hipGetLastError());
   rc = prepare_launch(ctx);
   if (rc) return rc;
@@ -339,7 +353,7 @@ extern "C" int gdb_mis(gdb_ctx* ctx, int n, int m, const int* row, const int* co
       if (r2) return r2;
       if (tuned)
         hipLaunchKernelGGL(k_mis_tuned<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col,
-                           cv, s, q0, q1, flags + 4, n, max_rounds, out);
+                           cv, s, joined_bits, q0, q1, flags + 4, n, max_rounds, out);
       else
         hipLaunchKernelGGL(k_mis_plain<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col,
                            node_value, s, c, cu, min_array, flags, n, max_rounds, out);

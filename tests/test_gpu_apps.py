@@ -71,6 +71,29 @@ def test_mis_rmat(ctx, sched, vals):
     assert st.rounds == rounds
 
 
+@pytest.mark.parametrize("extra", [0, 1, 31])
+@pytest.mark.parametrize("deg", [1, 15, 16, 17, 79, 80, 81, 300])
+def test_mis_one_deciding_edge(ctx, deg, extra):
+    """Hubs of one degree, each with its only smaller neighbour at another place
+    of its row; the leaves of neighbouring hubs are joined, for further rounds."""
+    spots = sorted({0, 3, 4, deg // 2, 14, 15, 16, 17, deg - 1} & set(range(deg)))
+    hubs = len(spots)
+    n = hubs * (deg + 1) + extra
+    nv = np.empty(n, np.float32)
+    nv[:hubs] = 2.0 + np.arange(hubs)
+    nv[hubs:] = 100.0 + gdb.permutation(n - hubs, deg + 1).astype(np.float32)
+    edges = []
+    for h, p in enumerate(spots):
+        leaves = hubs + h * deg + np.arange(deg)
+        nv[leaves[p]] = 1.0 + h / 100
+        edges += [(h, int(u)) for u in leaves]
+        edges += [(int(u), hubs + (int(u) - hubs + deg) % (hubs * deg)) for u in leaves if hubs > 1]
+    row, col, _ = csr_from_edges(n, edges)
+    want, rounds = oracle.mis_ref(row, col, nv)
+    got, st = gdb.mis(ctx, dev(row, col), gdb.DeviceBuffer.from_numpy(nv), gdb.Opts.make())
+    assert (got == want).all() and st.rounds == rounds
+
+
 # ---------------------------------------------------------------- pull SSSP
 @pytest.mark.parametrize("sched", SCHEDS, ids=SID)
 @pytest.mark.parametrize("fx", FX["sssp_pull"], ids=lambda f: f["name"])
