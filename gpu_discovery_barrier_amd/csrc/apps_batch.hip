@@ -1465,6 +1465,9 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
   constexpr int kScanEvery = kOwnedScanEvery;
   unsigned thresh = band;
   long long items = 0, edges = 0;
+  int ahead[2] = {0, 0};  // words of records loaded early, for the load alone
+  // What lanes without a target touch: 32 vertices (B is a multiple of 32) and words.
+  const int idle_v = lane & 31, idle_w = W >= 32 ? lane & 31 : 0;
   // Relaxes local vertices li[j] to cand[j] on lanes with act[j], N targets
   // per lane together: the N LDS minima are issued back to back, then the
   // marks, then one queue reservation for the wave (three LDS round trips
@@ -1472,29 +1475,41 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
   // qb (once: its inq bit); one above it, or one that finds the buffer full,
   // joins the far set.  All lanes of the wave call it.  imp[j]: target j of
   // this lane improved.
+  // No branch holds an LDS atomic: a lane without a target takes the minimum with
+  // ~0 (or the OR with 0) of a word of its own bank, so that each group of N is
+  // issued together and waited for once (a branch each cost a wait each).  The
+  // slot records of the vertices just queued are loaded now, while the queue is
+  // written and the group meets: the next round finds them in the cache.  2048^2
+  // grid, BFS + SSSP: 11.45 ms, 10.75 with the early loads, 9.9 with both.
   auto relax_many = [&](const auto& act, const auto& li, const auto& cand, auto& imp, int qb, int cb) {
     constexpr int N = (int)(sizeof(act) / sizeof(act[0]));
-    unsigned old[N];
+    unsigned old[N], prev[N];
+    bool near[N];
 #pragma unroll
     for (int j = 0; j < N; ++j)
-      old[j] = act[j] ? __hip_atomic_fetch_min(&dist[li[j]], cand[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                      : 0u;
-    unsigned prev[N];  // the inq word before this lane's mark (the bit itself when nothing is to be queued)
+      old[j] = __hip_atomic_fetch_min(&dist[act[j] ? li[j] : idle_v], act[j] ? cand[j] : ~0u, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_WORKGROUP);
+    bool any = false;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       imp[j] = act[j] && cand[j] < old[j];
-      const unsigned bit = 1u << (li[j] & 31);
-      prev[j] = bit;
-      if (imp[j]) {
-        if (cand[j] < thresh) prev[j] = lds_or(&inq[li[j] >> 5], bit);
-        else lds_or(&farb[li[j] >> 5], bit);
-      }
+      near[j] = imp[j] && cand[j] < thresh;
+      any |= imp[j];
+    }
+    if (!__ballot(any)) return;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      prev[j] = lds_or(&inq[imp[j] ? (li[j] >> 5) + (near[j] ? 0 : W) : idle_w], imp[j] ? 1u << (li[j] & 31) : 0u);
+    if (N <= 2) {  // rounds; a boundary scan's targets are few
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (near[j]) ahead[j & 1] = ((g_ci32*)slots)[(UNIT ? kChunk : 2 * kChunk) * (size_t)(lo + li[j])];
     }
     unsigned long long m[N], all = 0;
     int total = 0;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      m[j] = __ballot(!(prev[j] & (1u << (li[j] & 31))));
+      m[j] = __ballot(near[j] && !(prev[j] & (1u << (li[j] & 31))));
       all |= m[j];
       total += __popcll(m[j]);
     }
@@ -1564,7 +1579,7 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
     }
     if (__ballot(any) && lane == 0) s_flag = 1;
   };
-  // Relaxes the out-edges of queue buffer (qa, count ca) into (qb, cb).
+  // Relaxes the out-edges of queue buffer qa's ln entries into (qb, cb).
   // Several lanes per queued vertex, each relaxing kPer of its slot-record
   // edges: a round is usually run by a few waves, so its length is their
   // instruction count.  BFS: four lanes of one edge; SSSP: two lanes of two
@@ -1572,8 +1587,7 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
   // 2048^2 grid).  The first lane of a vertex marked kSlotCsr walks its CSR
   // row.
   constexpr int kLanes = UNIT ? 4 : 2, kPer = kChunk / kLanes;
-  auto round = [&](int qa, int ca, int qb, int cb) {
-    const int ln = min(s_cnt[ca], qc);
+  auto round = [&](int qa, int ln, int qb, int cb) {
     GDB_FOR_UNIFORM(t, valid, (int)threadIdx.x, (int)blockDim.x, ln * kLanes) {
       // A wave without an entry skips the body: its instructions would take
       // issue slots from the waves on its SIMD that have entries.
@@ -1608,6 +1622,7 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
         }
         if (sl == 0) ++items;
       }
+      asm volatile("" ::"v"(v[0]), "v"(ahead[0]), "v"(ahead[1]));  // the early loads stay in the program
       const bool csr = v[0] == kSlotCsr;  // slot 0 of a vertex with more than kChunk edges
       {
         bool act[kPer], imp[kPer];
@@ -1738,36 +1753,39 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
   };
 
   const unsigned long long limit = (unsigned long long)(unsigned)gdb::ld_rlx(&T.ctx->timeout_ticks.v);
-  int s = 0;  // round number: queue buffer s & 1, counter s % 3
+  int s = 0, c3 = 0;  // round number: queue buffer s & 1, counter c3 = s % 3
+  int scan_in = kScanEvery;
   int epoch = 0;
   bool done = false;
   __syncthreads();
   while (!done) {
     // Local rounds until the queue runs dry.
     for (;;) {
-      const int ca = s % 3;
-      if (s_cnt[ca] == 0) break;
-      const int cb = (s + 1) % 3, qa = s & 1, qb = qa ^ 1;
-      if (threadIdx.x == 0) s_cnt[(s + 2) % 3] = 0;
+      const int ln = min(__builtin_amdgcn_readfirstlane(s_cnt[c3]), qc);
+      if (ln == 0) break;
+      const int cb = c3 == 2 ? 0 : c3 + 1, qa = s & 1, qb = qa ^ 1;
+      if (threadIdx.x == 0) s_cnt[3 - c3 - cb] = 0;
       // A boundary scan every kScanEvery rounds.  When the waves without a
       // queue entry can load every boundary word in one batch, they scan
       // while the others run the round (the two overlap); otherwise the
       // whole group scans after it (a scan costs a far-memory latency per
       // batch).
-      const int split = (min(s_cnt[ca], qc) * kLanes + 63) & ~63;  // threads with an entry, in whole 64-lane waves
-      const bool due = s % kScanEvery == kScanEvery - 1;
+      const int split = (ln * kLanes + 63) & ~63;  // threads with an entry, in whole 64-lane waves
+      const bool due = --scan_in == 0;
+      if (due) scan_in = kScanEvery;
       const bool beside = ((int)blockDim.x - split) * kScanBatch >= nscan;
       if (due && beside && (int)threadIdx.x >= split) {
         scan(qb, cb, (int)threadIdx.x - split, (int)blockDim.x - split);
       } else {
-        round(qa, ca, qb, cb);
+        round(qa, ln, qb, cb);
         if (due && !beside) scan(qb, cb, (int)threadIdx.x, (int)blockDim.x);
       }
       ++s;
+      c3 = cb;
       __syncthreads();
     }
-    if (threadIdx.x == 0) s_cnt[(s + 1) % 3] = 0;
-    if (drain_far(s & 1, s % 3)) continue;
+    if (threadIdx.x == 0) s_cnt[c3 == 2 ? 0 : c3 + 1] = 0;
+    if (drain_far(s & 1, c3)) continue;
     // Idle: arrive on this epoch's counter and poll the boundary.
     int* const arr = T.word(TW_OARR0 + epoch % 3);
     int* const fin = T.word(TW_OFIN0 + epoch % 3);
@@ -1798,7 +1816,7 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
       __syncthreads();
       if (T.l->aborted) return -1;
       if (s_c == G) break;
-      scan(s & 1, s % 3, (int)threadIdx.x, (int)blockDim.x);
+      scan(s & 1, c3, (int)threadIdx.x, (int)blockDim.x);
       __syncthreads();
       if (s_flag) {
         if (threadIdx.x == 0) {
@@ -1825,7 +1843,7 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
     if (!pending) {
       if (threadIdx.x == 0) s_flag = 0;
       __syncthreads();
-      scan(s & 1, s % 3, (int)threadIdx.x, (int)blockDim.x);
+      scan(s & 1, c3, (int)threadIdx.x, (int)blockDim.x);
       __syncthreads();
       pending = s_flag != 0;
     }
@@ -1852,7 +1870,7 @@ __device__ int team_owned(Team& T, const DevTask& k, unsigned long long* work, i
         done = true;
       } else {
         thresh = (band >= kInf - gmin) ? kInf : gmin + band;
-        drain_far(s & 1, s % 3);
+        drain_far(s & 1, c3);
       }
     }
   }

@@ -191,3 +191,21 @@ def test_owned_batch_graph_replays_match_oracle(ctx):
             check(small, BOTH, got)
     finally:
         graph.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 33, 992, 1023, 1025])
+@pytest.mark.parametrize("wgs", [64, 1024])
+def test_owned_range_around_the_idle_lanes_words(ctx, n, wgs):
+    """One range of n vertices: lanes without a target use its first 32 vertices
+    and mark words, or fewer words where it has fewer.  Waves with no target, one
+    and 64 of them; sources at both ends."""
+    rng = np.random.default_rng(n)
+    src = np.concatenate([np.arange(n - 1), np.arange(1, n), rng.integers(0, n, 2 * n)])
+    dst = np.concatenate([np.arange(1, n), np.arange(n - 1), rng.integers(0, n, 2 * n)])
+    order = np.lexsort((dst, src))
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    g = gdb.CSR(n, row, dst[order].astype(np.int32), rng.integers(0, 40, len(src)).astype(np.int32))
+    for source in {0, n - 1}:
+        got, _ = solve(ctx, g, BOTH, 1, wgs=wgs, delta=60, source=source)
+        check(g, BOTH, got, source=source)
