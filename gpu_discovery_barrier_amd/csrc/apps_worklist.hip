@@ -11,7 +11,8 @@
 // (sssp_common.cl:58-81).  Both converge to exact levels / distances.
 //
 // Queues hold each vertex at most once per iteration: BFS claims a vertex
-// with a compare-and-swap on dist, SSSP stamps it with the iteration number;
+// with a compare-and-swap on dist (or sweeps, below), SSSP stamps it with the
+// iteration number;
 // a queue therefore never exceeds n entries (the reference sizes them by the
 // edge count and does not bounds-check pushes, worklist_cl.h:60-62).
 //
@@ -22,7 +23,8 @@
 //   tuned persistent - one barrier per iteration (queue tails rotate over
 //                      three slots so the reset of the next-next tail needs
 //                      no barrier); rows are walked by lanes, waves or in
-//                      pieces; pushes are staged in LDS.
+//                      pieces; pushes are staged in LDS; BFS iterations with
+//                      many edges mark vertices and collect them in a sweep.
 //                      With the launch shape left open, a sparse graph whose
 //                      vertex ids follow locality takes the batched engine's
 //                      owner-partitioned ranges instead (solve_if_local).
@@ -167,6 +169,19 @@ __global__ __launch_bounds__(WGS) void k_wl_plain(gdb_kernel_ctx_t* ctx, const i
 // the queue's items dealt to the waves; R-MAT 18 SSSP: 4.0 -> 1.43 -> 0.86.
 constexpr int kLongRow = 1024;
 
+// BFS iterations with many edges.  Claiming a vertex by compare-and-swap bounds
+// them: every edge to a vertex not reached before the iteration sends one, since
+// plain loads stay stale until the next barrier (a denser filter, a bit per vertex
+// claimed by OR, was slower: 0.67 -> 1.16 ms on R-MAT 20).  Such an iteration claims
+// nothing: its edges set a byte per vertex by plain stores, all of the same value,
+// which later edges of the same XCD see; then all waves sweep the bytes, give the
+// newly marked vertices their level and queue them.  The sweep costs a barrier and
+// 5 bytes per vertex, about 10 us and n / 0.6 ns, against up to 20 ps per claim:
+// hence the line at kSweepEdges + n / kSweepShare edges out of the queue (400000 +
+// n / 12 measured the same; no iteration sweeping: 0.56).  R-MAT 20: 0.65 -> 0.42
+// ms, 17: 0.217 -> 0.203, 12: unchanged.
+constexpr int kSweepEdges = 100000, kSweepShare = 16;
+
 template <int WGS, bool WEIGHTED>
 __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                                   const int* __restrict__ col,
@@ -175,18 +190,37 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
                                                   int4* pieces, int piece_cap, long long* work, int* out) {
   DISCOVERY_PROTOCOL(ctx);
   constexpr int kStage = 8 * WGS;  // pushes of this group awaiting queue space
-  __shared__ int s_q[kStage], s_n, s_base;
+  __shared__ int s_q[kStage], s_n, s_base, s_deg;
   const gdb::PushStage stage{s_q, &s_n, &s_base, kStage};
   const int tid = p_get_global_id(ctx, &local_ctx);
   const int threads = p_get_global_size(ctx, &local_ctx);
   const int lane = gdb::lane_id(), wave = tid >> 6, nwaves = threads >> 6;
   const int spare = n > 0 ? (int)((unsigned)tid % (unsigned)n) : 0;
   int* const piece_counts = tails + 3;  // rotating, like the tails
+  int* const edge_counts = tails + 12;  // BFS: edges of the queued vertices, rotating too
+  unsigned char* const mark = (unsigned char*)stamp;  // BFS: a byte per vertex, set once it is reached
+  const int sweep_from = kSweepEdges + n / kSweepShare;
+  const bool may_sweep = !WEIGHTED && n > 0 && row[n] > sweep_from;
+  // Moves staged vertices to the queue; BFS adds up their edges.
+  auto flush = [&](int above, int* queue, int* tail) {
+    if (may_sweep) {
+      __syncthreads();
+      const int c = min(s_n, kStage);
+      if (c > above) {
+        int d = 0;
+        for (int i = threadIdx.x; i < c; i += WGS) d += row[s_q[i] + 1] - row[s_q[i]];
+        for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
+        if (lane == 0 && d) atomicAdd(&s_deg, d);
+      }
+    }
+    gdb::group_flush(stage, above, queue, tail);
+  };
   int iteration = 1, nbar = 0;
   long long items = 0, edges = 0;
   int nin = gdb::ld_rlx(&tails[1]);
-  if (threadIdx.x == 0) s_n = 0;
+  if (threadIdx.x == 0) s_n = s_deg = 0;
   __syncthreads();
+  int ne = may_sweep && nin > 0 ? row[q0[0] + 1] - row[q0[0]] : 0;
   while (nin > 0) {
     if (nin > n) {
       gdb::set_error(ctx, GDB_ERR_QUEUE_OVERFLOW);
@@ -196,14 +230,23 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
     int* outq = (iteration & 1) ? q1 : q0;
     int* out_tail = &tails[(iteration + 1) % 3];
     int* npieces = &piece_counts[iteration % 3];
+    int* out_edges = &edge_counts[(iteration + 1) % 3];
+    const bool sweep = may_sweep && ne > sweep_from;
     if (tid == 0) {
       gdb::st_rlx(&tails[(iteration + 2) % 3], 0);
       gdb::st_rlx(&piece_counts[(iteration + 1) % 3], 0);
+      gdb::st_rlx(&edge_counts[(iteration + 2) % 3], 0);
     }
     items += nin;
+    auto flush_edges = [&]() {
+      if (may_sweep && threadIdx.x == 0 && s_deg) {
+        gdb::fadd_rlx(out_edges, s_deg);
+        s_deg = 0;
+      }
+    };
     // kChunk edges per lane step (long rows: the whole wave, carrying the
     // row owner's distance): the column and weight loads, then the
-    // targets' distances, then atomics only where a candidate improves
+    // targets' distances (BFS: their marks), then atomics only where a candidate improves
     // (lanes with none send no atomic), then the once-per-iteration stamps
     // of the improved targets, then the pushes.  Unused slots read edge
     // 0 and this thread's spare vertex, so that the slots stay branch-free.
@@ -229,17 +272,21 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
         for (int j = 0; j < kChunk; ++j) {
           act[j] = ok[j] && (unsigned)dst[j] < (unsigned)n && wt[j] < kInf;
           if (!ok[j]) dst[j] = -1;
-          cur[j] = gdb::ldg(dist + (act[j] ? dst[j] : spare));
+          cur[j] = WEIGHTED ? gdb::ldg(dist + (act[j] ? dst[j] : spare)) : (unsigned)gdb::ldg(mark + (act[j] ? dst[j] : spare));
         }
         // A stale distance is never below the current one, so it can
         // only let a needless atomic through.
         bool any_need = false;
 #pragma unroll
         for (int j = 0; j < kChunk; ++j) {
-          need[j] = act[j] && (WEIGHTED ? src + wt[j] < cur[j] : cur[j] == kInf);
+          need[j] = act[j] && (WEIGHTED ? src + wt[j] < cur[j] : cur[j] == 0u);
           any_need |= need[j];
         }
-        if (any_need) {
+        if (sweep) {
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j)
+            if (need[j]) mark[dst[j]] = 1;
+        } else if (any_need) {
           unsigned old[kChunk];
           bool imp[kChunk], any_imp = false;
 #pragma unroll
@@ -255,7 +302,10 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
           if (!WEIGHTED) {
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) push[j] = imp[j];
+            for (int j = 0; j < kChunk; ++j) {
+              push[j] = imp[j];
+              if (imp[j]) mark[dst[j]] = 1;
+            }
           } else if (any_imp) {
             // Stamps only grow (iteration numbers): the first to raise
             // one to this iteration queues the target.
@@ -268,7 +318,7 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
         }
       }
-      gdb::wave_stage_n<kChunk>(stage, push, dst, outq, out_tail);
+      if (!sweep) gdb::wave_stage_n<kChunk>(stage, push, dst, outq, out_tail);
       return 0;
     };
     auto any = [](int a, int c) { return a | c; };
@@ -293,9 +343,10 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
         }
       }
       gdb::wave_walk_np<kChunk>(valid != 0, b, e, (int)dv, 0, step, any, kSerialLimit);
-      gdb::group_flush(stage, kStage / 2, outq, out_tail);
+      flush(kStage / 2, outq, out_tail);
     }
-    gdb::group_flush(stage, 0, outq, out_tail);
+    flush(0, outq, out_tail);
+    flush_edges();
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
     const int np = min(gdb::ld_rlx(npieces), piece_cap);
@@ -313,12 +364,40 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
           step(ok, kk, pc.z);
         }
-        gdb::group_flush(stage, kStage / 2, outq, out_tail);
+        flush(kStage / 2, outq, out_tail);
       }
-      gdb::group_flush(stage, 0, outq, out_tail);
+      flush(0, outq, out_tail);
+      flush_edges();
       if (!discovery_barrier(ctx, &local_ctx)) return;
       ++nbar;
     }
+    if (sweep) {
+      for (long long p0 = 0; p0 < n; p0 += (long long)kChunk * threads) {
+        bool push[kChunk];
+        int v[kChunk];
+        unsigned mk[kChunk], dv[kChunk];
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+          const long long i = p0 + (long long)j * threads + tid;
+          push[j] = i < n;
+          v[j] = (int)i;
+          mk[j] = gdb::ldg(mark + (push[j] ? v[j] : spare));
+          dv[j] = gdb::ldg(dist + (push[j] ? v[j] : spare));
+        }
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+          push[j] = push[j] && mk[j] != 0 && dv[j] == kInf;
+          if (push[j]) dist[v[j]] = (unsigned)iteration;
+        }
+        gdb::wave_stage_n<kChunk>(stage, push, v, outq, out_tail);
+        flush(kStage / 2, outq, out_tail);
+      }
+      flush(0, outq, out_tail);
+      flush_edges();
+      if (!discovery_barrier(ctx, &local_ctx)) return;
+      ++nbar;
+    }
+    if (may_sweep) ne = gdb::ld_rlx(out_edges);
     nin = gdb::ld_rlx(out_tail);
     ++iteration;
   }
@@ -379,13 +458,13 @@ __global__ void k_wl_step(const int* __restrict__ row, const int* __restrict__ c
   }
 }
 
-__global__ void k_wl_init(unsigned* dist, int* stamp, int* q0, int* q1, int* flags, int n, int src) {
+__global__ void k_wl_init(unsigned* dist, int* stamp, int* q0, int* q1, int* flags, int n, int src, bool bytes) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {  // initialize (bfs_common.cl:64-71) + dist[source] = 0
     dist[i] = i == src ? 0u : kInf;
-    stamp[i] = 0;
+    stamp[i] = bytes && i == src >> 2 ? 1 << 8 * (src & 3) : 0;  // bytes: the source is marked
   }
-  if (i < 16) flags[i] = 0;
+  if (i < 32) flags[i] = 0;
   if (i == 0) {  // iteration 0: push the source (bfs_port_kernel.cl:130-137)
     q0[0] = src;
     q1[0] = src;
@@ -593,7 +672,7 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   rc = prepare_launch(ctx, (int*)work, 4);
   if (rc) return rc;
   hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, dist, stamp, q0, q1,
-                     flags, n, source);
+                     flags, n, source, !WEIGHTED);
   GDB_HIP(hipGetLastError());
 
   if (o.schedule == GDB_SCHED_RELAUNCH) {

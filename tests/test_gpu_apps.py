@@ -94,6 +94,26 @@ def test_mis_one_deciding_edge(ctx, deg, extra):
     assert (got == want).all() and st.rounds == rounds
 
 
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1025])
+@pytest.mark.parametrize("wgs,groups", [(64, 1), (256, 3), (0, 0)])
+def test_bfs_sweep(ctx, n, wgs, groups):
+    """Iterations of more than 100000 edges, by one row and by many, among small
+    ones; sizes around what one trip of the sweep covers."""
+    rng = np.random.default_rng(n)
+    chain = np.arange(n - 1)
+    mid = n // 2
+    src = np.concatenate([np.zeros(120000, np.int64), chain, rng.integers(0, max(1, mid), 130000)])
+    dst = np.concatenate([rng.integers(0, max(1, mid), 120000), chain + 1, rng.integers(0, n - n // 4, 130000)])
+    order = np.argsort(src, kind="stable")
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    col = dst[order].astype(np.int32)
+    for source in {0, n - 1}:
+        want, rounds = oracle.bfs_worklist_ref(row, col, source)
+        got, st = gdb.bfs_worklist(ctx, dev(row, col), source, gdb.Opts.make(wgs=wgs, groups=groups))
+        assert (got == want).all() and st.rounds == rounds
+
+
 # ---------------------------------------------------------------- pull SSSP
 @pytest.mark.parametrize("sched", SCHEDS, ids=SID)
 @pytest.mark.parametrize("fx", FX["sssp_pull"], ids=lambda f: f["name"])
