@@ -381,6 +381,7 @@ __global__ __launch_bounds__(WGS) void k_bc_tuned(gdb_kernel_ctx_t* ctx, const i
 // fetch-or of their nibbles (every claimer in step t ors the same level-t+1
 // nibble, and the winners are the sources whose reached bit it set); each
 // winner stores the full level in lev.
+typedef unsigned long long u64;
 constexpr int kMS = 8;
 constexpr int kNR = kMS / 4;  // int4 per lev / sg record
 // Edge slots per lane step: the gathers of a step are in flight together.
@@ -444,11 +445,15 @@ __device__ __forceinline__ int* rec_int(int4* a, size_t v, int s) { return (int*
 // pass).  The long walk is always cut into kParts parts, walked by whichever
 // waves there are and summed in order, so that sums do not depend on the launch
 // shape.  R-MAT 22, 16 sources: 27.5 ms against 33 without the two.
+// Forward steps with many edges (gdb::sweep_line) set a byte per vertex and source
+// by plain stores in place of three dependent atomics, and a sweep turns the bytes
+// into code nibbles, levels and queue entries: 27.8 -> 23.4 ms; R-MAT 18 3.0 -> 2.3,
+// 14 with 8 sources 0.42 -> 0.36.
 constexpr int kLongRowM = 4096, kParts = 8;
 template <int WGS>
 __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                                   const int* __restrict__ col, int4* lev, int4* sg,
-                                                  unsigned* code, float* bc, const int* sources, int nsrc,
+                                                  unsigned* code, u64* marks, float* bc, const int* sources, int nsrc,
                                                   int* q, int* stamp, int* loff, int* tail, int n, int* out) {
   DISCOVERY_PROTOCOL(ctx);
   const int tid = p_get_global_id(ctx, &local_ctx);
@@ -458,12 +463,12 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
   const int spare = (int)((unsigned)tid % (unsigned)n);
   const int qcap = kMS * n;  // a vertex is queued at most once per source level
   constexpr int kStage = 4 * WGS;
-  __shared__ int s_q[kStage], s_n, s_base, s_nlong;
+  __shared__ int s_q[kStage], s_n, s_base, s_nlong, s_deg;
   __shared__ int4 s_long[WGS];  // long rows of this trip: vertex, source mask, first edge, end
   __shared__ float s_part[kParts][kMS];
   const gdb::PushStage stage{s_q, &s_n, &s_base, kStage};
   const int lane = gdb::lane_id(), wave = (int)threadIdx.x >> 6;
-  if (threadIdx.x == 0) s_n = s_nlong = 0;
+  if (threadIdx.x == 0) s_n = s_nlong = s_deg = 0;
   // The group walks edges [b, e) with `step`, a part of them per wave at a
   // time, and leaves the sums over the parts in s_part[0].
   auto group_walk = [&](int b, int e, int mask, auto& step) {
@@ -506,6 +511,14 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     }
     if (nl > 0 && threadIdx.x == 0) s_nlong = 0;
   };
+  unsigned char* const mark = (unsigned char*)marks;  // a byte per vertex and source
+  int* const edge_counts = tail + 12;                 // edges of the next step's vertices, rotating
+  const int sweep_from = gdb::sweep_line(n);
+  const bool may_sweep = row[n] > sweep_from;
+  auto flush = [&](int above) {
+    if (may_sweep) gdb::stage_edges(stage, above, row, &s_deg);
+    gdb::group_flush(stage, above, q, tail);
+  };
   int nbar = 0, levels = 0;
   auto reset = [&](int v) {
 #pragma unroll
@@ -518,6 +531,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
   };
   for (int i = tid; i < n; i += stride) {
     bc[i] = 0.f;
+    marks[i] = 0ull;
     reset(i);
   }
   int prev_reached = 0;
@@ -543,6 +557,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
       }
       loff[0] = 0;
       loff[1] = cnt;
+      gdb::st_rlx(&edge_counts[1], 0);
       gdb::st_rlx(tail, cnt);
     }
     if (!discovery_barrier(ctx, &local_ctx)) return;
@@ -550,7 +565,11 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     const unsigned all = ns >= 32 ? ~0u : (1u << ns) - 1u;
     // Forward.
     int lb = 0, le = gdb::ld_rlx(tail), t = 0;
+    int ne = 0;  // the sources' own edges: a step of eight vertices claims
     for (;;) {
+      const bool sweep = may_sweep && ne > sweep_from;
+      int* const out_edges = &edge_counts[(t + 1) % 3];
+      if (tid == 0) gdb::st_rlx(&edge_counts[(t + 2) % 3], 0);
       const unsigned par = (unsigned)(t - 1) & 3u;                    // parents' level mod 4
       const unsigned nxt_nib = 8u | ((unsigned)(t + 1) & 3u);         // a claimed nibble
       GDB_FOR_SPREAD(i, valid, tid, stride, le - lb, 0) {
@@ -613,7 +632,11 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
                 // Only lanes with an unreached target send claims: one fetch-or
                 // of the claimed nibbles (winners are the sources whose reached
                 // bit it set), then each winner stores the full level.
-                if (any_claim) {
+                if (sweep) {
+#pragma unroll
+                  for (int j = 0; j < kSlotsM; ++j)
+                    for (unsigned r = cl[j]; r; r &= r - 1) mark[(size_t)w[j] * kMS + ((__ffs(r) - 1) >> 2)] = 1;
+                } else if (any_claim) {
                   unsigned oldc[kSlotsM];
 #pragma unroll
                   for (int j = 0; j < kSlotsM; ++j)
@@ -641,7 +664,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
                   }
                 }
               }
-              gdb::wave_stage_n<kSlotsM>(stage, push, w, q, tail);
+              if (!sweep) gdb::wave_stage_n<kSlotsM>(stage, push, w, q, tail);
               return acc;
         };
         const bool own = valid && mask != 0 && e - b <= kLongRowM;
@@ -657,11 +680,52 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
           const int s = (int)threadIdx.x;
           if (s < kMS && t > 0 && ((lm >> s) & 1u)) *rec_int(sg, lv, s) = __float_as_int(s_part[0][s]);
         });
-        gdb::group_flush(stage, kStage / 2, q, tail);
+        flush(kStage / 2);
       }
-      gdb::group_flush(stage, 0, q, tail);
+      if (sweep) {
+        if (!discovery_barrier(ctx, &local_ctx)) return;
+        ++nbar;
+        constexpr int kV = 4;  // vertices per thread and trip
+        for (long long p0 = 0; p0 < n; p0 += (long long)kV * stride) {
+          bool push[kV];
+          int v[kV];
+          u64 mk[kV];
+          unsigned c[kV];
+#pragma unroll
+          for (int j = 0; j < kV; ++j) {
+            const long long i = p0 + (long long)j * stride + tid;
+            push[j] = i < n;
+            v[j] = push[j] ? (int)i : spare;
+            mk[j] = gdb::ldg(marks + v[j]);
+            c[j] = gdb::ldg(code + v[j]);
+          }
+#pragma unroll
+          for (int j = 0; j < kV; ++j) {
+            push[j] = push[j] && mk[j] != 0ull;
+            if (!push[j]) continue;
+            marks[v[j]] = 0ull;
+            unsigned got = 0;
+#pragma unroll
+            for (int s = 0; s < kMS; ++s) got |= ((unsigned)(mk[j] >> (8 * s)) & 1u) << (4 * s);
+            got &= (~c[j] >> 3) & kNibLo;
+            push[j] = got != 0u;
+            code[v[j]] = c[j] | got * nxt_nib;
+#pragma unroll
+            for (int s = 0; s < kMS; ++s)
+              if ((got >> (4 * s)) & 1u) *rec_int(lev, v[j], s) = t + 1;
+          }
+          gdb::wave_stage_n<kV>(stage, push, v, q, tail);
+          flush(kStage / 2);
+        }
+      }
+      flush(0);
+      if (may_sweep && threadIdx.x == 0 && s_deg) {
+        gdb::fadd_rlx(out_edges, s_deg);
+        s_deg = 0;
+      }
       if (!discovery_barrier(ctx, &local_ctx)) return;
       ++nbar;
+      if (may_sweep) ne = gdb::ld_rlx(out_edges);
       const int tn = gdb::ld_rlx(tail);
       if (tn > qcap || tn < le) {  // stamps queue a vertex once per step
         gdb::set_error(ctx, GDB_ERR_QUEUE_OVERFLOW);
@@ -777,9 +841,12 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
 // pulls coef from the out-neighbours with byte tt + 2.  A search deeper than
 // kMaxStepD raises *deep and the caller runs k_bc_tuned.
 //
+// A step with many edges (gdb::sweep_line) stores the bytes plainly instead of
+// claiming them, and a sweep over the code words queues the vertices with a byte of
+// the next step.
+//
 // What it saves is steps: eight sources share one sweep's barriers and
 // dependent gathers.  R-MAT 15, 8 sources: 0.49 ms against 2.1 one by one.
-typedef unsigned long long u64;
 constexpr int kSlotsD = 8;
 constexpr int kMaxStepD = 253;  // byte kMaxStepD + 2 is the last one
 
@@ -811,9 +878,17 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
   const int spare = (int)((unsigned)tid % (unsigned)n);
   const int qcap = kMS * n;
   constexpr int kStage = 4 * WGS;
-  __shared__ int s_q[kStage], s_n, s_base;
+  __shared__ int s_q[kStage], s_n, s_base, s_deg;
   const gdb::PushStage stage{s_q, &s_n, &s_base, kStage};
-  if (threadIdx.x == 0) s_n = 0;
+  if (threadIdx.x == 0) s_n = s_deg = 0;
+  unsigned char* const mark = (unsigned char*)code;
+  int* const edge_counts = tail + 12;  // edges of the next step's vertices, rotating
+  const int sweep_from = gdb::sweep_line(n);
+  const bool may_sweep = row[n] > sweep_from;
+  auto flush = [&](int above) {
+    if (may_sweep) gdb::stage_edges(stage, above, row, &s_deg);
+    gdb::group_flush(stage, above, q, tail);
+  };
   int nbar = 0, levels = 0;
   auto reset = [&](int v) {
 #pragma unroll
@@ -883,13 +958,18 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
       }
       loff[0] = 0;
       loff[1] = cnt;
+      gdb::st_rlx(&edge_counts[1], 0);
       gdb::st_rlx(tail, cnt);
     }
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
     const unsigned all = (1u << ns) - 1u;
     int lb = 0, le = gdb::ld_rlx(tail), t = 0;
+    int ne = 0;  // the sources' own edges: a step of eight vertices claims
     for (;;) {
+      const bool sweep = may_sweep && ne > sweep_from;
+      int* const out_edges = &edge_counts[(t + 1) % 3];
+      if (tid == 0) gdb::st_rlx(&edge_counts[(t + 2) % 3], 0);
       if (t > kMaxStepD) {
         if (tid == 0) *deep = 1;
         return;
@@ -937,7 +1017,12 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
                   cl[j] = bytes_equal(gdb::ldg(code + (in ? w[j] : spare)), 0u) & (in ? omb : 0ull);
                   any_claim |= cl[j] != 0ull;
                 }
-                if (any_claim) {
+                if (sweep) {
+#pragma unroll
+                  for (int j = 0; j < kSlotsD; ++j)
+                    for (u64 r = cl[j]; r; r &= r - 1)
+                      mark[(size_t)w[j] * kMS + ((__ffsll((long long)r) - 1) >> 3)] = (unsigned char)(t + 2);
+                } else if (any_claim) {
                   u64 old[kSlotsD];
 #pragma unroll
                   for (int j = 0; j < kSlotsD; ++j)
@@ -958,7 +1043,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
                   }
                 }
               }
-              gdb::wave_stage_n<kSlotsD>(stage, push, w, q, tail);
+              if (!sweep) gdb::wave_stage_n<kSlotsD>(stage, push, w, q, tail);
               return 0;
             },
             [](int a, int c) { return a | c; }, kSerialLimit);
@@ -967,11 +1052,37 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
           for (int s = 0; s < kMS; ++s)
             if ((mask >> s) & 1u) *rec_int(sg, v, s) = __float_as_int(sgm.v[s]);
         }
-        gdb::group_flush(stage, kStage / 2, q, tail);
+        flush(kStage / 2);
       }
-      gdb::group_flush(stage, 0, q, tail);
+      if (sweep) {
+        if (!discovery_barrier(ctx, &local_ctx)) return;
+        ++nbar;
+        constexpr int kV = 4;  // vertices per thread and trip
+        for (long long p0 = 0; p0 < n; p0 += (long long)kV * stride) {
+          bool push[kV];
+          int v[kV];
+          u64 c[kV];
+#pragma unroll
+          for (int j = 0; j < kV; ++j) {
+            const long long i = p0 + (long long)j * stride + tid;
+            push[j] = i < n;
+            v[j] = push[j] ? (int)i : spare;
+            c[j] = gdb::ldg(code + v[j]);
+          }
+#pragma unroll
+          for (int j = 0; j < kV; ++j) push[j] = push[j] && bytes_equal(c[j], (unsigned)t + 2u) != 0ull;
+          gdb::wave_stage_n<kV>(stage, push, v, q, tail);
+          flush(kStage / 2);
+        }
+      }
+      flush(0);
+      if (may_sweep && threadIdx.x == 0 && s_deg) {
+        gdb::fadd_rlx(out_edges, s_deg);
+        s_deg = 0;
+      }
       if (!discovery_barrier(ctx, &local_ctx)) return;
       ++nbar;
+      if (may_sweep) ne = gdb::ld_rlx(out_edges);
       const int tn = gdb::ld_rlx(tail);
       if (tn > qcap || tn < le) {  // stamps queue a vertex once per step
         gdb::set_error(ctx, GDB_ERR_QUEUE_OVERFLOW);
@@ -1174,9 +1285,9 @@ extern "C" int gdb_bc(gdb_ctx* ctx, int n, int m, const int* row, const int* col
       if (r2) return r2;
       r2 = timer_start(ctx);
       if (r2) return r2;
-      if (multi)  // mst holds lev then sg; d the per-vertex queue stamps; q the level codes
+      if (multi)  // mst holds lev then sg; d the per-vertex queue stamps; q the level codes; ds the marks
         hipLaunchKernelGGL(k_bc_multi<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col, mst,
-                           mst + (size_t)kNR * n, (unsigned*)q, bc, sources, nsrc, mq, d, mloff, flags + 4, n,
+                           mst + (size_t)kNR * n, (unsigned*)q, (u64*)ds, bc, sources, nsrc, mq, d, mloff, flags + 4, n,
                            out);
       else if (multi_directed)  // ds holds the code words
         hipLaunchKernelGGL(k_bc_multi_directed<WG>, dim3(groups), dim3(WG), 0, ctx->stream, ctx->d, row, col, row_t,

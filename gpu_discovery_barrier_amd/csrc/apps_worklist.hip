@@ -169,18 +169,11 @@ __global__ __launch_bounds__(WGS) void k_wl_plain(gdb_kernel_ctx_t* ctx, const i
 // the queue's items dealt to the waves; R-MAT 18 SSSP: 4.0 -> 1.43 -> 0.86.
 constexpr int kLongRow = 1024;
 
-// BFS iterations with many edges.  Claiming a vertex by compare-and-swap bounds
-// them: every edge to a vertex not reached before the iteration sends one, since
-// plain loads stay stale until the next barrier (a denser filter, a bit per vertex
-// claimed by OR, was slower: 0.67 -> 1.16 ms on R-MAT 20).  Such an iteration claims
-// nothing: its edges set a byte per vertex by plain stores, all of the same value,
-// which later edges of the same XCD see; then all waves sweep the bytes, give the
-// newly marked vertices their level and queue them.  The sweep costs a barrier and
-// 5 bytes per vertex, about 10 us and n / 0.6 ns, against up to 20 ps per claim:
-// hence the line at kSweepEdges + n / kSweepShare edges out of the queue (400000 +
-// n / 12 measured the same; no iteration sweeping: 0.56).  R-MAT 20: 0.65 -> 0.42
-// ms, 17: 0.217 -> 0.203, 12: unchanged.
-constexpr int kSweepEdges = 100000, kSweepShare = 16;
+// BFS iterations with many edges (gdb::sweep_line) set a byte per vertex by plain
+// stores, all of the same value, which later edges of the same XCD see; then all
+// waves sweep the bytes, give the newly marked vertices their level and queue them.
+// R-MAT 20: 0.65 -> 0.42 ms, 17: 0.217 -> 0.203, 12: unchanged.  A bit per vertex
+// claimed by OR, as a denser filter in place of dist, was slower: 1.16 ms.
 
 template <int WGS, bool WEIGHTED>
 __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
@@ -199,20 +192,11 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
   int* const piece_counts = tails + 3;  // rotating, like the tails
   int* const edge_counts = tails + 12;  // BFS: edges of the queued vertices, rotating too
   unsigned char* const mark = (unsigned char*)stamp;  // BFS: a byte per vertex, set once it is reached
-  const int sweep_from = kSweepEdges + n / kSweepShare;
+  const int sweep_from = gdb::sweep_line(n);
   const bool may_sweep = !WEIGHTED && n > 0 && row[n] > sweep_from;
   // Moves staged vertices to the queue; BFS adds up their edges.
   auto flush = [&](int above, int* queue, int* tail) {
-    if (may_sweep) {
-      __syncthreads();
-      const int c = min(s_n, kStage);
-      if (c > above) {
-        int d = 0;
-        for (int i = threadIdx.x; i < c; i += WGS) d += row[s_q[i] + 1] - row[s_q[i]];
-        for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
-        if (lane == 0 && d) atomicAdd(&s_deg, d);
-      }
-    }
+    if (may_sweep) gdb::stage_edges(stage, above, row, &s_deg);
     gdb::group_flush(stage, above, queue, tail);
   };
   int iteration = 1, nbar = 0;

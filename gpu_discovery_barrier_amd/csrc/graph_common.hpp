@@ -262,6 +262,27 @@ __device__ __forceinline__ void group_flush(const PushStage& st, int above, int*
   __syncthreads();
 }
 
+// Traversal steps with more edges out of their queue than this mark what they reach
+// by plain stores and collect it in a sweep over all vertices; steps with fewer
+// claim each vertex by an atomic.  Claims bound the large steps: plain loads stay
+// stale until the next barrier, so nearly every edge to a vertex not reached before
+// the step sends one, up to 20 ps each.  A sweep costs a barrier and a few bytes
+// per vertex, about 10 us and n / 0.5 ns.  (Lines from 50000 + n / 8 to 400000 + n /
+// 12 measured within 3% of each other in BFS and BC.)
+__host__ __device__ inline int sweep_line(int n) { return 100000 + n / 16; }
+
+// Adds the edges of the staged vertices that group_flush(st, above, ...) is about
+// to move to *sum (LDS).  Called by all threads, right before it.
+__device__ __forceinline__ void stage_edges(const PushStage& st, int above, const int* row, int* sum) {
+  __syncthreads();
+  const int c = *st.count < st.cap ? *st.count : st.cap;
+  if (c <= above) return;
+  int d = 0;
+  for (int i = threadIdx.x; i < c; i += blockDim.x) d += row[st.items[i] + 1] - row[st.items[i]];
+  for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
+  if (lane_id() == 0 && d) atomicAdd(sum, d);
+}
+
 // Wave-wide OR of a predicate.
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0ull; }
 

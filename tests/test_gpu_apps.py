@@ -213,6 +213,35 @@ def test_bc_sweeps_partial_batch_and_repeated_sources(ctx):
         bc_close(got, want)
 
 
+@pytest.mark.parametrize("n", [1023, 1024, 1030])
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("wgs,groups", [(64, 4), (256, 3), (0, 0)])
+def test_bc_step_with_many_edges(ctx, n, directed, wgs, groups):
+    """A random core of 130 edges per vertex and a path of seven: steps that sweep
+    between steps that claim, two batches of sources, around a trip's vertices."""
+    rng = np.random.default_rng(n)
+    core = n - 7
+    a = np.concatenate([rng.integers(0, core, 130 * core), np.arange(core - 1, n - 1)])
+    b = np.concatenate([rng.integers(0, core, 130 * core), np.arange(core, n)])
+    key = a * n + b
+    key = np.unique(key if directed else np.concatenate([key, b * n + a]))
+    key = key[key // n != key % n]
+
+    def csr(k):
+        row = np.zeros(n + 1, np.int32)
+        row[1:] = np.cumsum(np.bincount(k // n, minlength=n))
+        return row, (k % n).astype(np.int32)
+
+    row, col = csr(key)
+    assert len(col) > 120000
+    src = np.concatenate([[n - 1], rng.permutation(n)[:10]]).astype(np.int32)
+    want = oracle.bc_brandes_tb(row, col, src)
+    g = dev(row, col)
+    gt = dev(*csr(np.sort(key % n * n + key // n))) if directed else g
+    got, _ = gdb.bc(ctx, g, gt, src, gdb.Opts.make(wgs=wgs, groups=groups))
+    bc_close(got, want)
+
+
 def test_bc_tuned_is_deterministic(ctx):
     g = gdb.gen_rmat(12, 16, seed=8)
     src = gdb.permutation(g.n, 8)[:8]
