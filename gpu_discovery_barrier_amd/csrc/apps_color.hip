@@ -527,12 +527,19 @@ __global__ __launch_bounds__(WGS) void k_color_flow(gdb_kernel_ctx_t* ctx, const
   }
 }
 
-// Colours and round count of a finished k_color_flow.
+// Colours and round count of a finished k_color_flow.  A wave takes `per` vertices:
+// 64 neighbours of a sparse graph, kOutRows of a dense one, each from another part
+// of the ids (64 neighbouring rows of an R-MAT graph's hubs on one wave were the
+// kernel's length: 81 us on R-MAT 14, 17 with 4 vertices a wave, 21 with 8, 32 with
+// 16).
+constexpr int kOutRows = 4;
 __global__ __launch_bounds__(256) void k_flow_out(const int* __restrict__ row, const int* __restrict__ col, int n,
-                                                  const int* __restrict__ poll, int* color, int* fw) {
+                                                  int per, const int* __restrict__ poll, int* color, int* fw) {
   if (fw[FW_GAVE_UP] || fw[FW_INVALID]) return;
-  const int v = blockIdx.x * 256 + threadIdx.x;
-  const bool valid = v < n;
+  const int lane = gdb::lane_id(), wave = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int share = (n + per - 1) / per;  // waves with vertices
+  const int v = per == 64 ? wave * 64 + lane : lane * share + wave;
+  const bool valid = wave < share && lane < per && v < n;
   int b = 0, e = 0, cv = 0;
   if (valid) {
     b = row[v];
@@ -560,8 +567,13 @@ __global__ __launch_bounds__(256) void k_flow_out(const int* __restrict__ row, c
         return best;
       },
       [](int a, int c) { return max(a, c); }, kSerialLimit);
+  __shared__ int s_max;  // one word of device memory takes 10 ns per atomic: one a group, if any
+  if (threadIdx.x == 0) s_max = 0;
+  __syncthreads();
   const int rm = gdb::wave_max(r);
-  if (gdb::lane_id() == 0 && rm > 0) atomicMax(&fw[FW_ROUNDS], rm);
+  if (lane == 0 && rm > 0) atomicMax(&s_max, rm);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_max > gdb::ld_rlx(&fw[FW_ROUNDS])) atomicMax(&fw[FW_ROUNDS], s_max);
 }
 
 // The same in one group, for a graph of at most kFlow1N vertices and 1024 *
@@ -815,7 +827,9 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
                          fw);
       hipLaunchKernelGGL(k_color_flow<WG>, dim3(nwin), dim3(WG), lds, ctx->stream, ctx->d, row, col, nv, n, m, poll,
                          gmx, gcnt, fw, limit);
-      hipLaunchKernelGGL(k_flow_out, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, row, col, n, poll, color, fw);
+      const int per = gdb::spread_rows(n, m) ? 64 : kOutRows;
+      hipLaunchKernelGGL(k_flow_out, dim3((n + 4 * per - 1) / (4 * per)), dim3(256), 0, ctx->stream, row, col, n, per,
+                         poll, color, fw);
       GDB_HIP(hipGetLastError());
       ran = true;
       s->launches = 3;

@@ -520,7 +520,7 @@ __global__ void k_levels(const unsigned* __restrict__ dist, int n, int* out) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     if (dist[i] < kInf) m = max(m, (int)dist[i] + 1);
   m = gdb::wave_max(m);
-  if (gdb::lane_id() == 0 && m > 0) atomicMax(out, m);
+  if (gdb::lane_id() == 0 && m > gdb::ld_rlx(out)) atomicMax(out, m);  // 10 ns each on one word
 }
 
 // Solves a sparse local graph (grids, meshes, road networks) by the batched

@@ -446,6 +446,6 @@ __device__ __forceinline__ long long spread_item(int start, int stride, int sh) 
 // one where rows are long enough to be walked by waves (four or eight at a time
 // measured 2 to 25% slower on R-MAT graphs), 64 together where they are short
 // (2^20-vertex grid MST 1.16 ms against 1.44).
-__device__ __forceinline__ int spread_rows(int n, long long m) { return m >= 8LL * n ? 0 : 6; }
+__host__ __device__ inline int spread_rows(int n, long long m) { return m >= 8LL * n ? 0 : 6; }
 
 }  // namespace gdb

@@ -148,6 +148,19 @@ def test_color_flow_edges(ctx, n, m, hub, wgs, groups):
     assert (got == want).all() and st.rounds == rr
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1025, 4099])
+@pytest.mark.parametrize("per", [7, 9])
+def test_color_flow_rounds_of_sparse_and_dense(ctx, n, per):
+    """Either side of eight edges a vertex, where the last kernel deals its
+    vertices out; sizes that leave its last waves part of a share."""
+    m = per * n if n > 1 else 0
+    row, col = directed(n, m, n, n // 4) if n > 1 else (np.zeros(2, np.int32), np.zeros(0, np.int32))
+    nv = (1 + np.random.default_rng(n).permutation(n).astype(np.float32)) / np.float32(n + 1)
+    want, rr = oracle.color_ref(row, col, nv)
+    got, st = run(ctx, row, col, nv, wgs=256, variant=gdb.VARIANT_TUNED)
+    assert (got == want).all() and st.rounds == rr
+
+
 @pytest.mark.parametrize("n", [3, 9000])
 def test_color_flow_ties_then_clean(ctx, n):
     # A cycle of equal priorities never resolves; the next solve on the same
