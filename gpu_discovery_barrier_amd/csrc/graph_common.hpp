@@ -304,7 +304,12 @@ __device__ __forceinline__ bool any_slot(const bool (&ok)[N]) {
 // the N slots cost one chain of memory round trips.  Short ranges are walked
 // by their own lane N edges per step; long ranges by the whole wave, N x 64
 // consecutive edges per step (slot j of lane i takes edge base + i + 64 j, so
-// each slot's loads are coalesced), and reduced into the owner lane.
+// each slot's loads are coalesced), and reduced into the owner lane.  Ranges of at
+// most 16 N edges, still long, are walked four at a time, 16 lanes each: one such
+// row on the whole wave leaves most slots empty and costs the same chain of trips
+// (BC on directed R-MAT 15 0.45 -> 0.40 ms, on R-MAT 22 23.4 -> 21.7; pull SSSP R-MAT
+// 16 0.44 -> 0.41; BFS R-MAT 20 0.42 -> 0.40; MST R-MAT 18 0.59 -> 0.575).  Which way a
+// range is walked depends on its length alone, and so does the order of its sum.
 // As wave_walk_n, but step(ok, kk, owner) also gets the `payload` of the
 // range's owner lane (for a long row walked by the whole wave, the leader's
 // payload on every lane).
@@ -325,8 +330,38 @@ __device__ __forceinline__ T wave_walk_np(bool active, int b, int e, int payload
     }
     acc = red(acc, step(ok, kk, payload));
   }
-  unsigned long long mask = __ballot(heavy);
   const int lane = lane_id();
+  const bool mid = heavy && (e - b) <= 16 * N;
+  unsigned long long mask = __ballot(mid);
+  while (mask) {
+    int owner[4];  // the owners of this trip's ranges, -1 none
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      owner[q] = mask ? __ffsll((long long)mask) - 1 : -1;
+      mask &= mask - 1;
+    }
+    const int mine = lane < 32 ? (lane < 16 ? owner[0] : owner[1]) : (lane < 48 ? owner[2] : owner[3]);
+    const int from = mine < 0 ? 0 : mine;
+    const int lb = __shfl(b, from, 64), le = __shfl(e, from, 64), lp = __shfl(payload, from, 64);
+    bool ok[N];
+    int kk[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      kk[j] = lb + (lane & 15) + 16 * j;
+      ok[j] = mine >= 0 && kk[j] < le;
+    }
+    T part = red(identity, step(ok, kk, lp));
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) part = red(part, shfl_xor(part, off));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      T x = (lane >> 4) == q ? part : identity;
+      x = red(x, shfl_xor(x, 16));
+      x = red(x, shfl_xor(x, 32));
+      if (lane == owner[q]) acc = x;
+    }
+  }
+  mask = __ballot(heavy && !mid);
   while (mask) {
     const int leader = __ffsll((long long)mask) - 1;
     const int lb = bcast(b, leader);

@@ -558,3 +558,36 @@ def test_bc_directed_sweeps(ctx, shape, nsrc, wgs, groups):
     got, _ = gdb.bc(ctx, gdb.DeviceCSR(g), gdb.DeviceCSR(gt), sources,
                     gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED))
     bc_close(got, np.asarray(oracle.bc_brandes_tb(row, col, sources), np.float64))
+
+
+@pytest.mark.parametrize("deg", [15, 16, 17, 63, 64, 65, 128, 129, 192, 193])
+@pytest.mark.parametrize("hubs", [1, 3, 4, 5, 64])
+def test_rows_walked_by_part_of_a_wave(ctx, deg, hubs):
+    """Rows either side of what a lane, a quarter of a wave and a wave walk (16
+    edges; 16 for each of 4, 8 or 12 slots a lane), one to 64 of them together."""
+    rng = np.random.default_rng(deg + hubs)
+    n = 300 + hubs
+    a, b = [np.arange(n)], [np.roll(np.arange(n), -1)]
+    for h in range(hubs):
+        a.append(np.full(deg - 2, h))
+        b.append(hubs + 1 + rng.permutation(n - hubs - 2)[:deg - 2])
+    a, b = np.concatenate(a), np.concatenate(b)
+    key = np.unique(np.concatenate([a * n + b, b * n + a]))
+    src, col = key // n, (key % n).astype(np.int32)
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    lo, hi = np.minimum(src, col), np.maximum(src, col)
+    w = (1 + (lo * 7919 + hi * 104729) % 97).astype(np.int32)
+    g = gdb.DeviceCSR(gdb.CSR(n, row, col, w))
+    sources = np.concatenate([[0, n - 1], rng.permutation(n)[:7]]).astype(np.int32)
+    assert (np.diff(row)[:hubs] == deg).all()
+    want = oracle.bc_brandes_tb(row, col, sources)
+    for gt in (g, gdb.DeviceCSR(gdb.CSR(n, row, col, w))):  # as its own transpose, and as a directed graph
+        got, _ = gdb.bc(ctx, g, gt, sources, gdb.Opts.make())
+        bc_close(got, want)
+    want = oracle.dijkstra_tb(row, col, w, n - 1)
+    got, _ = gdb.sssp_worklist(ctx, g, n - 1, gdb.Opts.make(wgs=64, groups=2))
+    assert (got.astype(np.int64) == want).all()
+    want, _ = oracle.sssp_pull_ref(row, col, w, n - 1)
+    got, _ = gdb.sssp_pull(ctx, g, n - 1, gdb.Opts.make())
+    assert (got == want).all()
