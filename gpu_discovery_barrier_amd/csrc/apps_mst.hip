@@ -29,7 +29,7 @@
 // pieces of kLongRow edges spread over all waves (a skewed graph's longest row
 // has as many edges as a thousand others); a vertex or piece without a cross
 // edge never gets one again and is left out of later rounds.  R-MAT 18 (7.6 M
-// edges, longest row 25 k): 0.60 ms (one lane walking each row twice per
+// edges, longest row 25 k): 0.58 ms (one lane walking each row twice per
 // round, six barriers: 46.4 ms; vertices 64 at a time: 0.93).  Walking the rows of a wave as one list, with
 // the minima in LDS, took 1.07 ms: the search for each edge's row costs more
 // than the steps it saves.
