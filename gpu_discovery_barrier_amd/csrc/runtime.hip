@@ -214,6 +214,9 @@ int launch_groups(gdb_ctx* ctx, const void* kernel, const gdb_opts* opts, long l
   }
   long long need = (work_items + wgs - 1) / wgs;
   if (need < 1) need = 1;
+  // A restricted launch needs a group on every XCD (they are dealt round-robin), or
+  // a small graph's few groups may all run elsewhere and nobody solves it.
+  if (ctx->xcd_active >= 0 && need < ctx->xcds) need = ctx->xcds;
   if (g > need) g = (int)need;
   if (g > GDB_MAX_GROUPS) g = GDB_MAX_GROUPS;
   if (g < 1) g = 1;
@@ -320,6 +323,7 @@ bool apply_tuning(const char* solver, long long n, gdb_opts* o, int* team_groups
 
 static int init_ctx(gdb_ctx* ctx, int skip) {
   ctx->skip = skip;
+  ctx->xcd_active = ctx->xcd_only;
   const int nlines = (int)(sizeof(gdb_kernel_ctx_t) / GDB_LINE_BYTES);
   hipLaunchKernelGGL(gdb_k_init_ctx, dim3((nlines + 255) / 256), dim3(256), 0, ctx->stream, ctx->d,
                      skip, ctx->lock_kind, ctx->bar_kind, (int)ctx->quiet_ticks,

@@ -15,6 +15,7 @@ struct gdb_ctx {
   int lock_kind = GDB_LOCK_FREE;
   int bar_kind = GDB_BAR_AUTO;
   int xcd_only = -1;
+  int xcd_active = -1;  // xcd_only as of the last init: what the device words hold
   int skip = 0;
   unsigned timeout_ticks = 1000000000u;  // 10 s at 100 MHz
   unsigned quiet_ticks = 2000u;          // 20 us
@@ -28,7 +29,7 @@ struct gdb_ctx {
   // scratch array (gdb_sssp_worklist_noalloc); resolved at context creation.
   void* noalloc_scratch = nullptr;
   // Pinned host words: [0, 8) stop-flag readbacks of the relaunch schedule, then
-  // what finish_launch collects (GDB_COLLECT_WORDS).
+  // what finish_launch collects (from kCollectBase on).
   int* h_flag = nullptr;
   // Grow-only pinned host buffer that uploads go through (a batch's task table).
   void* h_stage = nullptr;

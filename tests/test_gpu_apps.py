@@ -591,3 +591,39 @@ def test_rows_walked_by_part_of_a_wave(ctx, deg, hubs):
     want, _ = oracle.sssp_pull_ref(row, col, w, n - 1)
     got, _ = gdb.sssp_pull(ctx, g, n - 1, gdb.Opts.make())
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("xcd", [0, 3, 7])
+@pytest.mark.parametrize("side", [(4, 5), (40, 50), (50, 64)])
+@pytest.mark.parametrize("solver", ["bfs", "sssp", "pull", "mis", "mst", "bc"])
+def test_small_graphs_on_one_xcd(ctx, solver, side, xcd):
+    """Graphs of fewer groups than there are XCDs, on a context restricted to one."""
+    g = gdb.gen_grid(*side, 0.0, seed=1, wlo=1, whi=9)
+    d = gdb.DeviceCSR(g)
+    o = gdb.Opts.make(wgs=0, variant=gdb.VARIANT_TUNED)
+    nv = (gdb.permutation(g.n, 2).astype(np.float64) / (g.n + 1)).astype(np.float32)
+    src = np.array([0, g.n // 2], np.int32)
+    out = gdb.DeviceBuffer.from_numpy(np.full(g.n, -77, np.float32 if solver == "bc" else np.int32))
+    ctx.set_xcd_only(xcd)
+    try:
+        if solver == "mst":
+            weight, edges, components, _ = gdb.mst(ctx, d, o)
+        elif solver == "bc":
+            got, _ = gdb.bc(ctx, d, d, src, o, out=out)
+        elif solver == "mis":
+            got, _ = gdb.mis(ctx, d, gdb.DeviceBuffer.from_numpy(nv), o, out=out)
+        else:
+            fn = {"bfs": gdb.bfs_worklist, "sssp": gdb.sssp_worklist, "pull": gdb.sssp_pull}[solver]
+            got, _ = fn(ctx, d, 0, o, out=out)
+    finally:
+        ctx.set_xcd_only(-1)
+    if solver == "mst":
+        assert (weight, edges, components) == (oracle.mst_kruskal(g.row, g.col, g.w)[0], g.n - 1, 1)
+    elif solver == "bc":
+        bc_close(got, oracle.bc_brandes_tb(g.row, g.col, src))
+    else:
+        want = {"bfs": lambda: oracle.bfs_tb(g.row, g.col, 0),
+                "sssp": lambda: oracle.dijkstra_tb(g.row, g.col, g.w, 0),
+                "pull": lambda: oracle.sssp_pull_ref(g.row, g.col, g.w, 0)[0],
+                "mis": lambda: oracle.mis_ref(g.row, g.col, nv)[0]}[solver]()
+        assert (got.astype(np.int64) == np.asarray(want).astype(np.int64)).all()
