@@ -392,7 +392,7 @@ __global__ __launch_bounds__(WGS) void k_color_tuned(gdb_kernel_ctx_t* ctx, cons
 // R-MAT 14 (213 k blocking edges, 294 rounds): 0.52 ms against 6.5 with rounds;
 // the 400^2 grid with index-ordered values (799 rounds): 0.95 against 17.
 constexpr int kFlowK = 4;
-enum FlowWord { FW_ROUNDS = 0, FW_GAVE_UP, FW_INVALID, FW_WORDS };
+enum FlowWord { FW_ROUNDS = 0, FW_GAVE_UP, FW_INVALID, FW_DONE, FW_WORDS };  // FW_DONE: groups that finished
 
 __device__ __forceinline__ bool colourable(float x) { return x > -1.f; }
 
@@ -525,6 +525,8 @@ __global__ __launch_bounds__(WGS) void k_color_flow(gdb_kernel_ctx_t* ctx, const
     if (gdb::wave_any(moved)) t_last = gdb::now();
     else if (flow_stuck(fw, it, t_last, limit)) break;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) gdb::fadd_rlx(&fw[FW_DONE], 1);
 }
 
 // Colours and round count of a finished k_color_flow.  A wave takes `per` vertices:
@@ -700,7 +702,10 @@ __global__ __launch_bounds__(1024) void k_color_flow1(gdb_kernel_ctx_t* ctx, con
   if (gdb::lane_id() == 0 && r > 0) atomicMax(&s_rounds, r);
   for (int i = threadIdx.x; i < n; i += 1024) color[i] = c[i] ? c[i] : -1;
   __syncthreads();
-  if (threadIdx.x == 0) fw[FW_ROUNDS] = s_rounds;
+  if (threadIdx.x == 0) {
+    fw[FW_ROUNDS] = s_rounds;
+    fw[FW_DONE] = 1;
+  }
 }
 
 // ---- relaunch schedule: color (color_kernel.cl:80-123) and color2 (134-154)
@@ -765,9 +770,11 @@ using namespace gdbrt;
 
 namespace {
 
-// Launches the round-free kernels.  *done: the colouring is finished and s
-// filled in; otherwise (a shape that cannot hold the edges, too few
-// participants, ties) the caller runs the round-based kernel.
+// Launches the round-free kernels.  *done: every window's group reported that it
+// finished, the colouring is complete and s filled in; otherwise (a shape that
+// cannot hold the edges, too few participants, ties) the caller runs the
+// round-based kernel.  So it does on a context restricted to one XCD: the launch
+// has just the groups that the windows need, which run on all of them.
 //
 // The rule: one group when the graph fits its LDS and the caller left the
 // shape open; else as many groups as cover the edges, if the caller's launch
@@ -779,6 +786,7 @@ namespace {
 int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const float* nv, int* color,
                const gdb_opts& asked, gdb_stats* s, bool* done) {
   *done = false;
+  if (ctx->xcd_active >= 0) return GDB_SUCCESS;
   const bool open = asked.wgs == 0;
   gdb_opts o = asked;
   if (open) o.wgs = kFlowWgs;
@@ -795,6 +803,7 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
   int* poll = cv.take<int>((size_t)n + 1);
   int* gmx = cv.take<int>(n);
   int* gcnt = cv.take<int>(n);
+  int windows = 1;
   if (one) {
     const size_t lds = flow1_lds(n);
     if (lds > 49152)
@@ -832,6 +841,7 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
                          poll, color, fw);
       GDB_HIP(hipGetLastError());
       ran = true;
+      windows = nwin;
       s->launches = 3;
       return finish_launch(ctx, &s->kernel_ms, fw, FW_WORDS);
     });
@@ -841,7 +851,8 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
   rc = collected_error(ctx);
   if (rc) return rc;
   if (h[FW_INVALID]) return GDB_E_INVALID;
-  if (h[FW_GAVE_UP] || h[FW_ROUNDS] == INT_MAX) return GDB_SUCCESS;  // INT_MAX: neighbours that are never coloured
+  if (h[FW_DONE] != windows || h[FW_GAVE_UP]) return GDB_SUCCESS;
+  if (h[FW_ROUNDS] == INT_MAX) return GDB_SUCCESS;  // neighbours that are never coloured
   s->participating = collected_participating(ctx);
   s->rounds = h[FW_ROUNDS] + 1;
   *done = true;

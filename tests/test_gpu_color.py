@@ -176,6 +176,32 @@ def test_color_flow_ties_then_clean(ctx, n):
     assert (got == want).all() and st.rounds == rr
 
 
+@pytest.mark.parametrize("xcd", [1, 7])
+@pytest.mark.parametrize("wgs", [0, 1024])
+@pytest.mark.parametrize("shape", ["rmat10", "grid", "pairs"])
+def test_color_on_one_xcd_of_any_shape(ctx, shape, wgs, xcd):
+    """A restricted context, the shape left open or a group size given: graphs whose
+    edges fit fewer groups than there are XCDs, so that a launch of just those groups
+    may have none on the chosen one."""
+    if shape == "pairs":  # rows of one edge, whose blockers do not count
+        n = 20000
+        row, col = np.arange(n + 1, dtype=np.int32), (np.arange(n) ^ 1).astype(np.int32)
+    else:
+        g = gdb.gen_rmat(10, 16, seed=1) if shape == "rmat10" else gdb.gen_grid(100, 90, 0.05, seed=3)
+        n, row, col = g.n, np.asarray(g.row), np.asarray(g.col)
+    nv = (gdb.permutation(n, 2).astype(np.float64) / (n + 1)).astype(np.float32)
+    want, rounds = oracle.color_ref(row, col, nv)
+    d = gdb.DeviceCSR(gdb.CSR(n, row, col, np.ones_like(col)), weights=False)
+    out = gdb.DeviceBuffer.from_numpy(np.full(n, -77, np.int32))
+    ctx.set_xcd_only(xcd)
+    try:
+        got, st = gdb.color(ctx, d, gdb.DeviceBuffer.from_numpy(nv),
+                            gdb.Opts.make(wgs=wgs, variant=gdb.VARIANT_TUNED), out=out)
+    finally:
+        ctx.set_xcd_only(-1)
+    assert (got == want).all() and st.rounds == rounds
+
+
 # ---------------------------------------------------------------- max-min colouring
 @pytest.mark.parametrize("wgs,groups", [(64, 3), (256, 0), (1024, 16)])
 @pytest.mark.parametrize("graph", ["rmat14", "grid", "gnp", "hubs"])
