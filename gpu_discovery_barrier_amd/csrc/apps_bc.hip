@@ -498,8 +498,12 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     }
     __syncthreads();
   };
+  auto list_long = [&](int v, unsigned mask, int b, int e) {
+    s_long[atomicAdd(&s_nlong, 1)] = make_int4(v, (int)mask, b, e);
+  };
   // Long rows found in this trip; `done(v, mask)` is called by every thread with
-  // a row's sums in s_part[0].
+  // a row's sums in s_part[0].  The last barrier keeps the next trip's rows from
+  // a wave that has yet to read this trip's count, and from its reset.
   auto long_rows = [&](auto& step, auto done) {
     __syncthreads();
     const int nl = s_nlong;
@@ -510,6 +514,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
       __syncthreads();
     }
     if (nl > 0 && threadIdx.x == 0) s_nlong = 0;
+    __syncthreads();
   };
   unsigned char* const mark = (unsigned char*)marks;  // a byte per vertex and source
   int* const edge_counts = tail + 12;                 // edges of the next step's vertices, rotating
@@ -668,7 +673,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
               return acc;
         };
         const bool own = valid && mask != 0 && e - b <= kLongRowM;
-        if (valid && mask != 0 && !own) s_long[atomicAdd(&s_nlong, 1)] = make_int4(v, (int)mask, b, e);
+        if (valid && mask != 0 && !own) list_long(v, mask, b, e);
         const FV sgm = gdb::wave_walk_np<kSlotsM>(own, b, e, (int)mask, fv_zero(), step,
                                                   [](FV a, FV c) { return fv_add(a, c); }, kSerialLimit);
         if (own && t > 0) {
@@ -791,7 +796,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
               return a;
         };
         const bool own = valid && mask != 0 && e - b <= kLongRowM;
-        if (valid && mask != 0 && !own) s_long[atomicAdd(&s_nlong, 1)] = make_int4(v, (int)mask, b, e);
+        if (valid && mask != 0 && !own) list_long(v, mask, b, e);
         const FV acc = gdb::wave_walk_np<kSlotsM>(own, b, e, (int)mask, fv_zero(), step,
                                                   [](FV x, FV c) { return fv_add(x, c); }, kSerialLimit);
         if (own) {

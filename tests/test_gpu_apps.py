@@ -627,3 +627,32 @@ def test_small_graphs_on_one_xcd(ctx, solver, side, xcd):
                 "pull": lambda: oracle.sssp_pull_ref(g.row, g.col, g.w, 0)[0],
                 "mis": lambda: oracle.mis_ref(g.row, g.col, nv)[0]}[solver]()
         assert (got.astype(np.int64) == np.asarray(want).astype(np.int64)).all()
+
+
+@pytest.mark.parametrize("wgs,groups", [(64, 1), (128, 2), (512, 1), (0, 0)])
+def test_bc_rows_walked_by_a_group_in_many_trips(ctx, wgs, groups):
+    """Long rows in every few of the trips that a group makes through a level, in the
+    forward and in the backward pass."""
+    hubs, leaves = 60, 4200
+    rng = np.random.default_rng(3)
+    # A source that reaches 3000 vertices on one level, hubs spread among them;
+    # each hub has the same leaves on the next one.
+    first = 1 + rng.permutation(3000)
+    a = [np.zeros(3000, np.int64), rng.integers(1, 3001, 9000)]
+    b = [np.arange(1, 3001), rng.integers(1, 3001, 9000)]
+    n = 3001 + leaves
+    for h in first[:hubs]:
+        a.append(np.full(leaves, h))
+        b.append(np.arange(3001, n))
+    a, b = np.concatenate(a), np.concatenate(b)
+    key = np.unique(np.concatenate([a * n + b, b * n + a]))
+    key = key[key // n != key % n]
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(key // n, minlength=n))
+    col = (key % n).astype(np.int32)
+    assert (np.diff(row) > 4096).sum() == hubs
+    sources = np.concatenate([[0], rng.permutation(n)[:10]]).astype(np.int32)
+    want = oracle.bc_brandes_mt(row, col, sources)
+    d = dev(row, col)
+    got, _ = gdb.bc(ctx, d, d, sources, gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED))
+    bc_close(got, want)
