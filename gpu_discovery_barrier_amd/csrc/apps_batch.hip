@@ -102,6 +102,15 @@ constexpr int kLocalQDefault = 2048;
 constexpr int kLocalQMin = 256, kLocalQMax = 4096;
 constexpr int kMaxHops = 4096;  // local-step budget limit per team iteration
 
+// When a level-synchronous iteration looks at a target's distance before it claims
+// it (relax_n).  The look is one more dependent trip, and saves atomics.  Rows
+// walked by a wave always look: 600 vertices of 300 edges, BFS 0.63 -> 0.25 ms and
+// SSSP 2.8 -> 1.5, R-MAT 14 2.7 -> 1.9 and 9.6 -> 8.1.  Short rows look where the
+// atomics of many groups meet (1024 graphs: 17.1 -> 15.4 ms), in iterations of more
+// than a few vertices; else the trip is what counts (three BFS tasks of a 5000-vertex
+// path 11.9 ms against 13.6 with the look, of a 100^2 grid 0.62 against 0.70).
+constexpr int kCrowdedGroups = 64, kCheckItems = 32;
+
 struct Team {
   gdb_kernel_ctx_t* ctx;
   gdb_local_ctx* l;
@@ -111,6 +120,7 @@ struct Team {
   int* lq;             // LDS: two local queue buffers of qcap ints each
   int qcap;
   int* lcnt;           // LDS: three rotating local queue counters
+  bool crowded;        // many groups at work: the chip's atomics are what they wait for
   __device__ int word_off(int w) const { return w * kLine; }
   __device__ int* word(int w) const { return ts + w * kLine; }
   __device__ int tid() const { return rank * (int)blockDim.x + (int)threadIdx.x; }
@@ -563,31 +573,34 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
       // atomic (min with all ones, max with INT_MIN) to this thread's spare
       // word, a valid vertex that spreads such atomics over many lines.
       const int spare = (int)(((unsigned)blockIdx.x * blockDim.x + threadIdx.x) % (unsigned)n);
-      auto relax_n = [&](const bool (&ok)[kChunk], const int (&kk)[kChunk], unsigned src_d,
-                         int (&dst)[kChunk], int (&cls)[kChunk]) {
+      // `check`: most edges improve nothing, and a load of the target's
+      // distance comes first, atomics only from lanes that it lets through (a
+      // stale one is never below the current, so it can only let too many).
+      auto relax_n = [&](const auto& ok, const auto& kk, unsigned src_d, auto& dst, auto& cls, bool check) {
+        constexpr int N = (int)(sizeof(ok) / sizeof(ok[0]));
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
+        for (int j = 0; j < N; ++j) {
           dst[j] = -1;
           cls[j] = 0;
         }
         bool any = false;
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) any |= ok[j];
+        for (int j = 0; j < N; ++j) any |= ok[j];
         // Lanes without a slot this step stay out (no memory traffic); inside
         // the branch every result is consumed before it closes.
         if (!any) return;
-        unsigned wt[kChunk];
-        bool act[kChunk];
-        unsigned cand[kChunk];
-        int at[kChunk];
+        unsigned wt[N];
+        bool act[N];
+        unsigned cand[N];
+        int at[N];
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
+        for (int j = 0; j < N; ++j) {
           const int e = ok[j] ? kk[j] : 0;
           dst[j] = gdb::ldg(k.col + e);
           wt[j] = (!WEIGHTED || UNIT) ? 1u : (unsigned)gdb::ldg(k.w + e);
         }
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
+        for (int j = 0; j < N; ++j) {
           act[j] = ok[j] && (unsigned)dst[j] < (unsigned)n && wt[j] < kInf;
           if (!ok[j]) dst[j] = -1;
           at[j] = act[j] ? dst[j] : spare;
@@ -595,64 +608,64 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
           cls[j] = 0;
         }
         if constexpr (!WEIGHTED) {
-          // Most targets are reached already: a load first, and claims only from
-          // lanes that saw an unreached one (a stale load can only let a
-          // needless claim through).  A slot without one compares against
-          // all ones, which no distance is.
-          unsigned old[kChunk];
-          bool any_need = false;
+          // A slot without an unreached target compares against all ones,
+          // which no distance is.
+          unsigned old[N];
+          if (check) {
+            bool any_need = false;
 #pragma unroll
-          for (int j = 0; j < kChunk; ++j) old[j] = gdb::ldg(&dist[at[j]]);
+            for (int j = 0; j < N; ++j) old[j] = gdb::ldg(&dist[at[j]]);
 #pragma unroll
-          for (int j = 0; j < kChunk; ++j) {
-            act[j] = act[j] && old[j] == kInf;
-            any_need |= act[j];
+            for (int j = 0; j < N; ++j) {
+              act[j] = act[j] && old[j] == kInf;
+              any_need |= act[j];
+            }
+            if (!any_need) return;
           }
-          if (!any_need) return;
 #pragma unroll
-          for (int j = 0; j < kChunk; ++j)
+          for (int j = 0; j < N; ++j)
             old[j] = gdb::atomic_cas_g(&dist[act[j] ? dst[j] : spare], act[j] ? kInf : ~0u, act[j] ? src_d : ~0u);
 #pragma unroll
-          for (int j = 0; j < kChunk; ++j) cls[j] = (act[j] && old[j] == kInf) ? 1 : 0;
+          for (int j = 0; j < N; ++j) cls[j] = (act[j] && old[j] == kInf) ? 1 : 0;
         } else {
-          bool imp[kChunk], nearp[kChunk];
-          if (hops > 0) {
+          bool imp[N], nearp[N];
+          if (UNIT || hops > 0) {
             // The mark word stays 0 with local hops, so a 32-bit atomic on
             // the distance word does (a 64-bit one has a third of the
             // throughput).
-            unsigned old[kChunk];
+            unsigned old[N];
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j)
+            for (int j = 0; j < N; ++j)
               old[j] = gdb::atomic_min_g(reinterpret_cast<unsigned*>(&d64[at[j]]) + 1, act[j] ? cand[j] : ~0u);
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) {
+            for (int j = 0; j < N; ++j) {
               imp[j] = act[j] && cand[j] < old[j];
               nearp[j] = cand[j] < thresh;
               if (imp[j] && nearp[j]) cls[j] = 3;
             }
           } else {
-            // As in the BFS: the distance word first, then the 64-bit minima
-            // from lanes with a candidate below it.
-            unsigned cur[kChunk];
-            bool any_need = false;
+            if (check) {  // the distance word
+              unsigned cur[N];
+              bool any_need = false;
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) cur[j] = gdb::ldg(reinterpret_cast<unsigned*>(&d64[at[j]]) + 1);
+              for (int j = 0; j < N; ++j) cur[j] = gdb::ldg(reinterpret_cast<unsigned*>(&d64[at[j]]) + 1);
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) {
-              act[j] = act[j] && cand[j] < cur[j];
-              any_need |= act[j];
+              for (int j = 0; j < N; ++j) {
+                act[j] = act[j] && cand[j] < cur[j];
+                any_need |= act[j];
+              }
+              if (!any_need) return;
             }
-            if (!any_need) return;
-            unsigned long long old[kChunk];
+            unsigned long long old[N];
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) {
+            for (int j = 0; j < N; ++j) {
               nearp[j] = cand[j] < thresh;
               const unsigned long long nw =
                   ((unsigned long long)cand[j] << 32) | (nearp[j] ? near_mark : far_mark);
               old[j] = gdb::atomic_min_g(&d64[act[j] ? dst[j] : spare], act[j] ? nw : ~0ull);
             }
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) {
+            for (int j = 0; j < N; ++j) {
               imp[j] = act[j] && cand[j] < (unsigned)(old[j] >> 32);
               if (imp[j] && nearp[j]) cls[j] = (unsigned)old[j] == near_mark ? 0 : 1;
             }
@@ -662,28 +675,29 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
           // it (stamps only grow, and none exceeds gen while relaxing).
           bool far_any = false;
 #pragma unroll
-          for (int j = 0; j < kChunk; ++j) far_any |= imp[j] && !nearp[j];
+          for (int j = 0; j < N; ++j) far_any |= imp[j] && !nearp[j];
           if (far_any) {
-            int fs[kChunk];
+            int fs[N];
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j) {
+            for (int j = 0; j < N; ++j) {
               const bool f = imp[j] && !nearp[j];
               fs[j] = gdb::atomic_max_g(&fstamp[f ? dst[j] : spare], f ? gen : INT_MIN);
             }
 #pragma unroll
-            for (int j = 0; j < kChunk; ++j)
+            for (int j = 0; j < N; ++j)
               if (imp[j] && !nearp[j]) cls[j] = fs[j] < gen ? 2 : 0;
           }
         }
       };
       // Pushes the results of one relaxation step of this wave.  Class 3
       // goes to LDS buffer `lb` when there is room, else to the team queue.
-      auto push_n = [&](const int (&dst)[kChunk], const int (&cls)[kChunk], int lb, int* lc) {
-        bool to_team[kChunk], to_far[kChunk];
-        unsigned long long m3[kChunk];
+      auto push_n = [&](const auto& dst, const auto& cls, int lb, int* lc) {
+        constexpr int N = (int)(sizeof(dst) / sizeof(dst[0]));
+        bool to_team[N], to_far[N];
+        unsigned long long m3[N];
         int n3 = 0;
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
+        for (int j = 0; j < N; ++j) {
           to_team[j] = cls[j] == 1;
           to_far[j] = cls[j] == 2;
           m3[j] = __ballot(cls[j] == 3);
@@ -695,7 +709,7 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
           pos = gdb::bcast(pos, 0);
           const unsigned long long lt = (1ull << gdb::lane_id()) - 1ull;
 #pragma unroll
-          for (int j = 0; j < kChunk; ++j) {
+          for (int j = 0; j < N; ++j) {
             if (cls[j] == 3) {
               const int at = pos + __popcll(m3[j] & lt);
               if (at < qcap) lq[lb * qcap + at] = dst[j];
@@ -704,8 +718,8 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
             pos += __popcll(m3[j]);
           }
         }
-        gdb::wave_push_n<kChunk>(to_team, dst, outq, out_tail);
-        if (near_far) gdb::wave_push_n<kChunk>(to_far, dst, fpile, ftail);
+        gdb::wave_push_n<N>(to_team, dst, outq, out_tail);
+        if (near_far) gdb::wave_push_n<N>(to_far, dst, fpile, ftail);
       };
       // Relaxes the out-edges of items[start, count) with stride `step`.
       auto process = [&](const int* src_items, int count, int start, int step, int lb, int* lc) {
@@ -736,21 +750,19 @@ __device__ __forceinline__ int team_worklist(Team& T, const DevTask& k, unsigned
               ok[j] = c + j < len;
               kk[j] = b + c + j;
             }
-            relax_n(ok, kk, dv, dst, cls);
+            relax_n(ok, kk, dv, dst, cls, T.crowded && nin > kCheckItems);
             push_n(dst, cls, lb, lc);
           }
-          // Heavy rows: the whole wave walks one row, 64 edges per step.
+          // Heavy rows: the whole wave walks one row, 64 edges per step, a slot a
+          // lane (unused slots would send their no-op atomics: SSSP with local hops on
+          // 600 vertices of 300 edges 4.6 ms with three of them, 2.6 without).
           gdb::wave_coop_foreach(
               heavy, b, e, dv,
               [&](int e, bool ok, unsigned src_d) {
-                bool oks[kChunk];
-                int kk[kChunk], dst[kChunk], cls[kChunk];
-#pragma unroll
-                for (int j = 0; j < kChunk; ++j) {
-                  oks[j] = j == 0 && ok;
-                  kk[j] = e;
-                }
-                relax_n(oks, kk, src_d, dst, cls);
+                const bool oks[1] = {ok};
+                const int kk[1] = {e};
+                int dst[1], cls[1];
+                relax_n(oks, kk, src_d, dst, cls, true);
                 push_n(dst, cls, lb, lc);
               },
               -1);
@@ -1908,7 +1920,8 @@ __global__ __launch_bounds__(WGS) __attribute__((amdgpu_waves_per_eu(WGS == 512 
   const bool mlp = SEL && sel.mode == GDB_SEL_MLP && sel.w;
   if (mlp)
     for (int i = threadIdx.x; i < gdbsel::kParams; i += blockDim.x) sel_w[i] = sel.w[i];
-  Team T{ctx, &local_ctx, team_state + (size_t)team * TW_WORDS * kLine, &gen_cache, G, id % G, lq, qcap, lcnt};
+  Team T{ctx, &local_ctx, team_state + (size_t)team * TW_WORDS * kLine, &gen_cache, G, id % G, lq, qcap, lcnt,
+         min(nteams, ntasks) * G >= kCrowdedGroups};
   if (id == 0 && threadIdx.x == 0) *teams_used = nteams;
   int Gn = sel.narrow_groups > 0 ? sel.narrow_groups : 1;
   if (Gn > G) Gn = G;
@@ -1944,7 +1957,8 @@ __global__ __launch_bounds__(WGS) __attribute__((amdgpu_waves_per_eu(WGS == 512 
       else if (k.algo == GDB_TASK_BFS)
         rounds = k.hops > 0 ? team_worklist<true, true, false>(T, k, wk, R)
                             : team_worklist<false, false, SEL>(T, k, wk, R);
-      else if (k.algo == GDB_TASK_SSSP) rounds = team_worklist<true, false, SEL>(T, k, wk, R);
+      else if (k.algo == GDB_TASK_SSSP)
+        rounds = team_worklist<true, false, SEL>(T, k, wk, R);
       else {
         if (T.G == 1 && color_queue_lds(k.n) <= (size_t)region) rounds = team_color_queue(T, k);
         if (rounds == 0) rounds = team_color(T, k);
