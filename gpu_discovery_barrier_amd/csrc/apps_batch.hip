@@ -2003,7 +2003,8 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
   if (!ctx || ntasks <= 0 || !tasks || team_groups < 0) return GDB_E_INVALID;
   gdb_opts o{};
   if (opts) o = *opts;
-  bool open_shape = false;  // the launch shape is the table's "batch" row
+  bool open_shape = false;  // the launch shape, group count and all, is the table's "batch" row
+  const bool groups_given = o.groups > 0;
   {
     // A batch with an owner-partitioned task takes the "batch_owned" row
     // when the table has one (one group per CU), else the "batch" row.
@@ -2014,7 +2015,7 @@ int plan_batch(gdb_ctx* ctx, const gdb_task* tasks, int ntasks, int team_groups,
       any_owned |= tasks[t].owned != 0;
     }
     if (!any_owned || !apply_tuning("batch_owned", nmax, &o, &team_groups))
-      open_shape = apply_tuning("batch", nmax, &o, &team_groups) && !any_owned;
+      open_shape = apply_tuning("batch", nmax, &o, &team_groups) && !any_owned && !groups_given;
   }
   P->ctx = ctx;
   P->ntasks = ntasks;

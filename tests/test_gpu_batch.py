@@ -300,3 +300,17 @@ def test_batch_colour_queue(ctx, wgs, groups, team):
     for (name, g, nv, out), r in zip(outs, rounds):
         want, rr = oracle.color_ref(g.row, g.col, nv)
         assert (out.to_numpy() == want).all() and r == rr, (name, r, rr)
+
+
+@pytest.mark.parametrize("groups", [257, 512])
+def test_batch_open_group_size_keeps_a_given_group_count(ctx, groups):
+    """wgs = 0 takes the group size from the table; the count stays the caller's, also
+    where the engine would rather have one group per CU."""
+    gs = [gdb.gen_grid(30, 30, 0.0, seed=i, wlo=1, whi=9) for i in range(4)]
+    ds = [gdb.DeviceCSR(g) for g in gs]
+    outs = [gdb.DeviceBuffer.empty(g.n, np.uint32) for g in gs]
+    tasks = [gdb.make_task(gdb.TASK_BFS, d, o, source=0) for d, o in zip(ds, outs)]
+    _, st = gdb.batch_solve(ctx, tasks, 1, gdb.Opts.make(wgs=0, groups=groups))
+    assert st.participating == groups
+    for g, o in zip(gs, outs):
+        assert (o.to_numpy() == oracle.bfs_tb(g.row, g.col, 0)).all()
