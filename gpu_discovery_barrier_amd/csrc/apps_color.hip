@@ -777,16 +777,17 @@ namespace {
 // has just the groups that the windows need, which run on all of them.
 //
 // The rule: one group when the graph fits its LDS and the caller left the
-// shape open; else as many groups as cover the edges, if the caller's launch
-// or, with the shape open, one 1024-thread group per CU does (1 M edges).
-// Beyond that the polls bound it: every pending edge reads a device word again
-// and again, and those of a skewed graph's hubs meet in a few L2 lines.  R-MAT
-// 15 (0.88 M edges) 0.57 ms against 8.5 with rounds; R-MAT 17 at 16 edges a
-// lane 94 ms against 45.
+// shape open; else as many groups as cover the edges, if the launch has them and
+// there are no more edges than one 1024-thread group per CU holds (1 M).  Beyond
+// that, whatever the group size, the polls bound it: every pending edge reads a
+// device word again and again, and those of a skewed graph's hubs meet in a few
+// L2 lines.  R-MAT 15 (0.88 M edges) 0.57 ms against 8.5 with rounds, 0.95 against
+// 9.1 with 256-thread groups; R-MAT 16 (1.8 M) 164 against 27, G(230000) of degree
+// 8 (1.8 M) 28 to 500 against 3; R-MAT 17 at 16 edges a lane 94 against 45.
 int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const float* nv, int* color,
                const gdb_opts& asked, gdb_stats* s, bool* done) {
   *done = false;
-  if (ctx->xcd_active >= 0) return GDB_SUCCESS;
+  if (ctx->xcd_active >= 0 || m > ctx->num_cus * kFlowWgs * kFlowK) return GDB_SUCCESS;
   const bool open = asked.wgs == 0;
   gdb_opts o = asked;
   if (open) o.wgs = kFlowWgs;
@@ -828,7 +829,7 @@ int color_flow(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const
       int groups = 0;
       int r = launch_groups(ctx, kern, &o, (long long)GDB_MAX_GROUPS * WG, &groups, lds);
       if (r) return r;
-      if (nwin > (open ? std::min(groups, ctx->num_cus) : groups)) return GDB_SUCCESS;
+      if (nwin > groups) return GDB_SUCCESS;
       r = prepare_launch(ctx, fw, FW_WORDS);
       if (!r) r = timer_start(ctx);
       if (r) return r;

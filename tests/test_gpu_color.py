@@ -202,6 +202,23 @@ def test_color_on_one_xcd_of_any_shape(ctx, shape, wgs, xcd):
     assert (got == want).all() and st.rounds == rounds
 
 
+@pytest.mark.parametrize("wgs,groups", [(64, 0), (256, 0), (256, 2048), (1024, 0)])
+@pytest.mark.parametrize("rows", [513, 514])
+def test_color_flow_edge_limit(ctx, rows, wgs, groups):
+    """1 M edges (a group of 1024 threads per CU, four edges a lane) end the round-free
+    kernel's range for every launch shape; it meets no barrier, the other does."""
+    g = gdb.gen_grid(rows, 512, 0.0, seed=1)
+    below = g.m <= 256 * 1024 * 4
+    assert below == (rows == 513)
+    nv = (gdb.permutation(g.n, 2).astype(np.float64) / (g.n + 1)).astype(np.float32)
+    d = gdb.DeviceCSR(g, weights=False)
+    want, rounds = oracle.color_ref(g.row, g.col, nv)
+    got, st = gdb.color(ctx, d, gdb.DeviceBuffer.from_numpy(nv),
+                        gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED))
+    assert (got == want).all() and st.rounds == rounds
+    assert (st.barriers == 0) == (below and (groups or 4096) * wgs * 4 >= g.m)
+
+
 # ---------------------------------------------------------------- max-min colouring
 @pytest.mark.parametrize("wgs,groups", [(64, 3), (256, 0), (1024, 16)])
 @pytest.mark.parametrize("graph", ["rmat14", "grid", "gnp", "hubs"])
