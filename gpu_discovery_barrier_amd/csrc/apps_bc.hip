@@ -504,7 +504,9 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
   // Long rows found in this trip; `done(v, mask)` is called by every thread with
   // a row's sums in s_part[0].  The last barrier keeps the next trip's rows from
   // a wave that has yet to read this trip's count, and from its reset.
+  bool has_long = false, even = false;
   auto long_rows = [&](auto& step, auto done) {
+    if (!has_long) return;
     __syncthreads();
     const int nl = s_nlong;
     for (int l = 0; l < nl; ++l) {
@@ -520,10 +522,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
   int* const edge_counts = tail + 12;                 // edges of the next step's vertices, rotating
   const int sweep_from = gdb::sweep_line(n);
   const bool may_sweep = row[n] > sweep_from;
-  auto flush = [&](int above) {
-    if (may_sweep) gdb::stage_edges(stage, above, row, &s_deg);
-    gdb::group_flush(stage, above, q, tail);
-  };
+  auto flush = [&](int above) { gdb::group_flush(stage, above, q, tail, may_sweep ? row : nullptr, &s_deg); };
   int nbar = 0, levels = 0;
   auto reset = [&](int v) {
 #pragma unroll
@@ -534,11 +533,16 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     code[v] = 0u;
     stamp[v] = -1;
   };
+  int* const any_long = tail + 15;  // 1: some row has more than kEvenRow edges, 2: more than kLongRowM
+  int longest = 0;
   for (int i = tid; i < n; i += stride) {
     bc[i] = 0.f;
     marks[i] = 0ull;
     reset(i);
+    longest = max(longest, row[i + 1] - row[i]);
   }
+  longest = gdb::wave_max(longest);
+  if (longest > gdb::kEvenRow && lane == 0) gdb::atomic_max_g(any_long, longest > kLongRowM ? 2 : 1);
   int prev_reached = 0;
   for (int s0 = 0; s0 < nsrc; s0 += kMS) {
     const int ns = nsrc - s0 < kMS ? nsrc - s0 : kMS;
@@ -567,17 +571,21 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     }
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
+    has_long = gdb::ld_rlx(any_long) == 2;
+    even = gdb::even_rows(n, row[n], gdb::ld_rlx(any_long) != 0);
     const unsigned all = ns >= 32 ? ~0u : (1u << ns) - 1u;
     // Forward.
     int lb = 0, le = gdb::ld_rlx(tail), t = 0;
     int ne = 0;  // the sources' own edges: a step of eight vertices claims
     for (;;) {
       const bool sweep = may_sweep && ne > sweep_from;
+      const bool direct = !sweep && gdb::push_directly(even, le - lb);  // its edges are not counted: no sweep follows
       int* const out_edges = &edge_counts[(t + 1) % 3];
       if (tid == 0) gdb::st_rlx(&edge_counts[(t + 2) % 3], 0);
       const unsigned par = (unsigned)(t - 1) & 3u;                    // parents' level mod 4
       const unsigned nxt_nib = 8u | ((unsigned)(t + 1) & 3u);         // a claimed nibble
-      GDB_FOR_SPREAD(i, valid, tid, stride, le - lb, 0) {
+      long long left = le - lb;
+      GDB_FOR_SPREAD(i, valid, tid, stride, le - lb, gdb::spread_queue(even, le - lb)) {
         int v = -1, b = 0, e = 0;
         unsigned mask = 0;
         if (valid) {
@@ -669,7 +677,8 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
                   }
                 }
               }
-              if (!sweep) gdb::wave_stage_n<kSlotsM>(stage, push, w, q, tail);
+              if (direct) gdb::wave_push_n<kSlotsM>(push, w, q, tail);
+              else if (!sweep) gdb::wave_stage_n<kSlotsM>(stage, push, w, q, tail);
               return acc;
         };
         const bool own = valid && mask != 0 && e - b <= kLongRowM;
@@ -685,7 +694,8 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
           const int s = (int)threadIdx.x;
           if (s < kMS && t > 0 && ((lm >> s) & 1u)) *rec_int(sg, lv, s) = __float_as_int(s_part[0][s]);
         });
-        flush(kStage / 2);
+        left -= stride;
+        if (left > 0) flush(kStage / 2);
       }
       if (sweep) {
         if (!discovery_barrier(ctx, &local_ctx)) return;
@@ -720,10 +730,10 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
               if ((got >> (4 * s)) & 1u) *rec_int(lev, v[j], s) = t + 1;
           }
           gdb::wave_stage_n<kV>(stage, push, v, q, tail);
-          flush(kStage / 2);
+          if (p0 + (long long)kV * stride < n) flush(kStage / 2);
         }
       }
-      flush(0);
+      if (!direct) flush(0);
       if (may_sweep && threadIdx.x == 0 && s_deg) {
         gdb::fadd_rlx(out_edges, s_deg);
         s_deg = 0;
@@ -748,7 +758,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi(gdb_kernel_ctx_t* ctx, const i
     for (int tt = t; tt >= 0; --tt) {
       const int qb = tt == t ? lb : loff[tt];
       const int qe = tt == t ? le : loff[tt + 1];
-      GDB_FOR_SPREAD(i, valid, tid, stride, qe - qb, 0) {
+      GDB_FOR_SPREAD(i, valid, tid, stride, qe - qb, gdb::spread_queue(even, qe - qb)) {
         int v = -1, b = 0, e = 0;
         unsigned mask = 0;
         Half sv;
@@ -890,10 +900,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
   int* const edge_counts = tail + 12;  // edges of the next step's vertices, rotating
   const int sweep_from = gdb::sweep_line(n);
   const bool may_sweep = row[n] > sweep_from;
-  auto flush = [&](int above) {
-    if (may_sweep) gdb::stage_edges(stage, above, row, &s_deg);
-    gdb::group_flush(stage, above, q, tail);
-  };
+  auto flush = [&](int above) { gdb::group_flush(stage, above, q, tail, may_sweep ? row : nullptr, &s_deg); };
   int nbar = 0, levels = 0;
   auto reset = [&](int v) {
 #pragma unroll
@@ -979,6 +986,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
         if (tid == 0) *deep = 1;
         return;
       }
+      long long left = le - lb;
       GDB_FOR_SPREAD(i, valid, tid, stride, le - lb, 0) {
         int v = -1, b = 0, e = 0, bt = 0, et = 0;
         unsigned mask = 0;
@@ -1057,7 +1065,8 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
           for (int s = 0; s < kMS; ++s)
             if ((mask >> s) & 1u) *rec_int(sg, v, s) = __float_as_int(sgm.v[s]);
         }
-        flush(kStage / 2);
+        left -= stride;
+        if (left > 0) flush(kStage / 2);
       }
       if (sweep) {
         if (!discovery_barrier(ctx, &local_ctx)) return;
@@ -1077,7 +1086,7 @@ __global__ __launch_bounds__(WGS) void k_bc_multi_directed(gdb_kernel_ctx_t* ctx
 #pragma unroll
           for (int j = 0; j < kV; ++j) push[j] = push[j] && bytes_equal(c[j], (unsigned)t + 2u) != 0ull;
           gdb::wave_stage_n<kV>(stage, push, v, q, tail);
-          flush(kStage / 2);
+          if (p0 + (long long)kV * stride < n) flush(kStage / 2);
         }
       }
       flush(0);

@@ -180,7 +180,8 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
                                                   const int* __restrict__ col,
                                                   const int* __restrict__ w, unsigned* dist,
                                                   int* stamp, int* q0, int* q1, int* tails, int n,
-                                                  int4* pieces, int piece_cap, long long* work, int* out) {
+                                                  int4* pieces, int piece_cap, const int* long_row,
+                                                  long long* work, int* out) {
   DISCOVERY_PROTOCOL(ctx);
   constexpr int kStage = 8 * WGS;  // pushes of this group awaiting queue space
   __shared__ int s_q[kStage], s_n, s_base, s_deg;
@@ -193,11 +194,11 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
   int* const edge_counts = tails + 12;  // BFS: edges of the queued vertices, rotating too
   unsigned char* const mark = (unsigned char*)stamp;  // BFS: a byte per vertex, set once it is reached
   const int sweep_from = gdb::sweep_line(n);
-  const bool may_sweep = !WEIGHTED && n > 0 && row[n] > sweep_from;
+  const bool may_sweep = !WEIGHTED && row[n] > sweep_from;
+  const bool even = gdb::even_rows(n, row[n], *long_row != 0);
   // Moves staged vertices to the queue; BFS adds up their edges.
   auto flush = [&](int above, int* queue, int* tail) {
-    if (may_sweep) gdb::stage_edges(stage, above, row, &s_deg);
-    gdb::group_flush(stage, above, queue, tail);
+    gdb::group_flush(stage, above, queue, tail, may_sweep ? row : nullptr, &s_deg);
   };
   int iteration = 1, nbar = 0;
   long long items = 0, edges = 0;
@@ -216,6 +217,7 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
     int* npieces = &piece_counts[iteration % 3];
     int* out_edges = &edge_counts[(iteration + 1) % 3];
     const bool sweep = may_sweep && ne > sweep_from;
+    const bool direct = !sweep && gdb::push_directly(even, nin);  // its edges are not counted: no sweep follows
     if (tid == 0) {
       gdb::st_rlx(&tails[(iteration + 2) % 3], 0);
       gdb::st_rlx(&piece_counts[(iteration + 1) % 3], 0);
@@ -302,11 +304,13 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
         }
       }
-      if (!sweep) gdb::wave_stage_n<kChunk>(stage, push, dst, outq, out_tail);
+      if (direct) gdb::wave_push_n<kChunk>(push, dst, outq, out_tail);
+      else if (!sweep) gdb::wave_stage_n<kChunk>(stage, push, dst, outq, out_tail);
       return 0;
     };
     auto any = [](int a, int c) { return a | c; };
-    GDB_FOR_SPREAD(i, valid, tid, threads, nin, 0) {
+    long long left = nin;
+    GDB_FOR_SPREAD(i, valid, tid, threads, nin, gdb::spread_queue(even, nin)) {
       int v = -1, b = 0, e = 0;
       unsigned dv = 0;
       if (valid) {
@@ -327,13 +331,17 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
         }
       }
       gdb::wave_walk_np<kChunk>(valid != 0, b, e, (int)dv, 0, step, any, kSerialLimit);
-      flush(kStage / 2, outq, out_tail);
+      left -= threads;
+      if (left > 0) flush(kStage / 2, outq, out_tail);
     }
-    flush(0, outq, out_tail);
+    if (!direct) flush(0, outq, out_tail);
     flush_edges();
     if (!discovery_barrier(ctx, &local_ctx)) return;
     ++nbar;
-    const int np = min(gdb::ld_rlx(npieces), piece_cap);
+    // The words that say what comes next, in one trip: usually the next iteration.
+    const int pieces_out = gdb::ld_rlx(npieces), queued = gdb::ld_rlx(out_tail);
+    const int queued_edges = may_sweep ? gdb::ld_rlx(out_edges) : 0;
+    const int np = min(pieces_out, piece_cap);
     if (np > 0) {
       for (int p0 = 0; p0 < np; p0 += nwaves) {  // the same trips in every wave
         const int p = p0 + wave;
@@ -348,9 +356,9 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           }
           step(ok, kk, pc.z);
         }
-        flush(kStage / 2, outq, out_tail);
+        if (!direct && p0 + nwaves < np) flush(kStage / 2, outq, out_tail);
       }
-      flush(0, outq, out_tail);
+      if (!direct) flush(0, outq, out_tail);
       flush_edges();
       if (!discovery_barrier(ctx, &local_ctx)) return;
       ++nbar;
@@ -374,15 +382,19 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
           if (push[j]) dist[v[j]] = (unsigned)iteration;
         }
         gdb::wave_stage_n<kChunk>(stage, push, v, outq, out_tail);
-        flush(kStage / 2, outq, out_tail);
+        if (p0 + (long long)kChunk * threads < n) flush(kStage / 2, outq, out_tail);
       }
       flush(0, outq, out_tail);
       flush_edges();
       if (!discovery_barrier(ctx, &local_ctx)) return;
       ++nbar;
     }
-    if (may_sweep) ne = gdb::ld_rlx(out_edges);
-    nin = gdb::ld_rlx(out_tail);
+    nin = queued;
+    ne = queued_edges;
+    if (np > 0 || sweep) {
+      nin = gdb::ld_rlx(out_tail);
+      if (may_sweep) ne = gdb::ld_rlx(out_edges);
+    }
     ++iteration;
   }
   // Edges examined, summed over threads (one atomic per wave).
@@ -442,8 +454,11 @@ __global__ void k_wl_step(const int* __restrict__ row, const int* __restrict__ c
   }
 }
 
-__global__ void k_wl_init(unsigned* dist, int* stamp, int* q0, int* q1, int* flags, int n, int src, bool bytes) {
+// *long_row (0 before): whether a row has more than kEvenRow edges.
+__global__ void k_wl_init(const int* __restrict__ row, unsigned* dist, int* stamp, int* q0, int* q1, int* flags,
+                          int* long_row, int n, int src, bool bytes) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && row[i + 1] - row[i] > gdb::kEvenRow) *long_row = 1;
   if (i < n) {  // initialize (bfs_common.cl:64-71) + dist[source] = 0
     dist[i] = i == src ? 0u : kInf;
     stamp[i] = bytes && i == src >> 2 ? 1 << 8 * (src & 3) : 0;  // bytes: the source is marked
@@ -609,7 +624,14 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
     return GDB_E_INVALID;
   gdb_opts o{};
   if (opts) o = *opts;
-  if (o.variant == GDB_VARIANT_TUNED && o.schedule == GDB_SCHED_PERSISTENT) gdbrt::apply_tuning(WEIGHTED ? "sssp_wl" : "bfs_wl", n, &o);
+  if (o.variant == GDB_VARIANT_TUNED && o.schedule == GDB_SCHED_PERSISTENT) {
+    // A sparse graph's BFS that solve_if_local declines may have a thousand short
+    // iterations: a row of its own, with fewer groups to meet in each (a shuffled 500^2
+    // grid: 6.6 ms with 128 groups, 5.2 with 64, 4.3 with 32; G(400000) of degree 4 0.27,
+    // 0.27 and 0.32).
+    if (WEIGHTED || (long long)m > (long long)kLocalDegree * n || !gdbrt::apply_tuning("bfs_wl_sparse", n, &o))
+      gdbrt::apply_tuning(WEIGHTED ? "sssp_wl" : "bfs_wl", n, &o);
+  }
   const int wgs = default_wgs(&o);
   gdb_stats st{};
   if (n == 0) {
@@ -629,7 +651,7 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   const bool tuned_wl = o.variant == GDB_VARIANT_TUNED && o.schedule != GDB_SCHED_RELAUNCH;
   // A row longer than kLongRow has at most 2 * edges / kLongRow pieces.
   int piece_cap = tuned_wl ? (int)(2LL * m / kLongRow) + 1 : 0;
-  size_t bytes = carve_bytes<int>(n) * 3 + carve_bytes<int>(32) + carve_bytes<long long>(2);
+  size_t bytes = carve_bytes<int>(n) * 3 + carve_bytes<int>(32) + carve_bytes<long long>(3);
   if (fixed_ws) {  // the list takes what the caller's buffer has left
     if (bytes > fixed_bytes) return GDB_E_SCRATCH;
     piece_cap = (int)std::min<size_t>(piece_cap, (fixed_bytes - bytes) / sizeof(int4) & ~(size_t)15);
@@ -649,14 +671,15 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   int* q0 = cv.take<int>(n);
   int* q1 = cv.take<int>(n);
   int* flags = cv.take<int>(32);
-  long long* work = cv.take<long long>(2);
+  long long* work = cv.take<long long>(3);
   int4* pieces = cv.take<int4>(piece_cap);
   int* tails = flags + 4;
   int* out = flags + 12;
-  rc = prepare_launch(ctx, (int*)work, 4);
+  int* long_row = (int*)(work + 2);
+  rc = prepare_launch(ctx, (int*)work, 5);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, dist, stamp, q0, q1,
-                     flags, n, source, !WEIGHTED);
+  hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, row, dist, stamp, q0, q1,
+                     flags, long_row, n, source, !WEIGHTED);
   GDB_HIP(hipGetLastError());
 
   if (o.schedule == GDB_SCHED_RELAUNCH) {
@@ -700,7 +723,7 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
       if (tuned)
         hipLaunchKernelGGL((k_wl_tuned<WG, WEIGHTED>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
                            row, col, w, dist, stamp, q0, q1, tails, n, pieces, piece_cap,
-                           work, out);
+                           long_row, work, out);
       else
         hipLaunchKernelGGL((k_wl_plain<WG, WEIGHTED>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
                            row, col, w, dist, stamp, q0, q1, flags, n, out);

@@ -213,7 +213,8 @@ __device__ __forceinline__ void wave_push_n(const bool (&push)[N], const int (&i
 // space for a batch of them at once.  wave_stage_n appends the items of N push
 // slots of every lane to the stage (what does not fit goes straight to the
 // queue); group_flush, called by all threads of the group, moves the staged items
-// to the queue when more than `above` wait.
+// to the queue when more than `above` wait.  It holds two to three barriers of the
+// group: a loop calls it between its trips, and once at its end.
 struct PushStage {
   int* items;  // LDS, `cap` entries
   int* count;  // LDS, zeroed before the first use
@@ -248,16 +249,27 @@ __device__ __forceinline__ void wave_stage_n(const PushStage& st, bool (&push)[N
   }
   if (full) wave_push_n<N>(push, item, queue, tail);
 }
-__device__ __forceinline__ void group_flush(const PushStage& st, int above, int* queue, int* tail) {
+// With `row`, the edges of the moved vertices are added to *sum (LDS) while the
+// queue's reply is on its way.
+__device__ __forceinline__ void group_flush(const PushStage& st, int above, int* queue, int* tail, const int* row,
+                                            int* sum) {
   __syncthreads();
   const int c = *st.count < st.cap ? *st.count : st.cap;
-  __syncthreads();
-  if (c <= above) return;
-  if (threadIdx.x == 0) {
-    *st.base = fadd_rlx(tail, c);
-    *st.count = 0;
+  if (c <= above) {
+    __syncthreads();  // every wave has read the count before the next push
+    return;
   }
+  int at = 0;
+  if (threadIdx.x == 0) at = fadd_rlx(tail, c);
+  if (row) {
+    int d = 0;
+    for (int i = threadIdx.x; i < c; i += blockDim.x) d += row[st.items[i] + 1] - row[st.items[i]];
+    for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
+    if (lane_id() == 0 && d) atomicAdd(sum, d);
+  }
+  if (threadIdx.x == 0) *st.base = at;
   __syncthreads();
+  if (threadIdx.x == 0) *st.count = 0;
   for (int i = threadIdx.x; i < c; i += blockDim.x) queue[*st.base + i] = st.items[i];
   __syncthreads();
 }
@@ -270,18 +282,6 @@ __device__ __forceinline__ void group_flush(const PushStage& st, int above, int*
 // per vertex, about 10 us and n / 0.5 ns.  (Lines from 50000 + n / 8 to 400000 + n /
 // 12 measured within 3% of each other in BFS and BC.)
 __host__ __device__ inline int sweep_line(int n) { return 100000 + n / 16; }
-
-// Adds the edges of the staged vertices that group_flush(st, above, ...) is about
-// to move to *sum (LDS).  Called by all threads, right before it.
-__device__ __forceinline__ void stage_edges(const PushStage& st, int above, const int* row, int* sum) {
-  __syncthreads();
-  const int c = *st.count < st.cap ? *st.count : st.cap;
-  if (c <= above) return;
-  int d = 0;
-  for (int i = threadIdx.x; i < c; i += blockDim.x) d += row[st.items[i] + 1] - row[st.items[i]];
-  for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
-  if (lane_id() == 0 && d) atomicAdd(sum, d);
-}
 
 // Wave-wide OR of a predicate.
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0ull; }
@@ -482,5 +482,18 @@ __device__ __forceinline__ long long spread_item(int start, int stride, int sh) 
 // measured 2 to 25% slower on R-MAT graphs), 64 together where they are short
 // (2^20-vertex grid MST 1.16 ms against 1.44).
 __host__ __device__ inline int spread_rows(int n, long long m) { return m >= 8LL * n ? 0 : 6; }
+// The same for a step over `items` queued vertices.  Where all rows are short (`even`:
+// eight edges a vertex at most, none of more than kEvenRow) a wave takes 16 neighbours,
+// and 64 in a step of up to 256: the fewer groups have work, the fewer come late to
+// the barrier.  One by one against this: BFS of a 100^2 grid of shuffled ids 0.84 -> 0.76
+// ms, BC of it, 11 sources, 6.6 -> 5.8; 64 always: SSSP of a 500^2 one 7.9 -> 13.4.
+constexpr int kEvenRow = 64;
+__host__ __device__ inline bool even_rows(int n, long long m, bool long_row) { return m < 8LL * n && !long_row; }
+__host__ __device__ inline int spread_queue(bool even, int items) { return !even ? 0 : items <= 256 ? 6 : 4; }
+// Whether such a step pushes straight to the queue.  Its pushes are few, and the
+// barriers of the group that staging takes (group_flush) cost more than their atomics:
+// BFS of a shuffled 500^2 grid 5.0 -> 4.3 ms (512 items: 4.8), of a 100^2 grid 0.75 ->
+// 0.70; BC of the 300^2 grid 10.8 -> 10.3.
+__host__ __device__ inline bool push_directly(bool even, int items) { return even && items <= 1024; }
 
 }  // namespace gdb

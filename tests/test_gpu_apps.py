@@ -656,3 +656,39 @@ def test_bc_rows_walked_by_a_group_in_many_trips(ctx, wgs, groups):
     d = dev(row, col)
     got, _ = gdb.bc(ctx, d, d, sources, gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED))
     bc_close(got, want)
+
+
+@pytest.mark.parametrize("wgs,groups", [(0, 0), (64, 5), (512, 32)])
+@pytest.mark.parametrize("directed", [False, True])
+def test_steps_of_a_sparse_graph(ctx, directed, wgs, groups):
+    """Levels either side of 256 and 1024 vertices, where a sparse graph's steps change
+    how they deal and push vertices, then one whose edges make the next step sweep."""
+    rng = np.random.default_rng(8)
+    sizes = [1, 16, 256, 257, 1024, 1025, 60000]
+    first = np.concatenate([[0], np.cumsum(sizes)])
+    a, b = [], []
+    for lv in range(1, len(sizes)):
+        v = np.repeat(np.arange(first[lv], first[lv + 1]), 3)
+        a.append(rng.integers(first[lv - 1], first[lv], v.size))
+        b.append(v)
+    a, b, n = np.concatenate(a), np.concatenate(b), int(first[-1])
+    key = np.unique(a * n + b if directed else np.concatenate([a * n + b, b * n + a]))
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(key // n, minlength=n))
+    col = (key % n).astype(np.int32)
+    w = rng.integers(1, 60, col.size).astype(np.int32)
+    assert 100000 + n // 16 < col.size < 6 * n
+    g = dev(row, col, w)
+    o = gdb.Opts.make(wgs=wgs, groups=groups, variant=gdb.VARIANT_TUNED)
+    for source in (0, 20):
+        want, rounds = oracle.bfs_worklist_ref(row, col, source)
+        got, st = gdb.bfs_worklist(ctx, g, source, o)
+        assert (got == want).all() and st.rounds == rounds
+        got, _ = gdb.sssp_worklist(ctx, g, source, o)
+        assert (got.astype(np.int64) == oracle.dijkstra_tb(row, col, w, source)).all()
+    sources = np.array([0, 20, 3, 700, 2000, 1, 500, 9, 30000], np.int32)
+    gt = gdb.DeviceCSR(gdb.CSR(n, row, col, w).transpose()) if directed else g
+    want = oracle.bc_brandes_mt(row, col, sources)
+    for count in (1, sources.size):
+        got, _ = gdb.bc(ctx, g, gt, sources[:count], o)
+        bc_close(got, want if count > 1 else oracle.bc_brandes_mt(row, col, sources[:1]))
