@@ -274,7 +274,7 @@ __global__ __launch_bounds__(WGS) void k_color_tuned(gdb_kernel_ctx_t* ctx, cons
       };
       auto red = [](gdb::MaxAt a, gdb::MaxAt c) { return (c.at >= 0 && (a.at < 0 || c.mx > a.mx)) ? c : a; };
       const gdb::MaxAt res =
-          gdb::wave_walk_n<kSlots>(active && !deg1 && !blocked, b, e, gdb::MaxAt{-1.f, -1}, step, red, kHeavyDeg);
+          gdb::wave_walk_n<kSlots, true>(active && !deg1 && !blocked, b, e, gdb::MaxAt{-1.f, -1}, step, red, kHeavyDeg);
       if (active) {
         if (blocked) {
           md_cur[v] = mp;  // the maximum of the previous round stands

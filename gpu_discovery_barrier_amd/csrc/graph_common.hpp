@@ -312,8 +312,10 @@ __device__ __forceinline__ bool any_slot(const bool (&ok)[N]) {
 // range is walked depends on its length alone, and so does the order of its sum.
 // As wave_walk_n, but step(ok, kk, owner) also gets the `payload` of the
 // range's owner lane (for a long row walked by the whole wave, the leader's
-// payload on every lane).
-template <int N, typename T, typename Step, typename R>
+// payload on every lane).  SHORT: the caller's ranges are all short, and the long
+// walks' code and registers stay out (colouring by rounds, R-MAT 19: 305 ms, 323 with
+// them).
+template <int N, bool SHORT = false, typename T, typename Step, typename R>
 __device__ __forceinline__ T wave_walk_np(bool active, int b, int e, int payload, T identity, Step step, R red,
                                           int serial_limit) {
   const bool heavy = active && (e - b) > serial_limit;
@@ -330,6 +332,7 @@ __device__ __forceinline__ T wave_walk_np(bool active, int b, int e, int payload
     }
     acc = red(acc, step(ok, kk, payload));
   }
+  if constexpr (SHORT) return acc;
   const int lane = lane_id();
   const bool mid = heavy && (e - b) <= 16 * N;
   unsigned long long mask = __ballot(mid);
@@ -439,10 +442,10 @@ __device__ __forceinline__ bool wave_walk_any(bool active, int b, int e, int pay
   return found;
 }
 
-template <int N, typename T, typename Step, typename R>
+template <int N, bool SHORT = false, typename T, typename Step, typename R>
 __device__ __forceinline__ T wave_walk_n(bool active, int b, int e, T identity, Step step, R red,
                                          int serial_limit) {
-  return wave_walk_np<N>(
+  return wave_walk_np<N, SHORT>(
       active, b, e, 0, identity, [&](const bool (&ok)[N], const int (&kk)[N], int) { return step(ok, kk); }, red,
       serial_limit);
 }
