@@ -472,6 +472,7 @@ __device__ __forceinline__ T wave_walk_n(bool active, int b, int e, T identity, 
 // order gained nothing).  SH = 6 keeps a wave's 64 items together: short rows,
 // whose words it then reads in one line.
 __device__ __forceinline__ long long spread_item(int start, int stride, int sh) {
+  if (sh == 6) return start;  // what the rest comes to, without its division
   const unsigned waves = (unsigned)stride >> 6, l = (unsigned)lane_id(), share = l >> sh;
   const unsigned turn = (waves * 5u / 8u) | 1u;
   return (((long long)share * waves + ((unsigned)start / 64u + share * turn) % waves) << sh) + (l & ((1u << sh) - 1u));
