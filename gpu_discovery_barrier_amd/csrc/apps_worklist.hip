@@ -511,7 +511,9 @@ __global__ __launch_bounds__(256) void k_locality(const int* __restrict__ row, c
     const int v = (int)((long long)i * n / count);
     const int b = row[v], e = min(row[v + 1], b + kSampleEdges);
     for (int k = b; k < e; ++k) {
-      const int d = abs(col[k] - v);
+      const int u = col[k];
+      if ((unsigned)u >= (unsigned)n) continue;  // as the solvers, which skip such an edge
+      const int d = abs(u - v);
       atomicAdd(&s_hist[d == 0 ? 0 : 32 - __clz(d)], 1);
       ++edges;
       if (w) ws += min((unsigned)w[k], kInf);

@@ -692,3 +692,28 @@ def test_steps_of_a_sparse_graph(ctx, directed, wgs, groups):
     for count in (1, sources.size):
         got, _ = gdb.bc(ctx, g, gt, sources[:count], o)
         bc_close(got, want if count > 1 else oracle.bc_brandes_mt(row, col, sources[:1]))
+
+
+@pytest.mark.parametrize("wgs", [0, 256])
+def test_worklist_skips_columns_out_of_range(ctx, wgs):
+    """Columns that are no vertex are passed over, also where the graph is sampled."""
+    n = 3000
+    a = np.repeat(np.arange(n), 3)
+    b = np.stack([(np.arange(n) + 1) % n, np.maximum(np.arange(n) - 1, 0), np.arange(n)], 1).ravel()
+    col = b.astype(np.int32)
+    col[2::30] = -2**31
+    col[5::30] = 2**31 - 1
+    col[8::30] = -1
+    col[11::30] = n
+    row = np.arange(0, 3 * n + 1, 3, dtype=np.int32)
+    w = (1 + np.arange(3 * n) % 50).astype(np.int32)
+    keep = (col >= 0) & (col < n)
+    krow = np.concatenate([[0], np.cumsum(np.bincount(a[keep], minlength=n))]).astype(np.int32)
+    g = dev(row, b.astype(np.int32), w)
+    g.col = gdb.DeviceBuffer.from_numpy(col)  # what a caller of the C ABI may pass
+    o = gdb.Opts.make(wgs=wgs, variant=gdb.VARIANT_TUNED)
+    for source in (0, n - 1):
+        got, _ = gdb.bfs_worklist(ctx, g, source, o)
+        assert (got == oracle.bfs_tb(krow, col[keep], source)).all()
+        got, _ = gdb.sssp_worklist(ctx, g, source, o)
+        assert (got.astype(np.int64) == oracle.dijkstra_tb(krow, col[keep], w[keep], source)).all()
