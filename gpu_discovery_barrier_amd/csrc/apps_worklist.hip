@@ -561,7 +561,7 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
                    unsigned* dist, gdb_stats* st, bool* done) {
   using namespace gdbrt;
   *done = false;
-  if (ctx->xcd_only >= 0 || (long long)m > (long long)kLocalDegree * n || m < n / 2) return GDB_SUCCESS;
+  if (ctx->xcd_active >= 0 || (long long)m > (long long)kLocalDegree * n || m < n / 2) return GDB_SUCCESS;
   int rc = ensure_workspace(ctx, sizeof(Locality));
   if (rc) return rc;
   Locality* d = (Locality*)ctx->ws;
@@ -598,7 +598,12 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
   o.groups = G;
   o.barrier = -1;
   rc = gdb_batch_solve(ctx, &t, 1, G, &o, st);
+  // A range without work waits for the others as long as the solve takes, a queue
+  // iteration's barrier never that long: under a short wait bound the queues may
+  // still finish.  (The context has been reset.)
+  if (rc == GDB_E_TIMEOUT) return GDB_SUCCESS;
   if (rc) return rc;
+  if (t.rounds == 0) return GDB_SUCCESS;  // no group took part
   if (!WEIGHTED) {
     int* levels = (int*)ctx->ws;
     rc = prepare_launch(ctx, levels, 1);

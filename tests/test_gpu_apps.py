@@ -717,3 +717,22 @@ def test_worklist_skips_columns_out_of_range(ctx, wgs):
         assert (got == oracle.bfs_tb(krow, col[keep], source)).all()
         got, _ = gdb.sssp_worklist(ctx, g, source, o)
         assert (got.astype(np.int64) == oracle.dijkstra_tb(krow, col[keep], w[keep], source)).all()
+
+
+@pytest.mark.parametrize("solver", ["bfs", "sssp"])
+def test_worklist_local_graph_under_a_short_wait_bound(ctx, solver):
+    """A bound that every iteration's barrier meets with ease, but that a range of the
+    owner-partitioned solve, waiting for the first vertex to reach it, does not."""
+    g = gdb.gen_grid(1024, 1024, 0.05, seed=2, wlo=1, whi=255)
+    d = gdb.DeviceCSR(g)
+    fn = gdb.bfs_worklist if solver == "bfs" else gdb.sssp_worklist
+    want, _ = fn(ctx, d, 0, gdb.Opts.make(wgs=256, groups=64, variant=gdb.VARIANT_TUNED))
+    ctx.set_timeouts(700.0, 20.0)
+    try:
+        for _ in range(2):  # the bound given up on leaves nothing behind
+            got, _ = fn(ctx, d, 0, gdb.Opts.make(wgs=0, variant=gdb.VARIANT_TUNED))
+            assert (got == want).all()
+    finally:
+        ctx.set_timeouts(10e6, 20.0)
+    got, _ = fn(ctx, d, 0, gdb.Opts.make(wgs=0, variant=gdb.VARIANT_TUNED))
+    assert (got == want).all()
