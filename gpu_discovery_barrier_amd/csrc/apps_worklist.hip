@@ -496,7 +496,8 @@ struct Locality {
   int pad;
   unsigned long long wsum;
 };
-constexpr int kSampleVertices = 8192, kSampleEdges = 4;  // evenly spaced vertices, edges of each
+constexpr int kSampleVertices = 8192, kSampleEdges = 8;  // evenly spaced vertices, edges of each (a row's
+                                                         // long ones may be its last)
 
 __global__ __launch_bounds__(256) void k_locality(const int* __restrict__ row, const int* __restrict__ col,
                                                   const int* __restrict__ w, int n, Locality* out) {
@@ -547,13 +548,18 @@ __global__ void k_levels(const unsigned* __restrict__ dist, int n, int* out) {
 //
 // The rule: at most kLocalDegree edges per vertex (denser graphs, the sample's
 // cost not spent on them, are skewed or random in use, and a slot record holds
-// four edges), and 98% of the sampled edges shorter than half a range.  Ranges
+// four edges), and 99.5% of the sampled edges (SSSP: 98.5%) shorter than half a range:
+// more long ones cut the iterations short and leave the ranges crossing each
+// other (grids of 128^2 to 1024^2 with 0.5, 1 and 1.8% of random edges, against the
+// queues: BFS .93 to .67, 1.38 to .90 and 1.54 to 1.23 of the time, SSSP .74 to
+// .37, 1.08 to .61 and 1.23 to .73).  Ranges
 // of kLocalRange vertices, one group each (1024^2 grid: 64 ranges 4.63 ms,
 // 128 4.92, 256 6.0; 128^2: 1 to 8 within 10%), at most one per CU.  SSSP
 // bands of 96 mean weights (24 to 200 measured, within 15%).  1024^2 grid:
 // SSSP 33.4 ms with iteration queues, 4.7 here; BFS 13.7 and 2.7; a 64^2 grid
 // 0.57 and 0.20, 0.46 and 0.15.
 constexpr int kLocalDegree = 6, kLocalRange = 12288, kLocalBand = 96;
+constexpr int kLocalNearBfs = 995, kLocalNearSssp = 985;  // of a thousand edges
 constexpr int kLocalRangeMax = 30000;  // distances, marks, queues and boundary list of a range fit a CU's LDS
 
 template <bool WEIGHTED>
@@ -581,7 +587,8 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
   const int range = (n + G - 1) / G;
   long long near = 0;
   for (int b = 0; b < 31 && (1LL << b) <= range / 2; ++b) near += h.hist[b];
-  if (near * 100 < 98LL * h.edges || range > kLocalRangeMax) return GDB_SUCCESS;
+  if (near * 1000 < (WEIGHTED ? kLocalNearSssp : kLocalNearBfs) * (long long)h.edges || range > kLocalRangeMax)
+    return GDB_SUCCESS;
   gdb_task t{};
   t.algo = WEIGHTED ? GDB_TASK_SSSP : GDB_TASK_BFS;
   t.n = n;

@@ -736,3 +736,24 @@ def test_worklist_local_graph_under_a_short_wait_bound(ctx, solver):
         ctx.set_timeouts(10e6, 20.0)
     got, _ = fn(ctx, d, 0, gdb.Opts.make(wgs=0, variant=gdb.VARIANT_TUNED))
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("long_per_mille", [4, 8, 12, 25])
+def test_worklist_local_graph_with_long_edges(ctx, long_per_mille):
+    """Either side of the shares of long edges up to which BFS and SSSP take the
+    owner-partitioned solve (which meets no inter-group barrier)."""
+    rng = np.random.default_rng(long_per_mille)
+    g = gdb.gen_grid(300, 300, 0.05, seed=2, wlo=1, whi=255)
+    src, dst = np.repeat(np.arange(g.n), np.diff(g.row)), np.asarray(g.col, np.int64)
+    k = g.m * long_per_mille // 2000
+    a = rng.integers(0, g.n, k)
+    b = (a + g.n // 2) % g.n
+    src, dst = np.concatenate([src, a, b]), np.concatenate([dst, b, a])
+    row, col, w = csr_directed(g.n, src, dst, rng, 255)
+    d = dev(row, col, w)
+    o = gdb.Opts.make(wgs=0, variant=gdb.VARIANT_TUNED)
+    got, st = gdb.bfs_worklist(ctx, d, 5, o)
+    assert (got == oracle.bfs_tb(row, col, 5)).all() and (st.barriers == 0) == (long_per_mille < 6)
+    got, st = gdb.sssp_worklist(ctx, d, 5, o)
+    assert (got.astype(np.int64) == oracle.dijkstra_tb(row, col, w, 5)).all()
+    assert (st.barriers == 0) == (long_per_mille < 15)
