@@ -1320,9 +1320,11 @@ extern "C" int gdb_bc(gdb_ctx* ctx, int n, int m, const int* row, const int* col
     st.launches = 1;
     if (multi_directed && collected_words(ctx)[2] && collected_error(ctx) == GDB_SUCCESS) {
       multi_directed = false;
+      const double tried_ms = st.kernel_ms;
       rc = prepare_launch(ctx, flags, 32);
       if (!rc) rc = solve();
       if (rc) return rc;
+      st.kernel_ms += tried_ms;
       st.launches = 2;
     }
     st.rounds = collected_words(ctx)[0];

@@ -888,8 +888,8 @@ extern "C" int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* 
       if (stats) *stats = s;
       return GDB_SUCCESS;
     }
-    s = gdb_stats{};
   }
+  const gdb_stats tried = s;  // what the attempt took
   // Tuned schedule: rows longer than kHeavyDeg are split into chunks of
   // kChunkEdges edges; the rows and the (row, first edge) of every chunk
   // are listed here from the row offsets.
@@ -991,7 +991,8 @@ extern "C" int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* 
       return finish_launch(ctx, &s.kernel_ms, out, 2);
     });
     if (rc) return rc;
-    s.launches = 1;
+    s.kernel_ms += tried.kernel_ms;
+    s.launches = 1 + tried.launches;
     s.rounds = collected_words(ctx)[0];
     s.barriers = collected_words(ctx)[1];
     s.participating = collected_participating(ctx);

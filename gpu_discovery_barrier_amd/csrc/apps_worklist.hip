@@ -544,7 +544,8 @@ __global__ void k_levels(const unsigned* __restrict__ dist, int n, int* out) {
 // Solves a sparse local graph (grids, meshes, road networks) by the batched
 // engine's owner-partitioned ranges: such a graph has thousands of short
 // iterations, and there a hop inside a range costs an LDS round instead of
-// an inter-group barrier.  *done is false when the graph is none.
+// an inter-group barrier.  *done is false when the graph is none; st then holds the
+// device time and launches of finding out.
 //
 // The rule: at most kLocalDegree edges per vertex (denser graphs, the sample's
 // cost not spent on them, are skewed or random in use, and a slot record holds
@@ -579,8 +580,11 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
                      WEIGHTED ? w : nullptr, n, d);
   GDB_HIP(hipGetLastError());
   Locality h;
-  rc = finish_launch(ctx, nullptr, d, kWords);
+  double ms = 0;
+  rc = finish_launch(ctx, &ms, d, kWords);
   if (rc) return rc;
+  st->kernel_ms += ms;
+  ++st->launches;
   memcpy(&h, collected_words(ctx), sizeof(h));
   if (h.edges == 0) return GDB_SUCCESS;
   const int G = std::max(1, std::min(ctx->num_cus, (n + kLocalRange - 1) / kLocalRange));
@@ -604,13 +608,20 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
   o.wgs = 1024;
   o.groups = G;
   o.barrier = -1;
-  rc = gdb_batch_solve(ctx, &t, 1, G, &o, st);
+  gdb_stats solve{};
+  rc = gdb_batch_solve(ctx, &t, 1, G, &o, &solve);
   // A range without work waits for the others as long as the solve takes, a queue
   // iteration's barrier never that long: under a short wait bound the queues may
   // still finish.  (The context has been reset.)
-  if (rc == GDB_E_TIMEOUT) return GDB_SUCCESS;
+  solve.kernel_ms += st->kernel_ms;
+  solve.launches += st->launches;
+  if (rc == GDB_E_TIMEOUT || t.rounds == 0) {  // or no group took part
+    st->kernel_ms = solve.kernel_ms;
+    st->launches = solve.launches;
+    return rc == GDB_E_TIMEOUT ? GDB_SUCCESS : rc;
+  }
+  *st = solve;
   if (rc) return rc;
-  if (t.rounds == 0) return GDB_SUCCESS;  // no group took part
   if (!WEIGHTED) {
     int* levels = (int*)ctx->ws;
     rc = prepare_launch(ctx, levels, 1);
@@ -618,8 +629,10 @@ int solve_if_local(gdb_ctx* ctx, int n, int m, const int* row, const int* col, c
     if (rc) return rc;
     hipLaunchKernelGGL(k_levels, dim3(std::min(256, (n + 255) / 256)), dim3(256), 0, ctx->stream, dist, n, levels);
     GDB_HIP(hipGetLastError());
-    rc = finish_launch(ctx, nullptr, levels, 1);
+    rc = finish_launch(ctx, &ms, levels, 1);
     if (rc) return rc;
+    st->kernel_ms += ms;
+    ++st->launches;
     st->rounds = collected_words(ctx)[0];
   }
   *done = true;
@@ -660,8 +673,8 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
       if (stats) *stats = st;
       return lrc;
     }
-    st = gdb_stats{};
   }
+  const gdb_stats tried = st;  // what the attempt took
   const bool tuned_wl = o.variant == GDB_VARIANT_TUNED && o.schedule != GDB_SCHED_RELAUNCH;
   // A row longer than kLongRow has at most 2 * edges / kLongRow pieces.
   int piece_cap = tuned_wl ? (int)(2LL * m / kLongRow) + 1 : 0;
@@ -745,7 +758,8 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
       return finish_launch(ctx, &st.kernel_ms, flags, nwords);
     });
     if (rc) return rc;
-    st.launches = 1;
+    st.kernel_ms += tried.kernel_ms;
+    st.launches = 1 + tried.launches;
     const int* h = collected_words(ctx);
     st.rounds = h[out - flags];
     st.barriers = h[out + 1 - flags];

@@ -94,10 +94,13 @@ typedef struct {
 
 typedef struct {
   int participating;     /* groups that took part (discovered P)              */
-  int rounds;            /* rounds / levels / iterations executed             */
+  int rounds;            /* rounds / levels / iterations executed (worklist SSSP of
+                            a local graph, below: rounds inside the ranges)  */
   long long barriers;    /* inter-workgroup barriers executed (per group)     */
-  long long launches;    /* kernel launches in the solve                      */
-  double kernel_ms;      /* solve time, device events around the kernels      */
+  long long launches;    /* kernel launches in the solve, attempts that it gave
+                            up (colour, BC) and the worklists' locality sample
+                            and level count among them                       */
+  double kernel_ms;      /* solve time, device events around those kernels    */
   long long work_edges;  /* edges examined (for algorithmic-byte accounting)  */
   long long work_items;  /* vertices / worklist items processed               */
 } gdb_stats;
@@ -236,7 +239,11 @@ int gdb_tune_load(const char* path);
 int gdb_tune_lookup(const char* solver, long long n, gdb_tune_entry* out);
 
 /* ---- solvers (device pointers; CSR int32, row has n+1 entries) ------------- */
-/* Pannotia colouring (max rule): color[v] = round in which v was coloured. */
+/* Pannotia colouring (max rule): color[v] = round in which v was coloured.
+ * The tuned persistent variant colours graphs of up to 1 M edges without
+ * rounds (stats->barriers 0; participating counts the groups that hold edges)
+ * where the launch has room for them, and one group where the shape is open
+ * and a group holds the graph; the tuning table's row is for the rest. */
 int gdb_color(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const float* node_value,
               int* color, const gdb_opts* opts, gdb_stats* stats);
 /* Max-min colouring: the two-sided variant of the max rule above, which the
@@ -260,12 +267,18 @@ int gdb_sssp_pull(gdb_ctx* ctx, int n, int m, const int* row_t, const int* col_t
  * tuned persistent schedule sweeps eight sources at a time, a symmetric graph
  * (pass the CSR as its own transpose: row_t == row, col_t == col) with one
  * edge walk per vertex, a directed one with separate in- and out-edge walks;
- * one source at a time for a single source or a search deeper than 254
- * levels of a directed graph. */
+ * one source at a time for a single source or a search of more than 254 levels
+ * (the source's included) of a directed graph. */
 int gdb_bc(gdb_ctx* ctx, int n, int m, const int* row, const int* col, const int* row_t,
            const int* col_t, const int* sources, int nsrc, float* bc, const gdb_opts* opts,
            gdb_stats* stats);
-/* Lonestar worklist BFS: levels from `source`, unreachable = 1000000000. */
+/* Lonestar worklist BFS: levels from `source`, unreachable = 1000000000.
+ * With the launch shape left open (wgs and groups 0, tuned persistent) a
+ * sparse graph whose ids follow locality, as a sample of its edges tells, is
+ * solved by owner-partitioned ranges (gdb_task.owned) in place of iteration
+ * queues, here and in gdb_sssp_worklist: stats->barriers is 0 then, and an
+ * SSSP's rounds count the ranges' rounds.  Under a wait bound that the ranges
+ * do not meet the queues run after them. */
 int gdb_bfs_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, int source,
                      unsigned* dist, const gdb_opts* opts, gdb_stats* stats);
 /* Lonestar worklist SSSP (label-correcting, atomic min). */

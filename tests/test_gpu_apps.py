@@ -5,6 +5,8 @@ Bars: MIS sets, SSSP distances and BFS levels bit-exact; BC (FP32) within
 1e-4 relative of the FP64 Brandes oracle entry by entry, |got - want| <=
 1e-4 * |want|, with an absolute floor of 1e-6 that only matters for entries
 that are (near) zero."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -757,3 +759,26 @@ def test_worklist_local_graph_with_long_edges(ctx, long_per_mille):
     got, st = gdb.sssp_worklist(ctx, d, 5, o)
     assert (got.astype(np.int64) == oracle.dijkstra_tb(row, col, w, 5)).all()
     assert (st.barriers == 0) == (long_per_mille < 15)
+
+
+def test_stats_count_samples_and_attempts(ctx):
+    """kernel_ms and launches hold all of a solve's device work: the locality sample,
+    the level count, and attempts that were given up."""
+    o = gdb.Opts.make(wgs=0, variant=gdb.VARIANT_TUNED)
+    g = gdb.gen_grid(100, 100, 0.05, seed=3, wlo=1, whi=255)
+    local, other = gdb.DeviceCSR(g), gdb.DeviceCSR(g.relabel(gdb.permutation(g.n, 5)))
+    assert gdb.bfs_worklist(ctx, local, 0, o)[1].launches == 3
+    assert gdb.sssp_worklist(ctx, local, 0, o)[1].launches == 2
+    assert gdb.bfs_worklist(ctx, other, 0, o)[1].launches == 2
+    assert gdb.bfs_worklist(ctx, other, 0, gdb.Opts.make(wgs=256, variant=gdb.VARIANT_TUNED))[1].launches == 1
+    # Equal priorities: the round-free colouring waits 2 ms for progress.
+    row, col, _ = csr_from_edges(3, [(0, 1), (1, 2), (0, 2)])
+    d, nv = dev(row, col), gdb.DeviceBuffer.from_numpy(np.full(3, 0.5, np.float32))
+    out, st = gdb.DeviceBuffer.empty(3, np.int32), gdb.Stats()
+    rc = gdb.lib().gdb_color(ctx.h, 3, d.m, d.row.ptr, d.col.ptr, nv.ptr, out.ptr, C.byref(o), C.byref(st))
+    assert rc == gdb.GDB_E_TIMEOUT and st.launches == 2 and st.kernel_ms > 2.0
+    # Two sources of a directed chain deeper than the level bytes.
+    row = np.minimum(np.arange(301), 299).astype(np.int32)
+    g = gdb.CSR(300, row, np.arange(1, 300, dtype=np.int32), np.ones(299, np.int32))
+    _, st = gdb.bc(ctx, gdb.DeviceCSR(g), gdb.DeviceCSR(g.transpose()), np.array([0, 1], np.int32), o)
+    assert st.launches == 2
