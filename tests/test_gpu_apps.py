@@ -782,3 +782,36 @@ def test_stats_count_samples_and_attempts(ctx):
     g = gdb.CSR(300, row, np.arange(1, 300, dtype=np.int32), np.ones(299, np.int32))
     _, st = gdb.bc(ctx, gdb.DeviceCSR(g), gdb.DeviceCSR(g.transpose()), np.array([0, 1], np.int32), o)
     assert st.launches == 2
+
+
+# The default options of Opts.make are the plain variant's; these run four of the
+# tests above on the tuned kernels whose edges they were written for.
+@pytest.fixture
+def tuned(monkeypatch):
+    make = gdb.Opts.make
+    monkeypatch.setattr(gdb.Opts, "make", lambda **kw: make(**{"variant": gdb.VARIANT_TUNED, **kw}))
+
+
+@pytest.mark.parametrize("extra", [0, 1, 31])
+@pytest.mark.parametrize("deg", [1, 15, 16, 17, 79, 80, 81, 300])
+def test_mis_one_deciding_edge_tuned(ctx, tuned, deg, extra):
+    test_mis_one_deciding_edge(ctx, deg, extra)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1025])
+@pytest.mark.parametrize("wgs,groups", [(64, 1), (256, 3), (0, 0)])
+def test_bfs_sweep_tuned(ctx, tuned, n, wgs, groups):
+    test_bfs_sweep(ctx, n, wgs, groups)
+
+
+@pytest.mark.parametrize("n", [1023, 1024, 1030])
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("wgs,groups", [(64, 4), (256, 3), (0, 0)])
+def test_bc_step_with_many_edges_tuned(ctx, tuned, n, directed, wgs, groups):
+    test_bc_step_with_many_edges(ctx, n, directed, wgs, groups)
+
+
+@pytest.mark.parametrize("deg", [15, 16, 17, 63, 64, 65, 128, 129, 192, 193])
+@pytest.mark.parametrize("hubs", [1, 3, 4, 5, 64])
+def test_rows_walked_by_part_of_a_wave_tuned(ctx, tuned, deg, hubs):
+    test_rows_walked_by_part_of_a_wave(ctx, deg, hubs)
