@@ -13,7 +13,7 @@ called with wgs = 0, so the library, the CLIs (WORKGROUP_SIZE 0) and
 bench.py all run the tuned shapes.
 
 Usage: python -m gpu_discovery_barrier_amd.autotune [--quick] [--out PATH]
-          [--only color,mis,bc,batch_grid,batch_many,worklist]
+          [--only color,mis,bc,bfs_wl,bfs_wl_sparse,sssp_wl,sssp_pull,mst,batch_grid,batch_many]
 """
 from __future__ import annotations
 
@@ -87,59 +87,91 @@ def shapes(wgs_list, groups_list):
             yield w, g
 
 
-def tune_solver(ctx, name, graph_n, run, wgs_list, groups_list, repeats=2) -> tuple[dict, list]:
-    trials = []
-    for w, g in shapes(wgs_list, groups_list):
-        ms = min(run(w, g) for _ in range(repeats))
-        trials.append((ms, w, g))
-    ms, w, g = best_of(trials)
-    log(f"{name}: wgs {w} groups {g} {ms:.3f} ms ({len(trials)} shapes)")
-    return row(name, graph_n, w, g), trials
+# The single-task solvers' rows: (solver, n_max, work-group sizes, group counts,
+# graphs).  A row is tuned on graphs that read it: of n in its range, and that take
+# the kernel it shapes.  Colouring's row is for the kernel with rounds, so its
+# graph has more edges than the round-free one takes (about a million);
+# the worklists' are skewed or without locality in their ids, since the local
+# ones take owner-partitioned ranges (bfs_wl_sparse: up to six edges a vertex).
+# With several graphs a shape counts the geometric mean of its times.
+SINGLE = [
+    ("color", 1 << 20, (64, 128, 256, 512, 1024), (64, 128, 256, 512), ["rmat17"]),
+    ("mis", 1500000, (256, 512, 1024), (64, 128, 256, 512), ["rmat17", "gnp500000"]),
+    ("mis", 1 << 30, (256, 512, 1024), (256, 512, 1024, 2048), ["rmat22"]),
+    ("bc", 1 << 30, (256, 512), (256, 512, 1024), ["rmat22"]),
+    ("bfs_wl", 524287, (256, 512, 1024), (64, 128, 256), ["rmat17", "gnp300000"]),
+    ("bfs_wl", 1 << 30, (256, 512, 1024), (64, 128, 256, 512), ["rmat20"]),
+    ("bfs_wl_sparse", 300000, (256, 512), (16, 32, 64, 128), ["shuffled500", "gnp4_100000"]),
+    ("bfs_wl_sparse", 1 << 30, (256, 512), (32, 64, 128, 256), ["shuffled1000", "gnp4_500000"]),
+    ("sssp_wl", 20000, (128, 256, 512), (64, 128, 256), ["rmat13", "gnp15000"]),
+    ("sssp_wl", 262143, (256, 512, 1024), (64, 128, 256), ["rmat16", "gnp100000"]),
+    ("sssp_wl", 1 << 30, (256, 512, 1024), (128, 256, 512), ["rmat18"]),
+    ("sssp_pull", 12288, (128, 256, 512), (64, 128, 256), ["rmat11", "gnp3000"]),
+    ("sssp_pull", 1 << 30, (256, 512), (64, 128, 256), ["rmat16"]),
+    ("mst", 262143, (256, 512, 1024), (64, 128, 256), ["rmat16", "gnp200000"]),
+    ("mst", 1 << 30, (256, 512, 1024), (128, 256, 512), ["rmat18", "grid1000"]),
+]
+# A row stands unless another shape beats it by this much: what the runs of one
+# shape differ.
+KEEP = 0.97
 
 
-def tune_color(ctx, quick=False):
-    g = api.gen_rmat(14, 16, seed=1)
-    dg = api.DeviceCSR(g, weights=False)
-    nv = api.DeviceBuffer.from_numpy((api.permutation(g.n, 1).astype(np.float64) / (g.n + 1)).astype(np.float32))
-    out = api.DeviceBuffer.empty(g.n, np.int32)
-    run = lambda w, gr: api.color(ctx, dg, nv, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
-                                  out=out)[1].kernel_ms
-    return tune_solver(ctx, "color", 1 << 20, run, (64, 128, 256) if quick else (64, 128, 256, 512, 1024),
-                       (32, 64, 128, 256, 512))
+def graph_size(name) -> int:
+    kind = name.rstrip("0123456789")
+    size = int(name[len(kind):])
+    return {"rmat": 1 << size, "gnp": size, "gnp4_": size}.get(kind, size * size)
 
 
-def tune_mis_bc(ctx, quick=False):
-    scale = 20 if quick else 22
-    g = api.gen_rmat(scale, 16, seed=3)
-    dg = api.DeviceCSR(g, weights=False)
-    nv = api.DeviceBuffer.from_numpy((api.permutation(g.n, 3).astype(np.float64) / (g.n + 1)).astype(np.float32))
-    out = api.DeviceBuffer.empty(g.n, np.int32)
-    mis = lambda w, gr: api.mis(ctx, dg, nv, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
-                                out=out)[1].kernel_ms
-    r1, t1 = tune_solver(ctx, "mis", 1 << 30, mis, (256, 512, 1024), (256, 512, 1024, 2048))
+def graph(name):
+    kind = name.rstrip("0123456789")
+    size = int(name[len(kind):])
+    if kind == "rmat":
+        return api.gen_rmat(size, 16, seed=3, wlo=1, whi=100)
+    if kind.startswith("gnp"):
+        return api.gen_gnp(size, 4.0 if kind == "gnp4_" else 8.0, seed=3, wlo=1, whi=100)
+    g = api.gen_grid(size, size, 0.05, seed=3, wlo=1, whi=255)
+    return g.relabel(api.permutation(g.n, 5)) if kind == "shuffled" else g
+
+
+def solver_run(ctx, solver, name):
+    """A function that runs the solver on the graph with the given options; its device ms."""
+    g = graph(name)
+    d = api.DeviceCSR(g)
     deg = np.diff(g.row)
-    src = np.sort(np.random.default_rng(3).choice(np.flatnonzero(deg > 0), 16, replace=False)).astype(np.int32)
-    bout = api.DeviceBuffer.empty(g.n, np.float32)
-    bc = lambda w, gr: api.bc(ctx, dg, dg, src, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
-                              out=bout)[1].kernel_ms
-    r2, t2 = tune_solver(ctx, "bc", 1 << 30, bc, (256, 512), (256, 512, 1024), repeats=1)
-    return [r1, r2], t1 + t2
+    if solver in ("color", "mis"):
+        out = api.DeviceBuffer.empty(g.n, np.int32)
+        nv = api.DeviceBuffer.from_numpy((api.permutation(g.n, 3).astype(np.float64) / (g.n + 1)).astype(np.float32))
+        fn = {"color": api.color, "mis": api.mis}[solver]
+        return lambda o: fn(ctx, d, nv, o, out=out)[1].kernel_ms
+    if solver == "bc":
+        out = api.DeviceBuffer.empty(g.n, np.float32)
+        src = np.sort(np.random.default_rng(3).choice(np.flatnonzero(deg > 0), 16, replace=False)).astype(np.int32)
+        return lambda o: api.bc(ctx, d, d, src, o, out=out)[1].kernel_ms
+    if solver == "mst":
+        return lambda o: api.mst(ctx, d, o)[3].kernel_ms
+    out = api.DeviceBuffer.empty(g.n, np.int32 if solver == "sssp_pull" else np.uint32)
+    fn = {"sssp_pull": api.sssp_pull, "sssp_wl": api.sssp_worklist}.get(solver, api.bfs_worklist)
+    source = int(np.flatnonzero(deg > 0)[0])
+    return lambda o: fn(ctx, d, source, o, out=out)[1].kernel_ms
 
 
-def tune_worklist(ctx, quick=False):
-    # A skewed graph: local ones (grids) take the owner-partitioned solve when
-    # the shape is left open, so the rows serve the others.
-    g = api.gen_rmat(16 if quick else 18, 16, seed=2, wlo=1, whi=100)
-    dg = api.DeviceCSR(g)
-    out = api.DeviceBuffer.empty(g.n, np.uint32)
-    rows, trials = [], []
-    for name, fn in (("bfs_wl", api.bfs_worklist), ("sssp_wl", api.sssp_worklist)):
-        run = lambda w, gr: fn(ctx, dg, 0, api.Opts.make(wgs=w, groups=gr, variant=api.VARIANT_TUNED),
-                               out=out)[1].kernel_ms
-        r, t = tune_solver(ctx, name, 1 << 30, run, (256, 512), (64, 128, 256, 512), repeats=3)
-        rows.append(r)
-        trials += t
-    return rows, trials
+def tune_single(ctx, solver, n_max, wgs_list, groups_list, graphs, old, repeats=3) -> tuple[dict, list]:
+    runs = [solver_run(ctx, solver, name) for name in graphs]
+
+    def time_of(w, g):
+        o = api.Opts.make(wgs=w, groups=g, variant=api.VARIANT_TUNED)
+        return float(np.exp(np.mean([np.log(min(r(o) for _ in range(repeats))) for r in runs])))
+
+    trials = [(time_of(w, g), w, g) for w, g in shapes(wgs_list, groups_list)]
+    ms, w, g = best_of(trials)
+    kept = ""
+    if old:
+        stood = time_of(old["wgs"], old["groups"])
+        if ms > KEEP * stood:
+            ms, w, g, kept = stood, old["wgs"], old["groups"], ", stands"
+    log(f"{solver} up to {n_max} ({', '.join(graphs)}): wgs {w} groups {g} {ms:.3f} ms ({len(trials)} shapes, "
+        f"best {best_of(trials)[0]:.3f}{kept})")
+    return row(solver, n_max, w, g), trials
 
 
 def grid_batch_run(ctx, dg, out_b, out_s, w, gr, team, delta, hops, qcap, owned=False):
@@ -224,9 +256,9 @@ def tune_batch_many(ctx, quick=False):
 
 def main() -> int:
     ap = argparse.ArgumentParser(description=__doc__)
-    ap.add_argument("--quick", action="store_true", help="smaller search spaces and graphs")
+    ap.add_argument("--quick", action="store_true", help="smaller search spaces and graphs (batches)")
     ap.add_argument("--out", default=str(TABLE))
-    ap.add_argument("--only", default="color,mis,bc,worklist,batch_grid,batch_many")
+    ap.add_argument("--only", default=",".join(dict.fromkeys(r[0] for r in SINGLE)) + ",batch_grid,batch_many")
     ap.add_argument("--report", default="", help="also write every trial as JSON here")
     a = ap.parse_args()
     only = set(a.only.split(","))
@@ -234,21 +266,16 @@ def main() -> int:
     rows, report = [], {}
     t0 = time.time()
     try:
-        old = {(r["solver"], r["n_max"]): r for r in read_table(a.out)} if Path(a.out).exists() else {}
+        base = a.out if Path(a.out).exists() else TABLE
+        old = {(r["solver"], r["n_max"]): r for r in read_table(base)} if Path(base).exists() else {}
     except ValueError:
         old = {}
-    if "color" in only:
-        r, t = tune_color(ctx, a.quick)
+    for solver, n_max, wgs_list, groups_list, graphs in SINGLE:
+        if solver not in only:
+            continue
+        r, t = tune_single(ctx, solver, n_max, wgs_list, groups_list, graphs, old.get((solver, n_max)))
         rows.append(r)
-        report["color"] = t
-    if only & {"mis", "bc"}:
-        rs, t = tune_mis_bc(ctx, a.quick)
-        rows += rs
-        report["mis_bc"] = t
-    if "worklist" in only:
-        rs, t = tune_worklist(ctx, a.quick)
-        rows += rs
-        report["worklist"] = t
+        report[f"{solver}_{n_max}"] = t
     if "batch_grid" in only:
         rs, t = tune_batch_grid(ctx, a.quick)
         rows += rs

@@ -149,3 +149,20 @@ def test_relabel_by_degree_is_an_isomorphism():
 
     with pytest.raises(gdb.GdbError):
         g.relabel(np.zeros(g.n, np.int32))  # not a permutation
+
+
+def test_autotuner_covers_the_table_on_graphs_that_read_its_rows():
+    from gpu_discovery_barrier_amd import autotune
+
+    table = autotune.read_table()
+    single = {(s, n): graphs for s, n, _, _, graphs in autotune.SINGLE}
+    assert {(r["solver"], r["n_max"]) for r in table if not r["solver"].startswith("batch")} == set(single)
+    for (solver, n_max), graphs in single.items():
+        for name in graphs:
+            n = autotune.graph_size(name)
+            assert autotune.lookup(solver, n)["n_max"] == n_max, (solver, name)
+    shape = {(s, n): (w, g) for s, n, w, g, _ in autotune.SINGLE}
+    for r in table:  # each committed shape is among those tried
+        if (r["solver"], r["n_max"]) in shape:
+            w, g = shape[r["solver"], r["n_max"]]
+            assert r["wgs"] in w and r["groups"] in g, r
