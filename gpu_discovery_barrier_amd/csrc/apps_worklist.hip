@@ -175,7 +175,9 @@ constexpr int kLongRow = 1024;
 // R-MAT 20: 0.65 -> 0.42 ms, 17: 0.217 -> 0.203, 12: unchanged.  A bit per vertex
 // claimed by OR, as a denser filter in place of dist, was slower: 1.16 ms.
 
-template <int WGS, bool WEIGHTED>
+// SPARSE: fewer than eight edges a vertex, where rows may be even (gdb::even_rows); the
+// others do without that code.
+template <int WGS, bool WEIGHTED, bool SPARSE>
 __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                                   const int* __restrict__ col,
                                                   const int* __restrict__ w, unsigned* dist,
@@ -195,7 +197,7 @@ __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const i
   unsigned char* const mark = (unsigned char*)stamp;  // BFS: a byte per vertex, set once it is reached
   const int sweep_from = gdb::sweep_line(n);
   const bool may_sweep = !WEIGHTED && row[n] > sweep_from;
-  const bool even = gdb::even_rows(n, row[n], *long_row != 0);
+  const bool even = SPARSE && gdb::even_rows(n, row[n], *long_row != 0);
   // Moves staged vertices to the queue; BFS adds up their edges.
   auto flush = [&](int above, int* queue, int* tail) {
     gdb::group_flush(stage, above, queue, tail, may_sweep ? row : nullptr, &s_deg);
@@ -454,11 +456,11 @@ __global__ void k_wl_step(const int* __restrict__ row, const int* __restrict__ c
   }
 }
 
-// *long_row (0 before): whether a row has more than kEvenRow edges.
+// *long_row (0 before): whether a row has more than kEvenRow edges (row null: not asked).
 __global__ void k_wl_init(const int* __restrict__ row, unsigned* dist, int* stamp, int* q0, int* q1, int* flags,
                           int* long_row, int n, int src, bool bytes) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && row[i + 1] - row[i] > gdb::kEvenRow) *long_row = 1;
+  if (i < n && row && row[i + 1] - row[i] > gdb::kEvenRow) *long_row = 1;
   if (i < n) {  // initialize (bfs_common.cl:64-71) + dist[source] = 0
     dist[i] = i == src ? 0u : kInf;
     stamp[i] = bytes && i == src >> 2 ? 1 << 8 * (src & 3) : 0;  // bytes: the source is marked
@@ -705,8 +707,9 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
   int* long_row = (int*)(work + 2);
   rc = prepare_launch(ctx, (int*)work, 5);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, row, dist, stamp, q0, q1,
-                     flags, long_row, n, source, !WEIGHTED);
+  hipLaunchKernelGGL(k_wl_init, dim3((n + 255) / 256), dim3(256), 0, ctx->stream,
+                     gdb::even_rows(n, m, false) ? row : nullptr, dist, stamp, q0, q1, flags, long_row, n, source,
+                     !WEIGHTED);
   GDB_HIP(hipGetLastError());
 
   if (o.schedule == GDB_SCHED_RELAUNCH) {
@@ -741,14 +744,21 @@ int run_worklist(gdb_ctx* ctx, int n, int m, const int* row, const int* col, con
     const int nwords = (int)((int*)(work + 2) - flags);  // flags and work are neighbours in the workspace
     rc = gdb_dispatch_wgs(wgs, [&](auto W) -> int {
       constexpr int WG = decltype(W)::value;
-      const void* kern = tuned ? (const void*)k_wl_tuned<WG, WEIGHTED> : (const void*)k_wl_plain<WG, WEIGHTED>;
+      const bool sparse = gdb::even_rows(n, m, false);
+      const void* kern = !tuned   ? (const void*)k_wl_plain<WG, WEIGHTED>
+                         : sparse ? (const void*)k_wl_tuned<WG, WEIGHTED, true>
+                                  : (const void*)k_wl_tuned<WG, WEIGHTED, false>;
       int groups = 0;
       int r2 = launch_groups(ctx, kern, &o, tuned ? row_walk_items(n, m, wgs) : n, &groups);
       if (r2) return r2;
       r2 = timer_start(ctx);
       if (r2) return r2;
-      if (tuned)
-        hipLaunchKernelGGL((k_wl_tuned<WG, WEIGHTED>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
+      if (tuned && sparse)
+        hipLaunchKernelGGL((k_wl_tuned<WG, WEIGHTED, true>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
+                           row, col, w, dist, stamp, q0, q1, tails, n, pieces, piece_cap,
+                           long_row, work, out);
+      else if (tuned)
+        hipLaunchKernelGGL((k_wl_tuned<WG, WEIGHTED, false>), dim3(groups), dim3(WG), 0, ctx->stream, ctx->d,
                            row, col, w, dist, stamp, q0, q1, tails, n, pieces, piece_cap,
                            long_row, work, out);
       else

@@ -217,8 +217,9 @@ int gdb_probe_pingpong(gdb_ctx* ctx, int mode, int fine, int same_xcd, int iters
  * device and writes a text table, one row per line:
  *     solver n_max wgs groups team_groups delta hops lds_queue
  * (solver: color, mis, bc, sssp_pull, bfs_wl, bfs_wl_sparse, sssp_wl, mst,
- * batch, batch_owned; '#' starts a comment).  bfs_wl_sparse: worklist BFS of
- * at most six edges a vertex, bfs_wl where the table has no such row.  The library loads it once per process, at the first
+ * batch, batch_owned; '#' starts a comment).  bfs_wl_sparse is for worklist BFS
+ * of at most six edges a vertex, which takes bfs_wl where the table has none.
+ * The library loads the table once per process, at the first
  * gdb_ctx_create, from $GDB_TUNE_FILE or else tune_table.txt beside
  * libgdb_amd.so.  A solver called with opts == NULL or opts->wgs == 0 takes
  * wgs, groups (when opts->groups == 0) and lds_queue from the row for its
