@@ -175,8 +175,8 @@ constexpr int kLongRow = 1024;
 // R-MAT 20: 0.65 -> 0.42 ms, 17: 0.217 -> 0.203, 12: unchanged.  A bit per vertex
 // claimed by OR, as a denser filter in place of dist, was slower: 1.16 ms.
 
-// SPARSE: fewer than eight edges a vertex, where rows may be even (gdb::even_rows); the
-// others do without that code.
+// SPARSE: at most six edges a vertex, where rows may be even (gdb::even_rows); the others
+// do without that code.
 template <int WGS, bool WEIGHTED, bool SPARSE>
 __global__ __launch_bounds__(WGS) void k_wl_tuned(gdb_kernel_ctx_t* ctx, const int* __restrict__ row,
                                                   const int* __restrict__ col,

@@ -487,13 +487,15 @@ __device__ __forceinline__ long long spread_item(int start, int stride, int sh) 
 // (2^20-vertex grid MST 1.16 ms against 1.44).
 __host__ __device__ inline int spread_rows(int n, long long m) { return m >= 8LL * n ? 0 : 6; }
 // The same for a step over `items` queued vertices.  Where all rows are short (`even`:
-// eight edges a vertex at most, none of more than kEvenRow) a wave takes 16 neighbours,
-// and 64 in a step of up to 256: the fewer groups have work, the fewer come late to
-// the barrier.  One by one against this: BFS of a 100^2 grid of shuffled ids 0.84 -> 0.76
-// ms, BC of it, 11 sources, 6.6 -> 5.8; 64 always: SSSP of a 500^2 one 7.9 -> 13.4.
+// six edges a vertex at most, no row of more than kEvenRow) a wave takes 16 neighbours
+// in a step of up to 1024, and 64 in one of up to 256: the fewer groups have work, the
+// fewer come late to the barrier.  One by one against this: BFS of a 100^2 grid of
+// shuffled ids 0.84 -> 0.76 ms, BC of it, 11 sources, 6.6 -> 5.8.  Longer steps fill the
+// waves one by one (64 always: SSSP of a shuffled 500^2 grid 7.9 -> 13.4 ms), and so do
+// rows of eight edges (SSSP of G(3000) of degree 8 216 us, 228 by 16).
 constexpr int kEvenRow = 64;
-__host__ __device__ inline bool even_rows(int n, long long m, bool long_row) { return m < 8LL * n && !long_row; }
-__host__ __device__ inline int spread_queue(bool even, int items) { return !even ? 0 : items <= 256 ? 6 : 4; }
+__host__ __device__ inline bool even_rows(int n, long long m, bool long_row) { return m <= 6LL * n && !long_row; }
+__host__ __device__ inline int spread_queue(bool even, int items) { return !even || items > 1024 ? 0 : items <= 256 ? 6 : 4; }
 // Whether such a step pushes straight to the queue.  Its pushes are few, and the
 // barriers of the group that staging takes (group_flush) cost more than their atomics:
 // BFS of a shuffled 500^2 grid 5.0 -> 4.3 ms (512 items: 4.8), of a 100^2 grid 0.75 ->
